@@ -25,6 +25,8 @@
 // the coefficient gradients (adjoint) in registers before one read-modify-
 // write of the group's accumulator plane.  State is ping-ponged between two
 // buffer sets, so halo reads never race with neighbouring strips' writes.
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace {
@@ -1137,6 +1139,8 @@ __global__ void ac_inject(AcDev d, float *__restrict__ lam, const float *__restr
   if (g_w) atomicAdd(&lam[2 * d.field + o], g_w[gi]);
 }
 
+#include "acoustic_tile.hpp"
+
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
@@ -1240,6 +1244,73 @@ bool pair_drop_ok(const adfwi_layout &L) {
   const char *e = std::getenv("ADFWI_PAIR_DROP");
   if (e && e[0] == '0') return false;
   return 2 * L.field_floats * 4 < ((int64_t)1 << 31);
+}
+
+// ---- tiles (acoustic_tile.hpp): up to TK steps per launch
+// The tile kernels take any problem whose layout the caller left to the library (the strip
+// options of the descriptor belong to the strip kernels); their 8-byte accesses need an even
+// row pitch, and their descriptors span at most five planes.
+bool tile_ok(const adfwi_acoustic_desc *d) {
+  return d->shots_per_block == 0 && d->tile_z == 0 && d->row_unroll == 0 && d->adj_shots_per_block == 0 &&
+         d->pitch % 2 == 0 && (long long)d->nz * d->pitch * 5 * 4 < ((int64_t)1 << 31);
+}
+
+// Tile shapes: 40 x 64 (stores 16 x 40), 64 x 64 (40 x 40), 64 x 128 (40 x 104).  The smaller a
+// tile the more of it is halo, but the sooner its workgroup is done: a launch whose workgroups
+// all run at once (one per CU) lasts as long as one of them.  So: the smallest shape that still
+// gives at most one workgroup per CU, else the largest.  Measured, forward with records,
+// us per step: 140 x 240, 1 shot (54 / 24 / 12 workgroups): 2.4 / 2.9 / 4.3; 10 shots
+// (540 / 240 / 120): 5.1 / 3.3 / 4.6; 149 x 263, 40 shots (2520 / 1120 / 480): 16.2 / 13.3 / 9.6.
+enum class TileShape { SMALL, MEDIUM, LARGE };
+constexpr long long TILE_CUS = 256;
+
+template <int NR, int NW, int CPL>
+long long tile_count(const AcDev &v) {
+  constexpr int oz = tile::out_rows(NR * NW), ox = tile::out_cols(CPL);
+  return (long long)((v.X + ox - 1) / ox) * ((v.Z - v.zbase + oz - 1) / oz);
+}
+
+TileShape tile_shape(const AcDev &v) {
+  const long long groups = (v.S + v.spb - 1) / v.spb;
+  if (tile_count<4, 10, 1>(v) * groups <= TILE_CUS) return TileShape::SMALL;
+  if (tile_count<4, 16, 1>(v) * groups <= TILE_CUS) return TileShape::MEDIUM;
+  return TileShape::LARGE;
+}
+
+template <int NR, int NW, int CPL>
+tile::Grid tile_grid(const AcDev &v, int spg) {
+  constexpr int oz = tile::out_rows(NR * NW), ox = tile::out_cols(CPL);
+  tile::Grid g;
+  g.ntx = (v.X + ox - 1) / ox;
+  g.ntz = (v.Z - v.zbase + oz - 1) / oz;
+  g.spg = spg;
+  g.ngroups = (v.S + spg - 1) / spg;
+  return g;
+}
+
+template <int NR, int NW, int CPL, int F>
+void launch_fwd_tile_c(const AcDev &v, hipStream_t st, const tile::FwdIO &io) {
+  const tile::Grid g = tile_grid<NR, NW, CPL>(v, v.spb);
+  hipLaunchKernelGGL((tile::ac_fwd_tile<NR, NW, CPL, F>), dim3((unsigned)(g.ntx * g.ntz * g.ngroups)),
+                     dim3(NW * WAVE), 0, st, v, g, io);
+}
+
+template <int F>
+void launch_fwd_tile_f(const AcDev &v, hipStream_t st, const tile::FwdIO &io) {
+  switch (tile_shape(v)) {
+    case TileShape::SMALL: launch_fwd_tile_c<4, 10, 1, F>(v, st, io); break;
+    case TileShape::MEDIUM: launch_fwd_tile_c<4, 16, 1, F>(v, st, io); break;
+    default: launch_fwd_tile_c<4, 16, 2, F>(v, st, io);
+  }
+}
+
+void launch_fwd_tile(const AcDev &v, hipStream_t st, const tile::FwdIO &io) {
+  const bool rec = io.energy || io.rec_p;
+  if (!io.img_d && !io.img_p) launch_fwd_tile_f<PF_REC>(v, st, io);
+  else if (!rec && !io.img_p) launch_fwd_tile_f<PF_IMGD>(v, st, io);
+  else if (!rec) launch_fwd_tile_f<PF_IMGD | PF_IMGP>(v, st, io);
+  else if (!io.img_p) launch_fwd_tile_f<PF_REC | PF_IMGD>(v, st, io);
+  else launch_fwd_tile_f<PF_REC | PF_IMGD | PF_IMGP>(v, st, io);
 }
 
 dim3 step_grid(const adfwi_layout &L) { return dim3((L.ntiles + WPB - 1) / WPB, L.ngroups); }
@@ -1389,6 +1460,31 @@ int adfwi_acoustic_forward(const adfwi_acoustic_desc *d, adfwi_acoustic_fwd_args
     return nullptr;
   };
   const float *cur = a->state_in;
+  if (fuse && tile_ok(d)) {
+    for (int k = 0; k < a->nsteps;) {
+      const int t = a->t0 + k;
+      int n = min(tile::TK, a->nsteps - k);
+      // with a device time base the state returns to work[0] after whole windows of 4 steps: an
+      // even number of launches
+      if (a->t_base && k == 0 && ((a->nsteps + tile::TK - 1) / tile::TK) % 2) n = max(1, n / 2);
+      if (a->ckpt) n = min(n, a->ckpt_every - t % a->ckpt_every);   // up to the next checkpoint
+      float *nxt = ckpt_slot(t + n - 1);
+      if (!nxt) nxt = (cur == a->work[0]) ? a->work[1] : a->work[0];
+      tile::FwdIO io;
+      io.in = cur; io.out = nxt; io.t = t; io.n = n;
+      io.energy = a->energy;
+      io.img_d = a->image ? a->image + (long long)k * L.field_floats : nullptr;
+      io.img_p = a->image_p ? a->image_p + (long long)k * L.field_floats : nullptr;
+      io.rmap = recs && d->nrec > 0 ? a->rcv_map : nullptr;
+      io.rec_p = recs ? a->rec_p : nullptr; io.rec_u = a->rec_u; io.rec_w = a->rec_w;
+      launch_fwd_tile(v, st, io);
+      if ((rc = adfwi::check_launch("ac_fwd_tile"))) return rc;
+      cur = nxt;
+      k += n;
+    }
+    a->state_out = cur;
+    return ADFWI_OK;
+  }
   for (int k = 0; k < a->nsteps;) {
     const int t = a->t0 + k;
     const bool pair = fuse && k + 1 < a->nsteps && ckpt_slot(t) == nullptr;

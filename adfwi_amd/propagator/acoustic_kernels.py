@@ -95,8 +95,24 @@ class Timeline:
         return out
 
 
+TILE_STEPS = 4    # steps per launch of the tile kernels
+
+
+def tile_launches(t0: int, n: int, ckpt_every: int) -> int:
+    """Launches of the tile kernels for steps t0 .. t0+n-1: at most TILE_STEPS steps each, none
+    past a checkpoint."""
+    launches = k = 0
+    while k < n:
+        m = min(TILE_STEPS, n - k)
+        if ckpt_every:
+            m = min(m, ckpt_every - (t0 + k) % ckpt_every)
+        launches += 1
+        k += m
+    return launches
+
+
 def forward_launches(t0: int, n: int, nt: int, ckpt_every: int, fuse: bool):
-    """Launches adfwi_acoustic_forward issues for steps t0 .. t0+n-1: (pairs, single steps).
+    """Launches the strip kernels issue for steps t0 .. t0+n-1: (pairs, single steps).
     A step is paired with the next one unless it is the call's last step or its state is a
     checkpoint."""
     pairs = singles = 0
@@ -164,7 +180,7 @@ class AcousticGeometry:
         i32 = lambda a: torch.tensor(a.astype(np.int32), device=self.device)
         self.src_z, self.src_x = i32(src_z), i32(src_x)
         self.rcv_z, self.rcv_x = i32(rcv_z), i32(rcv_x)
-        # two steps per launch (the intermediate step's receivers written from inside the kernel)
+        # several steps per launch (the intermediate steps' receivers written from inside the kernel)
         self.fuse_steps = int(os.environ.get("ADFWI_FUSE_STEPS", "1"))
         self.rcv_map = self._receiver_map(rcv_z, rcv_x) if self.fuse_steps else None
         # what a captured launch sequence depends on besides its buffers and the source positions
@@ -176,6 +192,13 @@ class AcousticGeometry:
         self.layout = nat.Layout()
         nat.check(nat.load().adfwi_acoustic_get_layout(ctypes.byref(desc), ctypes.byref(self.layout)),
                   "adfwi_acoustic_get_layout")
+
+    @property
+    def tiled(self) -> bool:
+        """Whether fused steps run on the tile kernels (the strip options of the descriptor ask
+        for the strip kernels)."""
+        return bool(self.fuse_steps) and not (self.shots_per_block or self.adj_shots_per_block or self.row_unroll
+                                              or self.tile_z)
 
     @property
     def gradient_group(self) -> int:
@@ -351,8 +374,12 @@ def run_forward(geom: AcousticGeometry, coef: torch.Tensor, src: torch.Tensor, *
         a.image_p = None if img_p is None else img_p.data_ptr()
         a.rcv_map = None if geom.rcv_map is None else geom.rcv_map.data_ptr()
         a.fuse_steps = geom.fuse_steps
-        pairs, singles = forward_launches(t0, nsteps, nt, int(a.ckpt_every), fused)
-        TIMELINE.call(kind, "ac_fwd_pair" if fused else "ac_fwd_step", pairs + singles, dev, lambda: nat.check(
+        if fused and geom.tiled:
+            name, launches = "ac_fwd_tile", tile_launches(t0, nsteps, int(a.ckpt_every))
+        else:
+            name, launches = ("ac_fwd_pair" if fused else "ac_fwd_step",
+                              sum(forward_launches(t0, nsteps, nt, int(a.ckpt_every), fused)))
+        TIMELINE.call(kind, name, launches, dev, lambda: nat.check(
             lib.adfwi_acoustic_forward(ctypes.byref(d), ctypes.byref(a), nat.stream_handle(dev)),
             "adfwi_acoustic_forward"), steps=nsteps)
         return a.state_out
@@ -456,9 +483,12 @@ def run_backward(geom: AcousticGeometry, coef: torch.Tensor, src: torch.Tensor, 
             fa.image = None if image is None else image.data_ptr()
             fa.image_p = None if image_p is None else image_p.data_ptr()
             fa.fuse_steps = geom.fuse_steps
-            pairs, singles = forward_launches(t_lo, n, nt, 0, bool(geom.fuse_steps))
-            TIMELINE.call("recompute", "ac_fwd_pair" if geom.fuse_steps else "ac_fwd_step", pairs + singles,
-                          dev, lambda: nat.check(
+            if geom.tiled:
+                name, launches = "ac_fwd_tile", tile_launches(t_lo, n, 0)
+            else:
+                name, launches = ("ac_fwd_pair" if geom.fuse_steps else "ac_fwd_step",
+                                  sum(forward_launches(t_lo, n, nt, 0, bool(geom.fuse_steps))))
+            TIMELINE.call("recompute", name, launches, dev, lambda: nat.check(
                 lib.adfwi_acoustic_forward(ctypes.byref(d), ctypes.byref(fa), stream),
                 "adfwi_acoustic_forward (recompute)"), steps=n)
         aa = nat.AcousticAdjArgs()

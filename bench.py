@@ -412,10 +412,10 @@ def main():
     kern = {}
     for name, d in tl.items():
         steps_by = d["steps_by_call"]
-        if name in ("ac_fwd_step", "ac_fwd_pair"):
+        if name in ("ac_fwd_step", "ac_fwd_pair", "ac_fwd_tile"):
             byts = (steps_by.get("forward", 0) * BYTES_FWD + (steps_by.get("recompute", 0)
                     + steps_by.get("forward+images", 0)) * BYTES_RECOMPUTE) * N * S
-        elif name in ("ac_adj_step", "ac_adj_pair"):
+        elif name in ("ac_adj_step", "ac_adj_pair", "ac_adj_tile"):
             byts = d["steps"] * BYTES_ADJ * N * S
         elif name in ("el_fwd_step", "el3_fwd_step"):
             byts = d["steps"] * EL_BYTES_FWD * N * S

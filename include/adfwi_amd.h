@@ -113,10 +113,13 @@ typedef struct adfwi_acoustic_fwd_args {
   float *image_p;          /* [nsteps][S][Z][pitch] or NULL: p after each step */
   const float *state_out;  /* OUT: buffer holding the state after the last step */
   const int32_t *rcv_map;  /* [nz + nz*pitch] or NULL: receivers per row, then the receiver index
-                              at each point (-1 elsewhere); lets two steps share one launch while
+                              at each point (-1 elsewhere); lets several steps share one launch while
                               records are taken (receivers distinct, none on row fs-1 with a free
                               surface) */
-  int32_t fuse_steps;      /* 1: advance two steps per launch where possible; 0: one */
+  int32_t fuse_steps;      /* 1: advance several steps per launch where possible (four on register
+                              tiles; two when the descriptor sets shots_per_block,
+                              adj_shots_per_block, row_unroll or tile_z, which are options of the
+                              strip kernels, or the pitch is odd); 0: one */
   int32_t reserved2;
   const int32_t *t_base;   /* device int or NULL: added at run time to every step index of the
                               call (t0 .. t0+nsteps-1 are then relative), so that one captured
@@ -142,9 +145,9 @@ typedef struct adfwi_acoustic_adj_args {
   float *grad_a1, *grad_a2; /* [ngroups][Z][pitch] (+=) or NULL */
   float *grad_src;          /* [S][nt] or NULL: d loss / d src */
   const float *lam_out;     /* OUT: adjoint state after step t_hi-nsteps (its sources not added) */
-  const int32_t *rcv_map;   /* as in adfwi_acoustic_fwd_args: lets two steps share one launch
-                               while record adjoints are injected */
-  int32_t fuse_steps;       /* 1: reverse two steps per launch where possible; 0: one */
+  const int32_t *rcv_map;   /* as in adfwi_acoustic_fwd_args: lets several steps share one
+                               launch while record adjoints are injected */
+  int32_t fuse_steps;       /* 1: reverse several steps per launch where possible; 0: one */
   int32_t reserved2;
 } adfwi_acoustic_adj_args;
 
