@@ -1258,9 +1258,10 @@ bool tile_ok(const adfwi_acoustic_desc *d) {
 // Tile shapes: 40 x 64 (stores 16 x 40), 64 x 64 (40 x 40), 64 x 128 (40 x 104).  The smaller a
 // tile the more of it is halo, but the sooner its workgroup is done: a launch whose workgroups
 // all run at once (one per CU) lasts as long as one of them.  So: the smallest shape that still
-// gives at most one workgroup per CU, else the largest.  Measured, forward with records,
-// us per step: 140 x 240, 1 shot (54 / 24 / 12 workgroups): 2.4 / 2.9 / 4.3; 10 shots
-// (540 / 240 / 120): 5.1 / 3.3 / 4.6; 149 x 263, 40 shots (2520 / 1120 / 480): 16.2 / 13.3 / 9.6.
+// gives at most one workgroup per CU, else the largest.  Measured, forward with records / adjoint,
+// us per step: 140 x 240, 1 shot (54 / 24 / 12 workgroups): 2.4 / 2.9 / 4.3 and 2.6 / 3.0 / 4.7;
+// 10 shots (540 / 240 / 120): 5.1 / 3.3 / 4.6 and 5.5 / 3.5 / 5.2; 149 x 263, 40 shots
+// (2520 / 1120 / 480): 16.2 / 13.3 / 9.6 and 18.3 / 14.4 / 10.1.
 enum class TileShape { SMALL, MEDIUM, LARGE };
 constexpr long long TILE_CUS = 256;
 
@@ -1311,6 +1312,39 @@ void launch_fwd_tile(const AcDev &v, hipStream_t st, const tile::FwdIO &io) {
   else if (!rec) launch_fwd_tile_f<PF_IMGD | PF_IMGP>(v, st, io);
   else if (!io.img_p) launch_fwd_tile_f<PF_REC | PF_IMGD>(v, st, io);
   else launch_fwd_tile_f<PF_REC | PF_IMGD | PF_IMGP>(v, st, io);
+}
+
+template <int NR, int NW, int CPL, bool A2, bool FULL>
+void launch_adj_tile_c(const AcDev &v, hipStream_t st, const tile::AdjIO &io) {
+  const tile::Grid g = tile_grid<NR, NW, CPL>(v, v.spb);
+  hipLaunchKernelGGL((tile::ac_adj_tile<NR, NW, CPL, A2, FULL>), dim3((unsigned)(g.ntx * g.ntz * g.ngroups)),
+                     dim3(NW * WAVE), 0, st, v, g, io);
+}
+
+template <bool A2, bool FULL>
+void launch_adj_tile_f(const AcDev &v, hipStream_t st, const tile::AdjIO &io) {
+  switch (tile_shape(v)) {
+    case TileShape::SMALL: launch_adj_tile_c<4, 10, 1, A2, FULL>(v, st, io); break;
+    case TileShape::MEDIUM: launch_adj_tile_c<4, 16, 1, A2, FULL>(v, st, io); break;
+    default:
+      if constexpr (A2) launch_adj_tile_c<4, 16, 1, A2, FULL>(v, st, io);   // (two columns per lane spill)
+      else launch_adj_tile_c<4, 16, 2, A2, FULL>(v, st, io);
+  }
+}
+
+// With the rho gradient the adjoint reads the pressure image with its halo too, and the tile's
+// registers hold one column per lane only: 18.2 us per step against the two-step strips' 24.2 on
+// 241 x 441 with 12 shots (1008 tiles of 64 x 64), 21.9 against 31.2 on 149 x 263 with 40 (1120),
+// but 56.5 against 50.2 on 296 x 808 with 16 (2688) and 424 against 298 on 464 x 1232 with 64.
+constexpr long long A2_TILES = 1536;
+bool adj_tile_ok(const AcDev &v, bool a2) {
+  return !a2 || tile_count<4, 16, 1>(v) * ((v.S + v.spb - 1) / v.spb) <= A2_TILES;
+}
+
+void launch_adj_tile(const AcDev &v, hipStream_t st, const tile::AdjIO &io) {
+  const bool full = io.grad_src || io.g_u || io.g_w, a2 = io.grad_a2 && io.img_p;
+  if (a2) full ? launch_adj_tile_f<true, true>(v, st, io) : launch_adj_tile_f<true, false>(v, st, io);
+  else full ? launch_adj_tile_f<false, true>(v, st, io) : launch_adj_tile_f<false, false>(v, st, io);
 }
 
 dim3 step_grid(const adfwi_layout &L) { return dim3((L.ntiles + WPB - 1) / WPB, L.ngroups); }
@@ -1557,6 +1591,25 @@ int adfwi_acoustic_adjoint(const adfwi_acoustic_desc *d, adfwi_acoustic_adj_args
   const dim3 grid1(grid.x, (d->nshots + v1.spb - 1) / v1.spb);
   auto slot = [&](int t) -> long long { return (long long)(t - a->image_t0) * L.field_floats; };
   float *cur = const_cast<float *>(a->lam_in);
+  if (fuse && tile_ok(d) && adj_tile_ok(v1, a->grad_a2 && a->image_p)) {
+    for (int k = 0; k < a->nsteps;) {
+      const int t = a->t_hi - k, n = min(tile::TK, a->nsteps - k);
+      float *nxt = (cur == a->work[0]) ? a->work[1] : a->work[0];
+      tile::AdjIO io;
+      io.in = cur; io.out = nxt; io.t = t; io.n = n;
+      io.img_d = a->image ? a->image + slot(t) : nullptr;
+      io.img_p = a->image_p ? a->image_p + slot(t) : nullptr;
+      io.grad_a1 = a->grad_a1; io.grad_a2 = a->grad_a2; io.grad_src = a->grad_src;
+      io.rmap = recs && d->nrec > 0 ? a->rcv_map : nullptr;
+      io.g_p = a->grad_rec_p; io.g_u = a->grad_rec_u; io.g_w = a->grad_rec_w;
+      launch_adj_tile(v1, st, io);
+      if ((rc = adfwi::check_launch("ac_adj_tile"))) return rc;
+      cur = nxt;
+      k += n;
+    }
+    a->lam_out = cur;
+    return ADFWI_OK;
+  }
   for (int k = 0; k < a->nsteps;) {
     const int t = a->t_hi - k;
     const bool pair = fuse && k + 1 < a->nsteps;

@@ -400,4 +400,384 @@ __global__ __launch_bounds__(NW *WAVE) void ac_fwd_tile(AcDev d, Grid g, FwdIO i
   }
 }
 
+// ---------------------------------------------------------------------------
+// adjoint: up to TK reversed steps per launch, the transposes of ac_fwd_tile's stages on the same
+// tiles (ac_adj_step states them for one step)
+// ---------------------------------------------------------------------------
+struct AdjIO {
+  const float *in;                 // adjoint of the state after step t, its receiver sources not added
+  float *out;
+  int t, n;                        // steps t, t-1, ..., t-n+1 are reversed
+  const float *img_d, *img_p;      // images of step t (the step before one field back) or NULL
+  float *grad_a1, *grad_a2, *grad_src;
+  const int *rmap;
+  const float *g_p, *g_u, *g_w;    // record adjoints [S][nt][R] or NULL
+};
+
+// FULL: u and w record adjoints or the wavelet gradient; A2: the rho gradient
+template <int NR, int NW, int CPL, bool A2, bool FULL>
+__global__ __launch_bounds__(NW *WAVE) void ac_adj_tile(AcDev d, Grid g, AdjIO io) {
+  static_assert(NR >= 4 && H % NR + 2 < NR, "the free-surface rows fs-1 .. fs+1 lie in one wavefront");
+  constexpr int OZ = out_rows(NR * NW), OX = out_cols(CPL);
+  constexpr int NG = FULL ? 3 : 1;                // record components
+  typedef Cols<CPL> C;
+  __shared__ C sg[NW + 2][3][WAVE], sw[NW + 2][3][WAVE];    // rows of a1 lambda_p and of a2 lambda_w
+  __shared__ C srec[NW][NG][TK][WAVE];            // record adjoints of a wavefront's receiver row
+  int tx, tzi, grp;
+  place(g, tx, tzi, grp);
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+  if (wv == 0) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      sg[0][q][lane] = sg[NW + 1][q][lane] = C{};
+      sw[0][q][lane] = sw[NW + 1][q][lane] = C{};
+    }
+  }
+  const int x0 = tx * OX, z0 = d.zbase + tzi * OZ;
+  const int ca = x0 - H + CPL * lane;
+  const int zt = z0 - H + wv * NR;
+  const int fs = d.fs;
+  const unsigned rowb = 4u * (unsigned)d.pitch, planeb = 4u * (unsigned)d.plane;
+  const unsigned vin = ca >= 0 && ca < d.X ? 4u * (unsigned)ca : DROP;
+  const bool own = ca >= x0 && ca < min(x0 + OX, d.X);
+  const unsigned vout = own ? 4u * (unsigned)ca : DROP;
+  const int zend = min(z0 + OZ, d.Z);
+  auto bits = [&](int lo, int hi) -> unsigned {   // rows lo .. hi-1 of this wavefront
+    const int a = min(max(lo - zt, 0), NR), b = min(max(hi - zt, 0), NR);
+    return b > a ? ((1u << b) - 1u) & ~((1u << a) - 1u) : 0u;
+  };
+  const unsigned ownbits = bits(z0, zend), wbits = bits(z0, min(zend, d.Z - 1));
+  auto span = [&](unsigned b, int r) -> unsigned { return (b >> r) & 1u ? planeb : 0u; };
+  auto off = [&](int row) -> unsigned { return (unsigned)min(max(row, 0), d.Z - 1) * rowb; };
+  const int s0 = grp * g.spg, ns = min(g.spg, d.S - s0);
+
+  float p[NR][CPL], u[NR][CPL], w[NR][CPL];       // lambda_p, lambda_u, lambda_w
+  auto load = [&](int s) __attribute__((always_inline)) {
+    const long long so = (long long)s * d.plane;
+    const rsrc_t rP = rsrc(io.in + so, planeb), rU = rsrc(io.in + d.field + so, planeb);
+    const rsrc_t rW = rsrc(io.in + 2 * d.field + so, planeb);
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const unsigned o = off(zt + r);
+      const C x = ldc<CPL>(rP, vin, o), y = ldc<CPL>(rU, vin, o), z = ldc<CPL>(rW, vin, o);
+#pragma unroll
+      for (int q = 0; q < CPL; ++q) { p[r][q] = x.v[q]; u[r][q] = y.v[q]; w[r][q] = z.v[q]; }
+    }
+  };
+  auto clip = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+#pragma unroll
+      for (int q = 0; q < CPL; ++q) {
+        if (q) {
+          p[r][q] = ca + q < d.X ? p[r][q] : 0.f;
+          w[r][q] = ca + q < d.X ? w[r][q] : 0.f;
+        }
+        u[r][q] = ca + q < d.X - 1 ? u[r][q] : 0.f;
+      }
+    }
+  };
+  const bool right_edge = x0 - H + CPL * WAVE >= d.X - 2;
+  const bool edge = right_edge || zt + NR > d.Z - 2;
+
+  load(s0);
+  float k1[NR][CPL], a1[NR][CPL], k2[NR][CPL], a2[NR][CPL], k3[NR][CPL];
+  {
+    const rsrc_t rC = rsrc(coef_of(d, s0), 5u * planeb);
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const int row = zt + r;
+      const unsigned o = off(row);
+      const bool rp = row >= fs + 1 && row <= d.Z - 3, ru = row >= fs && row <= d.Z - 2;
+      const bool rw = row >= fs && row <= d.Z - 3;
+      const C m0 = ldc<CPL>(rC, vin, o), m1 = ldc<CPL>(rC, vin, planeb + o), m2 = ldc<CPL>(rC, vin, 2u * planeb + o);
+      const C m3 = ldc<CPL>(rC, vin, 3u * planeb + o), m4 = ldc<CPL>(rC, vin, 4u * planeb + o);
+#pragma unroll
+      for (int q = 0; q < CPL; ++q) {
+        const int c = ca + q;
+        const bool cp = c >= 2 && c <= d.X - 3, cu = c >= 1 && c <= d.X - 3, cw = c >= 1 && c <= d.X - 2;
+        k1[r][q] = rp && cp ? m0.v[q] : 1.f;
+        a1[r][q] = rp && cp ? m1.v[q] : 0.f;
+        k2[r][q] = ru && cu ? m2.v[q] : 1.f;
+        k3[r][q] = rw && cw ? m4.v[q] : 1.f;
+        a2[r][q] = (ru || rw) && (cu || cw) ? m3.v[q] : 0.f;   // (column X-2 and row Z-2: the edge variant)
+      }
+    }
+  }
+  // rows of this wavefront that hold receivers: their record adjoints enter every lane of the
+  // tile, halo included
+  unsigned rbits = 0;
+  if (io.rmap) {
+    const int row = zt + lane;
+    const bool mine = lane < NR && row >= 0 && row < d.Z;
+    rbits = (unsigned)__ballot(mine && io.rmap[mine ? row : 0] > 0);
+  }
+  const bool one_row = rbits && !(rbits & (rbits - 1));
+  const bool fsw = d.fsurf && tzi == 0 && wv == H / NR;     // this wavefront holds rows fs-1 .. fs+1
+  constexpr int RF = H % NR;
+  float ga1[NR][CPL] = {}, ga2[A2 ? NR : 1][CPL] = {};
+
+  auto march = [&](auto edge_) __attribute__((always_inline)) {
+  constexpr bool EDGE = decltype(edge_)::value;
+  for (int j = 0; j < ns; ++j) {
+    const int s = s0 + j;
+    // receiver slot of this lane's columns in a row, as a byte offset into a step's records
+    auto slots = [&](int r, unsigned (&v)[CPL]) __attribute__((always_inline)) {
+      const C m = ldc<CPL>(rsrc(io.rmap + d.Z, planeb), vin, off(zt + r));
+#pragma unroll
+      for (int q = 0; q < CPL; ++q) {
+        const int idx = __builtin_bit_cast(int, m.v[q]);
+        v[q] = vin != DROP && ca + q < d.X && idx >= 0 ? 4u * (unsigned)idx : DROP;
+      }
+    };
+    const float *const gr[3] = {io.g_p, FULL ? io.g_u : nullptr, FULL ? io.g_w : nullptr};
+    auto rec_at = [&](int c, int i) -> rsrc_t {   // records of component c in reversed step i
+      return rsrc(gr[c] ? gr[c] + ((long long)s * d.nt + io.t - i) * d.nrec : nullptr, gr[c] ? 4u * (unsigned)d.nrec : 0u);
+    };
+    if (one_row) {   // a line of receivers: all steps' values of the row are fetched up front
+      unsigned v[CPL];
+      slots(__builtin_ctz(rbits), v);
+#pragma unroll
+      for (int c = 0; c < NG; ++c)
+#pragma unroll
+        for (int i = 0; i < TK; ++i) {
+          C x{};
+          if (i < io.n) {
+#pragma unroll
+            for (int q = 0; q < CPL; ++q) x.v[q] = bld(rec_at(c, i), v[q], 0u);
+          }
+          srec[wv][c][i][lane] = x;
+        }
+    }
+    clip();
+    const int zs = scalar_ld(d.src_z + s), xs = scalar_ld(d.src_x + s);
+    const bool src_here = FULL && io.grad_src && zs >= zt && zs < zt + NR;
+    auto row_of = [&](const float (&x)[CPL]) { C c; for (int q = 0; q < CPL; ++q) c.v[q] = x[q]; return c; };
+#pragma unroll 1
+    for (int i = 0; i < io.n; ++i) {
+      const long long fi = (long long)s * d.plane - (long long)i * d.field;
+      C im[NR];
+      if (io.grad_a1) {
+        const float *const img = io.img_d + fi;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) im[r] = ldc<CPL>(rsrc(img, span(ownbits, r)), vout, off(zt + r));
+      }
+      // pressures of rows -1 .. NR+1 after the step: one lane column leaves the registers to fetch
+      // them this early
+      C q0[A2 ? NR + 3 : 1];
+      auto load_p = [&]() __attribute__((always_inline)) {
+        const float *const imp = io.img_p + fi;
+#pragma unroll
+        for (int r = 0; r < NR + 3; ++r) q0[r] = ldc<CPL>(rsrc(imp, planeb), vin, off(zt + r - 1));
+      };
+      if constexpr (A2 && CPL == 1) load_p();
+      // the record adjoints of the step
+      if (rbits) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          if ((rbits >> r) & 1u) {
+            C x[NG];
+            if (one_row) {
+#pragma unroll
+              for (int c = 0; c < NG; ++c) x[c] = srec[wv][c][i][lane];
+            } else {
+              unsigned v[CPL];
+              slots(r, v);
+#pragma unroll
+              for (int c = 0; c < NG; ++c)
+#pragma unroll
+                for (int q = 0; q < CPL; ++q) x[c].v[q] = bld(rec_at(c, i), v[q], 0u);
+            }
+#pragma unroll
+            for (int q = 0; q < CPL; ++q) {
+              p[r][q] = p[r][q] + x[0].v[q];
+              if constexpr (FULL) {
+                u[r][q] = u[r][q] + x[1].v[q];
+                w[r][q] = w[r][q] + x[2].v[q];
+              }
+            }
+          }
+      }
+      if (fsw) {   // stage 6 transposed: row fs gathers row fs-1
+#pragma unroll
+        for (int q = 0; q < CPL; ++q) {
+          w[RF + 1][q] = w[RF + 1][q] + w[RF][q];
+          w[RF][q] = 0.f;
+        }
+      }
+      // stages 5 and 4 transposed: lambda_p3
+      auto fw = [&](int r, int q) __attribute__((always_inline)) -> float {
+        if (EDGE && zt + r > d.Z - 3) return 0.f;
+        return a2[r][q] * w[r][q];
+      };
+      {
+        C x, y, z;
+#pragma unroll
+        for (int q = 0; q < CPL; ++q) { x.v[q] = fw(0, q); y.v[q] = fw(NR - 2, q); z.v[q] = fw(NR - 1, q); }
+        sw[wv + 1][0][lane] = x;
+        sw[wv + 1][1][lane] = y;
+        sw[wv + 1][2][lane] = z;
+      }
+      lds_barrier();
+      const C wa2 = sw[wv][1][lane], wa1 = sw[wv][2][lane], wb = sw[wv + 2][0][lane];
+      {
+        float f[NR + 3][CPL];   // a2 lambda_w of rows -2 .. NR
+#pragma unroll
+        for (int r = 0; r < NR + 3; ++r)
+#pragma unroll
+          for (int q = 0; q < CPL; ++q)
+            f[r][q] = r == 0 ? wa2.v[q] : r == 1 ? wa1.v[q] : r == NR + 2 ? wb.v[q] : fw(r - 2, q);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          __builtin_amdgcn_sched_barrier(0);
+          float fu[CPL], dx1[CPL], dx2[CPL];    // fu[j-1] - fu[j], fu[j-2] - fu[j+1]
+#pragma unroll
+          for (int q = 0; q < CPL; ++q) {
+            fu[q] = a2[r][q] * u[r][q];
+            if constexpr (EDGE) fu[q] = ca + q <= d.X - 3 ? fu[q] : 0.f;
+          }
+          if constexpr (CPL == 2) {
+            const float l0 = from_left(fu[0]), l1 = from_left(fu[1]), r0 = from_right(fu[0]);
+            dx1[0] = l1 - fu[0]; dx2[0] = l0 - fu[1];
+            dx1[1] = fu[0] - fu[1]; dx2[1] = l1 - r0;
+          } else {
+            const float l1 = from_left(fu[0]), l2 = from_left(l1);
+            dx1[0] = l1 - fu[0]; dx2[0] = l2 - from_right(fu[0]);
+          }
+#pragma unroll
+          for (int q = 0; q < CPL; ++q) {
+            const float dxt = C1 * dx1[q] + C2 * dx2[q];
+            const float dzt = C1 * (f[r + 1][q] - f[r + 2][q]) + C2 * (f[r][q] - f[r + 3][q]);
+            p[r][q] = p[r][q] - (dxt + dzt);
+          }
+        }
+      }
+      if (fsw) {   // stage 3 transposed
+#pragma unroll
+        for (int q = 0; q < CPL; ++q) {
+          p[RF + 2][q] = p[RF + 2][q] - p[RF][q];
+          p[RF][q] = 0.f;
+        }
+      }
+      if (FULL && src_here) {   // stage 2 transposed
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          if (zs == zt + r && ((ownbits >> r) & 1u)) {
+#pragma unroll
+            for (int q = 0; q < CPL; ++q)
+              if (own && ca + q == xs) io.grad_src[(long long)s * d.nt + io.t - i] = p[r][q];
+          }
+      }
+      if (io.grad_a1) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+          for (int q = 0; q < CPL; ++q) ga1[r][q] -= p[r][q] * im[r].v[q];
+      }
+      {
+        C x, y, z;
+#pragma unroll
+        for (int q = 0; q < CPL; ++q) {
+          x.v[q] = a1[0][q] * p[0][q]; y.v[q] = a1[1][q] * p[1][q]; z.v[q] = a1[NR - 1][q] * p[NR - 1][q];
+        }
+        sg[wv + 1][0][lane] = x;
+        sg[wv + 1][1][lane] = y;
+        sg[wv + 1][2][lane] = z;
+      }
+      if constexpr (A2) {   // zero-lag image of the velocity updates: the pressures after step t
+        if constexpr (CPL > 1) load_p();
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          const C &pc = q0[r + 1];
+          float dx1[CPL], dx2[CPL];
+          if constexpr (CPL == 2) {
+            const float l1 = from_left(pc.v[1]), r0 = from_right(pc.v[0]), r1 = from_right(pc.v[1]);
+            dx1[0] = pc.v[1] - pc.v[0]; dx2[0] = r0 - l1;
+            dx1[1] = r0 - pc.v[1]; dx2[1] = r1 - pc.v[0];
+          } else {
+            const float r1 = from_right(pc.v[0]);
+            dx1[0] = r1 - pc.v[0]; dx2[0] = from_right(r1) - from_left(pc.v[0]);
+          }
+#pragma unroll
+          for (int q = 0; q < CPL; ++q) {
+            float tu = u[r][q] * (C1 * dx1[q] + C2 * dx2[q]);
+            float tw = w[r][q] * (C1 * (q0[r + 2].v[q] - pc.v[q]) + C2 * (q0[r + 3].v[q] - q0[r].v[q]));
+            if constexpr (EDGE) {
+              tu = ca + q <= d.X - 3 ? tu : 0.f;
+              tw = zt + r <= d.Z - 3 ? tw : 0.f;
+            }
+            ga2[r][q] -= tu;
+            ga2[r][q] -= tw;
+          }
+        }
+      }
+      lds_barrier();
+      // stage 1 transposed and the adjoint state before the step
+      const C gm = sg[wv][2][lane], gb1 = sg[wv + 2][0][lane], gb2 = sg[wv + 2][1][lane];
+      {
+        float gg[NR + 3][CPL];   // a1 lambda_p of rows -1 .. NR+1
+#pragma unroll
+        for (int r = 0; r < NR + 3; ++r)
+#pragma unroll
+          for (int q = 0; q < CPL; ++q)
+            gg[r][q] = r == 0 ? gm.v[q] : r == NR + 1 ? gb1.v[q] : r == NR + 2 ? gb2.v[q] : a1[r - 1][q] * p[r - 1][q];
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          __builtin_amdgcn_sched_barrier(0);
+          const float (&gc)[CPL] = gg[r + 1];
+          float dx1[CPL], dx2[CPL];    // g[j] - g[j+1], g[j-1] - g[j+2]
+          if constexpr (CPL == 2) {
+            const float l1 = from_left(gc[1]), r0 = from_right(gc[0]), r1 = from_right(gc[1]);
+            dx1[0] = gc[0] - gc[1]; dx2[0] = l1 - r0;
+            dx1[1] = gc[1] - r0; dx2[1] = gc[0] - r1;
+          } else {
+            const float r1 = from_right(gc[0]);
+            dx1[0] = gc[0] - r1; dx2[0] = from_left(gc[0]) - from_right(r1);
+          }
+#pragma unroll
+          for (int q = 0; q < CPL; ++q) {
+            p[r][q] = k1[r][q] * p[r][q];
+            u[r][q] = k2[r][q] * u[r][q] - (C1 * dx1[q] + C2 * dx2[q]);
+            w[r][q] = k3[r][q] * w[r][q] - (C1 * (gc[q] - gg[r + 2][q]) + C2 * (gg[r][q] - gg[r + 3][q]));
+            if constexpr (EDGE) {
+              u[r][q] = ca + q < d.X - 1 ? u[r][q] : 0.f;
+              w[r][q] = zt + r < d.Z - 1 ? w[r][q] : 0.f;
+            }
+          }
+        }
+      }
+    }
+    {
+      const long long so = (long long)s * d.plane;
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        const unsigned o = off(zt + r), b = span(ownbits, r);
+        stc<CPL>(p[r], rsrc(io.out + so, b), vout, o);
+        stc<CPL>(u[r], rsrc(io.out + d.field + so, b), vout, o);
+        stc<CPL>(w[r], rsrc(io.out + 2 * d.field + so, span(wbits, r)), vout, o);
+      }
+    }
+    if (j + 1 < ns) load(s + 1);
+  }
+  };
+  if (edge) march(std::true_type{}); else march(std::false_type{});
+  // the images of all steps and shots into the group's planes: points of the update windows only
+  auto add = [&](float *plane, const float (&sum)[NR][CPL], int r0, int r1, int c0, int c1) __attribute__((always_inline)) {
+    const unsigned b = ownbits & bits(r0, r1);
+    C old[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) old[r] = ldc<CPL>(rsrc(plane, span(b, r)), vout, off(zt + r));
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      float v[CPL];
+#pragma unroll
+      for (int q = 0; q < CPL; ++q) v[q] = old[r].v[q] + (ca + q >= c0 && ca + q < c1 ? sum[r][q] : 0.f);
+      stc<CPL>(v, rsrc(plane, span(b, r)), vout, off(zt + r));
+    }
+  };
+  if (io.grad_a1) add(io.grad_a1 + (long long)grp * d.plane, ga1, fs + 1, d.Z - 2, 2, d.X - 2);
+  if constexpr (A2) add(io.grad_a2 + (long long)grp * d.plane, ga2, fs, d.Z - 1, 1, d.X - 1);
+}
+
 }  // namespace tile

@@ -200,6 +200,12 @@ class AcousticGeometry:
         return bool(self.fuse_steps) and not (self.shots_per_block or self.adj_shots_per_block or self.row_unroll
                                               or self.tile_z)
 
+    def adjoint_tiled(self, need_a2: bool) -> bool:
+        """Whether the adjoint does too: with the rho gradient on up to 1536 tiles of 40 x 40
+        points and shot groups, as the library chooses."""
+        tiles = -(-self.X // 40) * -(-(self.Z - int(self.layout.zbase)) // 40) * -(-self.S // self.gradient_group)
+        return self.tiled and (not need_a2 or tiles <= 1536)
+
     @property
     def gradient_group(self) -> int:
         """Consecutive shots that share one gradient accumulator plane in the adjoint."""
@@ -514,8 +520,11 @@ def run_backward(geom: AcousticGeometry, coef: torch.Tensor, src: torch.Tensor, 
         else:
             call = lambda: nat.check(lib.adfwi_acoustic_adjoint(ctypes.byref(d), ctypes.byref(aa), stream),
                                      "adfwi_acoustic_adjoint")
-        TIMELINE.call("adjoint", "ac_adj_pair" if fused else "ac_adj_step", (n + 1) // 2 if fused else n, dev,
-                      call, steps=n)
+        if fused and geom.adjoint_tiled(need_a2):
+            name, launches = "ac_adj_tile", -(-n // TILE_STEPS)
+        else:
+            name, launches = "ac_adj_pair" if fused else "ac_adj_step", (n + 1) // 2 if fused else n
+        TIMELINE.call("adjoint", name, launches, dev, call, steps=n)
         lam = lw[0] if aa.lam_out == lw[0].data_ptr() else lw[1]
         kept = seg_image = seg_image_p = None     # a kept segment's images are free for reuse now
     if group_planes:
