@@ -389,10 +389,12 @@ __global__ void el_gather(ElDev d, const float *__restrict__ st, float *__restri
 // every field, 4/tz of its loads.
 constexpr int ETZA = 8;   // strip rows of the adjoints that keep a per-strip LDS gradient slab
 
-template <bool ANISO, bool INJ>
-__global__ __launch_bounds__(ENT) void el_adj_step(ElDev d, const float *__restrict__ lin, float *__restrict__ lout,
-                                                   const float *__restrict__ fv, const float *__restrict__ fsn, int t,
-                                                   float *__restrict__ gacc, float *__restrict__ gsrc, ElInj inj) {
+// TOT: the forward wavefield comes as the five totals (a trace of the tile kernels) instead of the
+// ten splits: half the bytes, and the sums the step would form itself.
+template <bool ANISO, bool INJ, bool TOT>
+__device__ __forceinline__ void el_adj_body(const ElDev &d, const float *__restrict__ lin, float *__restrict__ lout,
+                                            const float *__restrict__ fv, const float *__restrict__ fsn, int t,
+                                            float *__restrict__ gacc, float *__restrict__ gsrc, const ElInj &inj) {
   constexpr int NGF = ANISO ? 8 : 6;
   // gradient terms of the rows finished in one iteration, per wavefront, double-buffered by
   // iteration parity (one barrier per iteration keeps a buffer from being rewritten early)
@@ -424,8 +426,10 @@ __global__ __launch_bounds__(ENT) void el_adj_step(ElDev d, const float *__restr
   auto rb = [&](int k) -> unsigned { return (unsigned)min(max(k, 0), zmax) * rowb; };
   const rsrc_t rLi = rsrc(lin, (unsigned)NFIELD * fieldb);
   const rsrc_t rLo = rsrc(lout, (unsigned)NFIELD * fieldb);
-  const rsrc_t rFv = rsrc(fv, (unsigned)NFIELD * fieldb);
-  const rsrc_t rFs = rsrc(fsn, (unsigned)NFIELD * fieldb);
+  constexpr int NFV = TOT ? 2 : 4, NFS = TOT ? 3 : 6;          // velocity / stress planes of the forward state
+  constexpr int FV0 = TOT ? (int)VX : (int)VX_X, FS0 = TOT ? (int)TXX : (int)TXX_X;
+  const rsrc_t rFv = rsrc(fv, (unsigned)(TOT ? NFIELD5 : NFIELD) * fieldb);
+  const rsrc_t rFs = rsrc(fsn, (unsigned)(TOT ? NFIELD5 : NFIELD) * fieldb);
   const rsrc_t rC = rsrc(d.coef, (unsigned)NCOEF * planeb);
   // rows z0-4 .. z0+tz+3 are read (tz <= 64)
   const adfwi::RowMask rrows = adfwi::receiver_rows(INJ ? inj.map : nullptr, d.Z, z0 - 4, lane);
@@ -497,8 +501,11 @@ __global__ __launch_bounds__(ENT) void el_adj_step(ElDev d, const float *__restr
       const int rr = __builtin_amdgcn_readfirstlane(rr_);   // uniform (a rolled loop's counter)
       const unsigned o = rb(rr);
       const bool in_grid = rr >= 0 && rr <= zmax;
-      const float a = bld(rFv, vc, F(VX_X) + o) + bld(rFv, vc, F(VX_Z) + o);
-      const float b = bld(rFv, vc, F(VZ_X) + o) + bld(rFv, vc, F(VZ_Z) + o);
+      float a = bld(rFv, vc, F(FV0) + o), b = bld(rFv, vc, F(FV0 + NFV / 2) + o);
+      if constexpr (!TOT) {
+        a = a + bld(rFv, vc, F(FV0 + 1) + o);
+        b = b + bld(rFv, vc, F(FV0 + 3) + o);
+      }
       fvx = in_grid ? a : 0.f;
       fvz = in_grid ? b : 0.f;
       ea = eb = ec = ed = 0.f;
@@ -536,7 +543,7 @@ __global__ __launch_bounds__(ENT) void el_adj_step(ElDev d, const float *__restr
     // forward velocity splits, the velocity adjoints and the buoyancies; row k of the stress
     // adjoints, the moduli and the forward stress splits; row k-2 of the velocity adjoints
     struct Row {
-      float fv[4], lv[4], b[2], ls[6], cm[ANISO ? 6 : 4], fs[6];
+      float fv[NFV], lv[4], b[2], ls[6], cm[ANISO ? 6 : 4], fs[NFS];
     };
     // velocity adjoints of rows k-2 .. k+2 as loaded (the row k-2 ones are the old values the
     // velocity stage needs, so they are not loaded a second time)
@@ -545,7 +552,7 @@ __global__ __launch_bounds__(ENT) void el_adj_step(ElDev d, const float *__restr
       if (!active) return;
       const unsigned o2 = rb(k + 2), o0 = rb(k);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) R.fv[q] = bld(rFv, vc, F(VX_X + q) + o2);
+      for (int q = 0; q < NFV; ++q) R.fv[q] = bld(rFv, vc, F(FV0 + q) + o2);
 #pragma unroll
       for (int q = 0; q < 4; ++q) R.lv[q] = bld(rLi, vc, F(VX_X + q) + o2);
       R.b[0] = bld(rC, vc, BX * planeb + o2); R.b[1] = bld(rC, vc, BZ * planeb + o2);
@@ -557,7 +564,7 @@ __global__ __launch_bounds__(ENT) void el_adj_step(ElDev d, const float *__restr
         R.cm[4] = bld(rC, vc, C15 * planeb + o0); R.cm[5] = bld(rC, vc, C35 * planeb + o0);
       }
 #pragma unroll
-      for (int q = 0; q < 6; ++q) R.fs[q] = bld(rFs, vc, F(TXX_X + q) + o0);
+      for (int q = 0; q < NFS; ++q) R.fs[q] = bld(rFs, vc, F(FS0 + q) + o0);
     };
     Row cur;
     load(z0 - 2, cur);
@@ -608,8 +615,13 @@ __global__ __launch_bounds__(ENT) void el_adj_step(ElDev d, const float *__restr
         }
 #pragma unroll
         for (int q = 0; q < 4; ++q) lw[4][q] = cur.lv[q];
-        const float fvx = in_grid ? cur.fv[0] + cur.fv[1] : 0.f;
-        const float fvz = in_grid ? cur.fv[2] + cur.fv[3] : 0.f;
+        float fvx = cur.fv[0], fvz = cur.fv[NFV / 2];
+        if constexpr (!TOT) {
+          fvx = fvx + cur.fv[1];
+          fvz = fvz + cur.fv[3];
+        }
+        fvx = in_grid ? fvx : 0.f;
+        fvz = in_grid ? fvz : 0.f;
         float ea = 0.f, eb = 0.f, ec = 0.f, ed = 0.f;
         if (rr >= 2 && rr <= zw1 && cwin) {
           const float vz_w = d.dt / (d.dz * pzf(1, rr));
@@ -723,9 +735,12 @@ __global__ __launch_bounds__(ENT) void el_adj_step(ElDev d, const float *__restr
       // forward stress totals of row k (after the step), free surface once row 3 exists
       {
         const bool in_grid = k >= 0 && k <= zmax;
-        const float a = cur.fs[0] + cur.fs[1];
-        const float b = cur.fs[2] + cur.fs[3];
-        const float e = cur.fs[4] + cur.fs[5];
+        float a = cur.fs[0], b = cur.fs[NFS / 3], e = cur.fs[2 * NFS / 3];
+        if constexpr (!TOT) {
+          a = a + cur.fs[1];
+          b = b + cur.fs[3];
+          e = e + cur.fs[5];
+        }
         xx0 = xx1; xx1 = xx2; xx2 = in_grid ? a : 0.f;
         zz0 = zz1; zz1 = zz2; zz2 = zz3; zz3 = zz4; zz4 = in_grid ? b : 0.f;
         xz0 = xz1; xz1 = xz2; xz2 = xz3; xz3 = xz4; xz4 = in_grid ? e : 0.f;
@@ -796,6 +811,20 @@ __global__ __launch_bounds__(ENT) void el_adj_step(ElDev d, const float *__restr
       }
     }
   }
+}
+
+template <bool ANISO, bool INJ>
+__global__ __launch_bounds__(ENT) void el_adj_step(ElDev d, const float *__restrict__ lin, float *__restrict__ lout,
+                                                   const float *__restrict__ fv, const float *__restrict__ fsn, int t,
+                                                   float *__restrict__ gacc, float *__restrict__ gsrc, ElInj inj) {
+  el_adj_body<ANISO, INJ, false>(d, lin, lout, fv, fsn, t, gacc, gsrc, inj);
+}
+
+template <bool INJ>
+__global__ __launch_bounds__(ENT) void el_adj_totals(ElDev d, const float *__restrict__ lin, float *__restrict__ lout,
+                                                     const float *__restrict__ fv, const float *__restrict__ fsn, int t,
+                                                     float *__restrict__ gacc, float *__restrict__ gsrc, ElInj inj) {
+  el_adj_body<false, INJ, true>(d, lin, lout, fv, fsn, t, gacc, gsrc, inj);
 }
 
 // adds the record adjoints of step t to both splits of each recorded field (free-surface tzz
@@ -2285,6 +2314,8 @@ __global__ __launch_bounds__(ENT) void el3_abl_adj(ElDev d, const float *__restr
     }
 }
 
+#include "elastic_tile.hpp"
+
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
@@ -2371,6 +2402,42 @@ ElDev el_dev(const adfwi_elastic_desc *d, const adfwi_layout &L) {
   return v;
 }
 
+// ---- tiles (elastic_tile.hpp): up to two steps per launch of the 4th-order PML scheme without
+// C15 / C35, where the caller left the layout to the library, records (if any) go through the
+// receiver map, and a state set stays under the 2 GiB that dropped buffer accesses need
+bool el_tile_ok(const adfwi_elastic_desc *d, const ElDev &v, const adfwi_layout &L, bool recs) {
+  return !d->damping && v.nn == 2 && !d->aniso && d->shots_per_wave == 0 && d->tile_z == 0 &&
+         (!recs || d->rcv_map) && L.state_floats * 4 < ((int64_t)1 << 31) &&
+         (int64_t)NCOEF * d->nz * d->pitch * 4 < ((int64_t)1 << 31);
+}
+
+template <int NR, int NW>
+void launch_el_fwd_tile_c(const ElDev &v, hipStream_t st, const tile::FwdIO &io) {
+  constexpr int oz = tile::out_rows(NR * NW);
+  tile::Grid g;
+  g.ntx = (v.X - 4 + tile::OX - 1) / tile::OX;
+  g.ntz = (v.Z - 4 + oz - 1) / oz;
+  hipLaunchKernelGGL((tile::el_fwd_tile<NR, NW>), dim3((unsigned)(g.ntx * g.ntz * v.S)), dim3(NW * WAVE), 0, st, v, g, io);
+}
+
+// Tile heights: 32, 48 and 64 rows (20, 36 and 52 stored).  A launch whose workgroups all run at
+// once lasts as long as one of them, and a lower tile is done sooner: the lowest that gives at most
+// one workgroup per CU.  Above that, 32 rows again: two such workgroups fit a CU and overlap each
+// other's loads, stores and arithmetic, which outweighs their larger halo.  Measured, forward with
+// records, us per step, 32 / 48 / 64 rows: 122 x 240, 1 shot 6.1 / 7.9 / 9.4; 142 x 341, 6 shots
+// (294 / 168 / 126 workgroups) 10.4 / 8.6 / 10.2; 171 x 373, 8 shots (576 / 320 / 256) 14.2 / 15.3 /
+// 11.0; 242 x 680, 32 shots 81 / 119 / 106; 362 x 1040, 48 shots 267 / 390 / 336.
+void launch_el_fwd_tile(const ElDev &v, hipStream_t st, const tile::FwdIO &io) {
+  auto count = [&](int rows) {
+    const int oz = tile::out_rows(rows);
+    return (long long)((v.X - 4 + tile::OX - 1) / tile::OX) * ((v.Z - 4 + oz - 1) / oz) * v.S;
+  };
+  constexpr long long CUS = 256;
+  if (count(32) > CUS && count(48) <= CUS) launch_el_fwd_tile_c<4, 12>(v, st, io);
+  else if (count(32) > CUS && count(64) <= CUS) launch_el_fwd_tile_c<4, 16>(v, st, io);
+  else launch_el_fwd_tile_c<4, 8>(v, st, io);
+}
+
 }  // namespace
 
 extern "C" {
@@ -2393,7 +2460,7 @@ int adfwi_elastic_forward(const adfwi_elastic_desc *d, adfwi_elastic_fwd_args *a
   ADFWI_CHECK_ARG(!recs || (a->rec[0] && a->rec[1] && a->rec[2] && a->rec[3] && a->rec[4]),
                   "records must be all set or all NULL");
   if (recs && d->nrec > 0) ADFWI_CHECK_ARG(d->rcv_z && d->rcv_x, "null receiver table pointer");
-  ADFWI_CHECK_ARG(a->state_in && (a->trace || (a->work[0] && a->work[1] && a->work[0] != a->work[1])),
+  ADFWI_CHECK_ARG(a->state_in && ((a->trace && !a->trace_totals) || (a->work[0] && a->work[1] && a->work[0] != a->work[1])),
                   "state_in and two distinct work buffers (or a trace buffer) are required");
   ADFWI_CHECK_ARG(!(a->trace && a->ckpt), "trace and ckpt are exclusive");
   ADFWI_CHECK_ARG(a->t0 >= 0 && a->nsteps >= 0 && a->t0 + a->nsteps <= d->nt,
@@ -2412,6 +2479,30 @@ int adfwi_elastic_forward(const adfwi_elastic_desc *d, adfwi_elastic_fwd_args *a
     for (int q = 0; q < 5; ++q) rk.r[q] = a->rec[q];
   }
   const float *cur = a->state_in;
+  const bool tiles = el_tile_ok(d, v, L, recs && ng > 0);
+  ADFWI_CHECK_ARG(!a->trace_totals || (a->trace && tiles),
+                  "a trace of totals needs a trace buffer and the tile kernels (4th-order PML without C15 / C35, "
+                  "library tiling, a receiver map for records, state sets under 2 GiB)");
+  if (tiles && (!a->trace || a->trace_totals)) {
+    for (int k = 0; k < a->nsteps;) {
+      const int t = a->t0 + k;
+      int n = min(tile::TK, a->nsteps - k);
+      if (a->ckpt) n = min(n, a->ckpt_every - t % a->ckpt_every);   // up to the next checkpoint
+      float *nxt = (cur == a->work[0]) ? a->work[1] : a->work[0];
+      if (a->ckpt && (t + n) % a->ckpt_every == 0 && t + n < d->nt)
+        nxt = a->ckpt + (long long)((t + n) / a->ckpt_every - 1) * L.state_floats;
+      tile::FwdIO io;
+      io.in = cur; io.out = nxt; io.t = t; io.n = n;
+      io.trace = a->trace ? a->trace + (long long)k * NFIELD5 * L.field_floats : nullptr;
+      io.rec = rk;
+      launch_el_fwd_tile(v, st, io);
+      if ((rc = adfwi::check_launch("el_fwd_tile"))) return rc;
+      cur = nxt;
+      k += n;
+    }
+    a->state_out = cur;
+    return ADFWI_OK;
+  }
   for (int k = 0; k < a->nsteps; ++k) {
     const int t = a->t0 + k;
     float *nxt;
@@ -2466,8 +2557,7 @@ int adfwi_elastic_forward(const adfwi_elastic_desc *d, adfwi_elastic_fwd_args *a
   return ADFWI_OK;
 }
 
-int adfwi_elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a, adfwi_stream_t stream) {
-  if (int rc = adfwi::fault_injected("adfwi_elastic_adjoint")) return rc;
+static int elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a, adfwi_stream_t stream, bool totals) {
   adfwi_layout L;
   int rc = el_layout(d, &L);
   if (rc) return rc;
@@ -2483,6 +2573,9 @@ int adfwi_elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a
   const bool recs = a->grad_rec[0] || a->grad_rec[1] || a->grad_rec[2] || a->grad_rec[3] || a->grad_rec[4];
   if (recs && d->nrec > 0) ADFWI_CHECK_ARG(d->rcv_z && d->rcv_x, "null receiver table pointer");
   ElDev v = el_dev(d, L);
+  ADFWI_CHECK_ARG(!totals || (!d->damping && v.nn == 2 && !d->aniso),
+                  "a trace of totals belongs to the 4th-order PML scheme without C15 / C35");
+  const long long slot = totals ? NFIELD5 * L.field_floats : L.state_floats;
   // the free-surface transposes need rows 0..3 inside the first strip (every strip height here
   // is at least 8)
   // (damping scheme: strips of ETZA rows, so that no strip but the first reaches the
@@ -2534,8 +2627,8 @@ int adfwi_elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a
                            a->grad_rec[2], a->grad_rec[3], a->grad_rec[4], t);
       if ((rc = adfwi::check_launch("el_inject"))) return rc;
     }
-    const float *fv = i == 0 ? a->fwd0 : a->trace + (long long)(i - 1) * L.state_floats;
-    const float *fsn = a->trace + (long long)i * L.state_floats;
+    const float *fv = i == 0 ? a->fwd0 : a->trace + (long long)(i - 1) * slot;
+    const float *fsn = a->trace + (long long)i * slot;
     float *nxt = (cur == a->work[0]) ? a->work[1] : a->work[0];
     if (d->damping && v.nn > 2) {
       if (d->aniso)
@@ -2557,7 +2650,11 @@ int adfwi_elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a
       if ((rc = adfwi::check_launch("el3_adj_step"))) return rc;
     } else {
       float *gc = a->grad_coef, *gs = a->grad_src;
-      if (d->aniso && fused)
+      if (totals && fused)
+        hipLaunchKernelGGL(el_adj_totals<true>, grid, block, 0, st, v, cur, nxt, fv, fsn, t, gc, gs, ij);
+      else if (totals)
+        hipLaunchKernelGGL(el_adj_totals<false>, grid, block, 0, st, v, cur, nxt, fv, fsn, t, gc, gs, ij);
+      else if (d->aniso && fused)
         hipLaunchKernelGGL((el_adj_step<true, true>), grid, block, 0, st, v, cur, nxt, fv, fsn, t, gc, gs, ij);
       else if (d->aniso)
         hipLaunchKernelGGL((el_adj_step<true, false>), grid, block, 0, st, v, cur, nxt, fv, fsn, t, gc, gs, ij);
@@ -2565,12 +2662,22 @@ int adfwi_elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a
         hipLaunchKernelGGL((el_adj_step<false, true>), grid, block, 0, st, v, cur, nxt, fv, fsn, t, gc, gs, ij);
       else
         hipLaunchKernelGGL((el_adj_step<false, false>), grid, block, 0, st, v, cur, nxt, fv, fsn, t, gc, gs, ij);
-      if ((rc = adfwi::check_launch("el_adj_step"))) return rc;
+      if ((rc = adfwi::check_launch(totals ? "el_adj_totals" : "el_adj_step"))) return rc;
     }
     cur = nxt;
   }
   a->lam_out = cur;
   return ADFWI_OK;
+}
+
+int adfwi_elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a, adfwi_stream_t stream) {
+  if (int rc = adfwi::fault_injected("adfwi_elastic_adjoint")) return rc;
+  return elastic_adjoint(d, a, stream, false);
+}
+
+int adfwi_elastic_adjoint_totals(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a, adfwi_stream_t stream) {
+  if (int rc = adfwi::fault_injected("adfwi_elastic_adjoint_totals")) return rc;
+  return elastic_adjoint(d, a, stream, true);
 }
 
 }  // extern "C"

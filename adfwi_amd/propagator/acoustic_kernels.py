@@ -98,12 +98,12 @@ class Timeline:
 TILE_STEPS = 4    # steps per launch of the tile kernels
 
 
-def tile_launches(t0: int, n: int, ckpt_every: int) -> int:
-    """Launches of the tile kernels for steps t0 .. t0+n-1: at most TILE_STEPS steps each, none
-    past a checkpoint."""
+def tile_launches(t0: int, n: int, ckpt_every: int, steps: int = TILE_STEPS) -> int:
+    """Launches of the tile kernels for steps t0 .. t0+n-1: at most `steps` steps each, none past
+    a checkpoint."""
     launches = k = 0
     while k < n:
-        m = min(TILE_STEPS, n - k)
+        m = min(steps, n - k)
         if ckpt_every:
             m = min(m, ckpt_every - (t0 + k) % ckpt_every)
         launches += 1

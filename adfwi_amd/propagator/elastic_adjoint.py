@@ -10,7 +10,8 @@ from typing import List, Optional, Sequence
 import torch
 
 from .. import _native as nat
-from .acoustic_kernels import TIMELINE
+from .acoustic_kernels import TIMELINE, tile_launches
+from .elastic_kernels import TILE_STEPS
 
 NCOEF = 8
 
@@ -18,13 +19,14 @@ NCOEF = 8
 def run_backward(geom, coef: torch.Tensor, src: torch.Tensor, pml_x: Optional[torch.Tensor],
                  pml_z: Optional[torch.Tensor], scalars, ckpt: Optional[torch.Tensor], k: int,
                  g_rec: Sequence[Optional[torch.Tensor]], needs: Sequence[bool], damp: Optional[torch.Tensor] = None,
-                 traces: Optional[dict] = None):
+                 traces: Optional[dict] = None, totals: Optional[bool] = None):
     """Adjoint of all nt steps.
 
     ckpt: the forward's checkpoints (slot j = state after step (j+1)k-1), g_rec: five (S, nt, R)
     record adjoints (txx, tzz, txz, vx, vz; None = zero).  traces: {segment: per-step states}
     kept by run_forward(resident=...); those segments are not recomputed, and each is released
-    once the segment before it no longer needs its last state.  Returns (list of 8 (Z, pitch)
+    once the segment before it no longer needs its last state.  totals: whether traces hold the
+    five totals of a state instead of its fields (run_forward's; default geom.tiled).  Returns (list of 8 (Z, pitch)
     gradients of the padded coefficient planes C11, C13, C33, C55, bx, bz, C15, C35 -- None
     where not needed -- and the (S, nt) wavelet gradient or None).
     """
@@ -37,8 +39,13 @@ def run_backward(geom, coef: torch.Tensor, src: torch.Tensor, pml_x: Optional[to
     first_resident = min(traces) if traces else nseg
     if first_resident > 1 and (ckpt is None or ckpt.shape[0] < first_resident - 1):
         raise RuntimeError("the forward pass kept no checkpoints for the adjoint")
+    totals = geom.tiled if totals is None else bool(totals)
     lam = geom.state(2)
-    trace = geom.state(min(k, nt)) if len(traces) < nseg else None
+    trace = geom.trace(min(k, nt), totals) if len(traces) < nseg else None
+    # with totals: ping-pong states of the recomputation, and the totals before a segment
+    rw = geom.state(2) if totals and trace is not None else None
+    before = geom.trace(1, True)[0] if totals else None
+    adjoint = lib.adfwi_elastic_adjoint_totals if totals else lib.adfwi_elastic_adjoint
     zero = None
     gacc = torch.zeros(int(L.accum_floats), device=dev, dtype=torch.float32)
     gsrc = torch.zeros((S, nt), device=dev, dtype=torch.float32)
@@ -64,9 +71,20 @@ def run_backward(geom, coef: torch.Tensor, src: torch.Tensor, pml_x: Optional[to
             fa.state_in = fwd0.data_ptr()
             fa.trace = trace.data_ptr()
             fa.t0, fa.nsteps = t0, n
-            TIMELINE.call("recompute", geom.kernel_names[0], n, dev, lambda: nat.check(
+            if totals:
+                fa.trace_totals = 1
+                fa.work[0], fa.work[1] = rw[0].data_ptr(), rw[1].data_ptr()
+            TIMELINE.call("recompute", "el_fwd_tile" if totals else geom.kernel_names[0],
+                          tile_launches(t0, n, 0, TILE_STEPS) if totals else n, dev, lambda: nat.check(
                 lib.adfwi_elastic_forward(ctypes.byref(d), ctypes.byref(fa), stream),
-                "adfwi_elastic_forward (recompute)"))
+                "adfwi_elastic_forward (recompute)"), steps=n)
+        if totals and seg - 1 not in traces:   # (a resident segment's last totals are there already)
+            if seg == 0:
+                before.zero_()
+            else:                              # vx and vz, which the first reversed step reads
+                torch.add(fwd0[6], fwd0[7], out=before[3])
+                torch.add(fwd0[8], fwd0[9], out=before[4])
+            fwd0 = before
         aa = nat.ElasticAdjArgs()
         aa.lam_in = cur.data_ptr()
         aa.work[0], aa.work[1] = lam[0].data_ptr(), lam[1].data_ptr()
@@ -76,8 +94,8 @@ def run_backward(geom, coef: torch.Tensor, src: torch.Tensor, pml_x: Optional[to
             aa.grad_rec[i] = None if g[i] is None else g[i].data_ptr()
         aa.grad_coef = gacc.data_ptr()
         aa.grad_src = gsrc.data_ptr()
-        TIMELINE.call("adjoint", geom.kernel_names[1], n, dev, lambda: nat.check(
-            lib.adfwi_elastic_adjoint(ctypes.byref(d), ctypes.byref(aa), stream), "adfwi_elastic_adjoint"))
+        TIMELINE.call("adjoint", "el_adj_totals" if totals else geom.kernel_names[1], n, dev, lambda: nat.check(
+            adjoint(ctypes.byref(d), ctypes.byref(aa), stream), "adfwi_elastic_adjoint"))
         cur = lam[0] if aa.lam_out == lam[0].data_ptr() else lam[1]
         traces.pop(seg, None)              # done; segment seg + 1, which read its last state, too
         seg_trace = fwd0 = None

@@ -17,10 +17,11 @@ import torch
 
 from .. import _native as nat
 from .acoustic_kernels import (PITCH_ALIGN, TIMELINE, ResidentSet, checkpoint_interval, replicate_pad,
-                               resident_budget_bytes)
+                               resident_budget_bytes, tile_launches)
 
 NAMES = ("txx", "tzz", "txz", "vx", "vz")
 NFIELD = 10
+TILE_STEPS = 2    # steps per launch of the tile kernels
 
 
 def DiffCoef(order: int, grid_scheme: str) -> torch.Tensor:
@@ -111,6 +112,24 @@ class ElasticGeometry:
         nat.check(nat.load().adfwi_elastic_get_layout(ctypes.byref(d), ctypes.byref(self.layout)),
                   "adfwi_elastic_get_layout")
 
+    @property
+    def tiled(self) -> bool:
+        """Whether the forward runs on the tile kernels (two steps per launch; a trace then holds
+        the five totals of a step instead of its ten splits): the 4th-order PML scheme without
+        C15 / C35, library tiling, a receiver map if there are receivers, state sets and
+        coefficients under 2 GiB."""
+        plane = 4 * self.Z * self.pitch
+        return (not self.damping and self.nn == 2 and not self.aniso and not self.shots_per_wave and not self.tile_z
+                and (self.R == 0 or self.rcv_map is not None) and self.nfield * self.S * plane < 1 << 31
+                and 8 * plane < 1 << 31)
+
+    def trace_fields(self, totals: bool) -> int:
+        return 5 if totals else self.nfield
+
+    def trace(self, n: int, totals: bool) -> torch.Tensor:
+        return torch.zeros((n, self.trace_fields(totals), self.S, self.Z, self.pitch), device=self.device,
+                           dtype=torch.float32)
+
     def _receiver_map(self, rcv_z: np.ndarray, rcv_x: np.ndarray) -> Optional[torch.Tensor]:
         """[Z] receivers per row, then [Z][pitch] receiver index (-1 elsewhere); None without
         receivers, when receivers repeat a point (their records are then taken and their adjoints
@@ -196,15 +215,17 @@ def resident_trace_segments(geom: ElasticGeometry, k: int) -> int:
     """How many of the last checkpoint segments keep their per-step states from the forward pass
     (the backward then skips their recomputation): at most geom.resident_traces (0 = none; None =
     as many as resident_budget_bytes allows once the checkpoints, the backward's recompute trace
-    and its three states are set aside)."""
+    and its five states are set aside)."""
     nseg = -(-geom.nt // k)
     cap = geom.resident_traces
     if cap == 0:
         return 0
     state_bytes = int(geom.layout.state_floats) * 4
     seg_bytes = k * state_bytes
+    if getattr(geom, "tiled", False):     # five totals instead of ten splits
+        seg_bytes //= 2
     if cap is None:
-        cap = resident_budget_bytes(geom.device, (nseg + 3) * state_bytes + seg_bytes) // seg_bytes
+        cap = resident_budget_bytes(geom.device, (nseg + 5) * state_bytes + seg_bytes) // seg_bytes
     return int(max(0, min(cap, nseg)))
 
 
@@ -226,7 +247,8 @@ def run_forward(geom: ElasticGeometry, coef, pml_x, pml_z, src, scalars, *, reco
                 ckpt_every: int = 0, damp=None, resident: int = 0):
     """All nt steps from a zero state.  Returns dict(rec=[5 x (S, nt, R)] or None,
     energy=[5 x (Z, X)] summed over the states after the steps in energy_ends, ckpt,
-    traces={segment: per-step states}).
+    traces={segment: per-step states}, totals: whether the traces hold five totals instead of the
+    state's fields, geom.tiled).
 
     resident > 0 (with ckpt_every): the last `resident` checkpoint segments write the state after
     each of their steps to a trace buffer of their own, which run_backward uses instead of
@@ -234,6 +256,7 @@ def run_forward(geom: ElasticGeometry, coef, pml_x, pml_z, src, scalars, *, reco
     lib = nat.load()
     dev = geom.device
     S, nt, R = geom.S, geom.nt, geom.R
+    totals = geom.tiled
     work = geom.state(2)
     k = int(ckpt_every)
     nseg = -(-nt // k) if k else 1
@@ -249,7 +272,7 @@ def run_forward(geom: ElasticGeometry, coef, pml_x, pml_z, src, scalars, *, reco
     poison = os.environ.get("ADFWI_POISON_RESIDENT") == "1"
 
     def trace_buffer(n):
-        t = torch.empty((n, geom.nfield, S, geom.Z, geom.pitch), device=dev, dtype=torch.float32)
+        t = torch.empty((n, geom.trace_fields(totals), S, geom.Z, geom.pitch), device=dev, dtype=torch.float32)
         if poison:
             t.fill_(float("nan"))
         w = geom.nn
@@ -262,7 +285,8 @@ def run_forward(geom: ElasticGeometry, coef, pml_x, pml_z, src, scalars, *, reco
     traces = ResidentSet((seg, trace_buffer(min(nt, (seg + 1) * k) - seg * k)) for seg in range(nseg - resident, nseg))
     if resident:
         state_bytes = int(geom.layout.state_floats) * 4
-        traces.hold(3 * state_bytes + (k * state_bytes if resident < nseg else 0))
+        traces.hold(5 * state_bytes + (k * state_bytes * geom.trace_fields(totals) // geom.nfield
+                                       if resident < nseg else 0))
     rec = [torch.zeros((S, nt, R), device=dev) for _ in range(5)] if record and R else None
     d = geom.desc(coef, pml_x, pml_z, src, scalars, damp)
     ends = sorted(set(energy_ends or [])) or [nt - 1]
@@ -280,6 +304,7 @@ def run_forward(geom: ElasticGeometry, coef, pml_x, pml_z, src, scalars, *, reco
         if t0 >= head:            # inside a resident segment: every state goes to its trace
             seg = t0 // k
             a.trace = traces[seg][t0 - seg * k].data_ptr()
+            a.trace_totals = int(totals)
         else:
             a.ckpt = None if ckpt is None else ckpt.data_ptr()
             a.ckpt_every = k if ckpt is not None else 0
@@ -287,15 +312,17 @@ def run_forward(geom: ElasticGeometry, coef, pml_x, pml_z, src, scalars, *, reco
         if rec is not None:
             for i in range(5):
                 a.rec[i] = rec[i].data_ptr()
-        TIMELINE.call("forward" if t0 < head else "forward+trace", geom.kernel_names[0], a.nsteps, dev,
+        launches = tile_launches(t0, a.nsteps, int(a.ckpt_every), TILE_STEPS) if totals else a.nsteps
+        TIMELINE.call("forward" if t0 < head else "forward+trace", "el_fwd_tile" if totals else geom.kernel_names[0],
+                      launches, dev,
                       lambda: nat.check(lib.adfwi_elastic_forward(ctypes.byref(d), ctypes.byref(a), stream),
-                                        "adfwi_elastic_forward"))
+                                        "adfwi_elastic_forward"), steps=a.nsteps)
         cur = _state_at(a.state_out, work, bufs)
         if energy_ends is not None and te in ends:
             e = _energy(cur, geom.X, geom.free_surface, geom.nn)
             energy = e if energy is None else [x + y for x, y in zip(energy, e)]
         t0 = te + 1
-    return {"rec": rec, "energy": energy, "ckpt": ckpt, "final": cur, "traces": traces}
+    return {"rec": rec, "energy": energy, "ckpt": ckpt, "final": cur, "traces": traces, "totals": totals}
 
 
 class ElasticWave(torch.autograd.Function):
@@ -319,6 +346,7 @@ class ElasticWave(torch.autograd.Function):
         res = run_forward(geom, coef, absorb[0], absorb[1], src, scalars, record=True, energy_ends=energy_ends,
                           ckpt_every=k if need_grad else 0, damp=absorb[2], resident=resident)
         ctx.traces = res["traces"] if need_grad else None
+        ctx.totals = res["totals"]
         rec = res["rec"] or [torch.zeros((geom.S, geom.nt, geom.R), device=geom.device) for _ in range(5)]
         ctx.geom, ctx.k, ctx.scalars = geom, k, scalars
         ctx.ckpt = res["ckpt"] if need_grad else None
@@ -337,7 +365,7 @@ class ElasticWave(torch.autograd.Function):
         coef, src, pml_x, pml_z = ctx.saved_tensors
         absorb = (None, None, pml_x) if ctx.geom.damping else (pml_x, pml_z, None)
         gcoef, gsrc = run_backward(ctx.geom, coef, src, absorb[0], absorb[1], ctx.scalars, ctx.ckpt, ctx.k, grads[:5],
-                                   ctx.needs_input_grad[:9], damp=absorb[2], traces=traces)
+                                   ctx.needs_input_grad[:9], damp=absorb[2], traces=traces, totals=ctx.totals)
         ctx.ckpt = None
         out = []
         for i, shp in enumerate(ctx.shapes):

@@ -417,7 +417,7 @@ def main():
                     + steps_by.get("forward+images", 0)) * BYTES_RECOMPUTE) * N * S
         elif name in ("ac_adj_step", "ac_adj_pair", "ac_adj_tile"):
             byts = d["steps"] * BYTES_ADJ * N * S
-        elif name in ("el_fwd_step", "el3_fwd_step"):
+        elif name in ("el_fwd_step", "el_fwd_tile", "el3_fwd_step"):
             byts = d["steps"] * EL_BYTES_FWD * N * S
         elif name in ("el_abl_fwd", "el3_abl_fwd"):
             byts = d["steps"] * EL_BYTES_FWD / 2 * N * S

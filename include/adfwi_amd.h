@@ -233,7 +233,11 @@ typedef struct adfwi_elastic_fwd_args {
   float *ckpt;             /* [n][10][S][Z][pitch] or NULL */
   int32_t ckpt_every;
   int32_t t0, nsteps;
-  int32_t reserved;
+  int32_t trace_totals;    /* 1: `trace` receives the five totals after every step (txx, tzz, txz, vx, vz
+                              as split sums, [nsteps][5][S][Z][pitch]) and the states go through
+                              work[]; only where adfwi_elastic_forward can run its tile kernels: 4th-order
+                              PML, aniso 0, shots_per_wave and tile_z 0, rcv_map given when records are
+                              taken, state sets under 2 GiB.  0: full states, as described at trace */
   float *rec[5];           /* txx, tzz, txz, vx, vz records [S][nt][R], or all NULL */
   float *trace;            /* [nsteps][10][S][Z][pitch] or NULL: the state after every step of the
                               call is written to its slot (work[] unused; ckpt must be NULL) */
@@ -264,6 +268,12 @@ typedef struct adfwi_elastic_adj_args {
  * zero-lag cross-correlation gradients of the padded coefficient fields.  Replaces the
  * autograd replay of step_forward_PML_4order (elastic_kernels.py:975-1008 checkpoints). */
 int adfwi_elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a, adfwi_stream_t stream);
+
+/* The same from a trace of totals (adfwi_elastic_fwd_args.trace_totals): a->trace holds
+ * [nsteps][5][S][Z][pitch] and a->fwd0 the totals before step t_hi-nsteps, [5][S][Z][pitch] (vx and
+ * vz are read).  Half the bytes of the forward wavefield; the gradients are the same bit for bit.
+ * 4th-order PML scheme with aniso 0. */
+int adfwi_elastic_adjoint_totals(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a, adfwi_stream_t stream);
 
 /* ------------------------------------------------------------------------ */
 /* Record post-processing                                                     */
