@@ -83,15 +83,18 @@ struct FwdIO {
   float *rec_p, *rec_u, *rec_w;
 };
 
-// workgroup -> (tile, shot group).  Blocks go round-robin to the 8 XCDs: every XCD takes a
-// contiguous run of (tile, group) with the groups of one tile next to each other, so that the
-// tile's coefficients are read from its L2 for all of them.
+// workgroup -> (tile, shot group): blocks go round-robin to the 8 XCDs, and every XCD takes a
+// contiguous run of a group's tiles, row by row, so that its L2 serves the halos neighbouring tiles
+// share and joins the ends of their rows, which share cache lines, before they are written back.
+// (With the groups of one tile next to each other instead, for the sake of its coefficients: 136
+// against 128 us per step forward and 190 against 168 adjoint on 464 x 1232 with 64 shots.)
 __device__ __forceinline__ void place(const Grid &g, int &tx, int &tz, int &grp) {
   const int n = (int)gridDim.x, b = (int)blockIdx.x;
   const int xcd = b & 7, per = n >> 3, rem = n & 7;
   const int logical = xcd * per + min(xcd, rem) + (b >> 3);
-  const int tl = logical / g.ngroups;
-  grp = logical - tl * g.ngroups;
+  const int nt = g.ntx * g.ntz;
+  grp = logical / nt;
+  const int tl = logical - grp * nt;
   tz = tl / g.ntx;
   tx = tl - tz * g.ntx;
 }
