@@ -389,12 +389,10 @@ __global__ void el_gather(ElDev d, const float *__restrict__ st, float *__restri
 // every field, 4/tz of its loads.
 constexpr int ETZA = 8;   // strip rows of the adjoints that keep a per-strip LDS gradient slab
 
-// TOT: the forward wavefield comes as the five totals (a trace of the tile kernels) instead of the
-// ten splits: half the bytes, and the sums the step would form itself.
-template <bool ANISO, bool INJ, bool TOT>
-__device__ __forceinline__ void el_adj_body(const ElDev &d, const float *__restrict__ lin, float *__restrict__ lout,
-                                            const float *__restrict__ fv, const float *__restrict__ fsn, int t,
-                                            float *__restrict__ gacc, float *__restrict__ gsrc, const ElInj &inj) {
+template <bool ANISO, bool INJ>
+__global__ __launch_bounds__(ENT) void el_adj_step(ElDev d, const float *__restrict__ lin, float *__restrict__ lout,
+                                                   const float *__restrict__ fv, const float *__restrict__ fsn, int t,
+                                                   float *__restrict__ gacc, float *__restrict__ gsrc, ElInj inj) {
   constexpr int NGF = ANISO ? 8 : 6;
   // gradient terms of the rows finished in one iteration, per wavefront, double-buffered by
   // iteration parity (one barrier per iteration keeps a buffer from being rewritten early)
@@ -426,10 +424,8 @@ __device__ __forceinline__ void el_adj_body(const ElDev &d, const float *__restr
   auto rb = [&](int k) -> unsigned { return (unsigned)min(max(k, 0), zmax) * rowb; };
   const rsrc_t rLi = rsrc(lin, (unsigned)NFIELD * fieldb);
   const rsrc_t rLo = rsrc(lout, (unsigned)NFIELD * fieldb);
-  constexpr int NFV = TOT ? 2 : 4, NFS = TOT ? 3 : 6;          // velocity / stress planes of the forward state
-  constexpr int FV0 = TOT ? (int)VX : (int)VX_X, FS0 = TOT ? (int)TXX : (int)TXX_X;
-  const rsrc_t rFv = rsrc(fv, (unsigned)(TOT ? NFIELD5 : NFIELD) * fieldb);
-  const rsrc_t rFs = rsrc(fsn, (unsigned)(TOT ? NFIELD5 : NFIELD) * fieldb);
+  const rsrc_t rFv = rsrc(fv, (unsigned)NFIELD * fieldb);
+  const rsrc_t rFs = rsrc(fsn, (unsigned)NFIELD * fieldb);
   const rsrc_t rC = rsrc(d.coef, (unsigned)NCOEF * planeb);
   // rows z0-4 .. z0+tz+3 are read (tz <= 64)
   const adfwi::RowMask rrows = adfwi::receiver_rows(INJ ? inj.map : nullptr, d.Z, z0 - 4, lane);
@@ -501,11 +497,8 @@ __device__ __forceinline__ void el_adj_body(const ElDev &d, const float *__restr
       const int rr = __builtin_amdgcn_readfirstlane(rr_);   // uniform (a rolled loop's counter)
       const unsigned o = rb(rr);
       const bool in_grid = rr >= 0 && rr <= zmax;
-      float a = bld(rFv, vc, F(FV0) + o), b = bld(rFv, vc, F(FV0 + NFV / 2) + o);
-      if constexpr (!TOT) {
-        a = a + bld(rFv, vc, F(FV0 + 1) + o);
-        b = b + bld(rFv, vc, F(FV0 + 3) + o);
-      }
+      const float a = bld(rFv, vc, F(VX_X) + o) + bld(rFv, vc, F(VX_Z) + o);
+      const float b = bld(rFv, vc, F(VZ_X) + o) + bld(rFv, vc, F(VZ_Z) + o);
       fvx = in_grid ? a : 0.f;
       fvz = in_grid ? b : 0.f;
       ea = eb = ec = ed = 0.f;
@@ -543,7 +536,7 @@ __device__ __forceinline__ void el_adj_body(const ElDev &d, const float *__restr
     // forward velocity splits, the velocity adjoints and the buoyancies; row k of the stress
     // adjoints, the moduli and the forward stress splits; row k-2 of the velocity adjoints
     struct Row {
-      float fv[NFV], lv[4], b[2], ls[6], cm[ANISO ? 6 : 4], fs[NFS];
+      float fv[4], lv[4], b[2], ls[6], cm[ANISO ? 6 : 4], fs[6];
     };
     // velocity adjoints of rows k-2 .. k+2 as loaded (the row k-2 ones are the old values the
     // velocity stage needs, so they are not loaded a second time)
@@ -552,7 +545,7 @@ __device__ __forceinline__ void el_adj_body(const ElDev &d, const float *__restr
       if (!active) return;
       const unsigned o2 = rb(k + 2), o0 = rb(k);
 #pragma unroll
-      for (int q = 0; q < NFV; ++q) R.fv[q] = bld(rFv, vc, F(FV0 + q) + o2);
+      for (int q = 0; q < 4; ++q) R.fv[q] = bld(rFv, vc, F(VX_X + q) + o2);
 #pragma unroll
       for (int q = 0; q < 4; ++q) R.lv[q] = bld(rLi, vc, F(VX_X + q) + o2);
       R.b[0] = bld(rC, vc, BX * planeb + o2); R.b[1] = bld(rC, vc, BZ * planeb + o2);
@@ -564,7 +557,7 @@ __device__ __forceinline__ void el_adj_body(const ElDev &d, const float *__restr
         R.cm[4] = bld(rC, vc, C15 * planeb + o0); R.cm[5] = bld(rC, vc, C35 * planeb + o0);
       }
 #pragma unroll
-      for (int q = 0; q < NFS; ++q) R.fs[q] = bld(rFs, vc, F(FS0 + q) + o0);
+      for (int q = 0; q < 6; ++q) R.fs[q] = bld(rFs, vc, F(TXX_X + q) + o0);
     };
     Row cur;
     load(z0 - 2, cur);
@@ -615,13 +608,8 @@ __device__ __forceinline__ void el_adj_body(const ElDev &d, const float *__restr
         }
 #pragma unroll
         for (int q = 0; q < 4; ++q) lw[4][q] = cur.lv[q];
-        float fvx = cur.fv[0], fvz = cur.fv[NFV / 2];
-        if constexpr (!TOT) {
-          fvx = fvx + cur.fv[1];
-          fvz = fvz + cur.fv[3];
-        }
-        fvx = in_grid ? fvx : 0.f;
-        fvz = in_grid ? fvz : 0.f;
+        const float fvx = in_grid ? cur.fv[0] + cur.fv[1] : 0.f;
+        const float fvz = in_grid ? cur.fv[2] + cur.fv[3] : 0.f;
         float ea = 0.f, eb = 0.f, ec = 0.f, ed = 0.f;
         if (rr >= 2 && rr <= zw1 && cwin) {
           const float vz_w = d.dt / (d.dz * pzf(1, rr));
@@ -735,12 +723,9 @@ __device__ __forceinline__ void el_adj_body(const ElDev &d, const float *__restr
       // forward stress totals of row k (after the step), free surface once row 3 exists
       {
         const bool in_grid = k >= 0 && k <= zmax;
-        float a = cur.fs[0], b = cur.fs[NFS / 3], e = cur.fs[2 * NFS / 3];
-        if constexpr (!TOT) {
-          a = a + cur.fs[1];
-          b = b + cur.fs[3];
-          e = e + cur.fs[5];
-        }
+        const float a = cur.fs[0] + cur.fs[1];
+        const float b = cur.fs[2] + cur.fs[3];
+        const float e = cur.fs[4] + cur.fs[5];
         xx0 = xx1; xx1 = xx2; xx2 = in_grid ? a : 0.f;
         zz0 = zz1; zz1 = zz2; zz2 = zz3; zz3 = zz4; zz4 = in_grid ? b : 0.f;
         xz0 = xz1; xz1 = xz2; xz2 = xz3; xz3 = xz4; xz4 = in_grid ? e : 0.f;
@@ -811,20 +796,6 @@ __device__ __forceinline__ void el_adj_body(const ElDev &d, const float *__restr
       }
     }
   }
-}
-
-template <bool ANISO, bool INJ>
-__global__ __launch_bounds__(ENT) void el_adj_step(ElDev d, const float *__restrict__ lin, float *__restrict__ lout,
-                                                   const float *__restrict__ fv, const float *__restrict__ fsn, int t,
-                                                   float *__restrict__ gacc, float *__restrict__ gsrc, ElInj inj) {
-  el_adj_body<ANISO, INJ, false>(d, lin, lout, fv, fsn, t, gacc, gsrc, inj);
-}
-
-template <bool INJ>
-__global__ __launch_bounds__(ENT) void el_adj_totals(ElDev d, const float *__restrict__ lin, float *__restrict__ lout,
-                                                     const float *__restrict__ fv, const float *__restrict__ fsn, int t,
-                                                     float *__restrict__ gacc, float *__restrict__ gsrc, ElInj inj) {
-  el_adj_body<false, INJ, true>(d, lin, lout, fv, fsn, t, gacc, gsrc, inj);
 }
 
 // adds the record adjoints of step t to both splits of each recorded field (free-surface tzz
@@ -2319,6 +2290,33 @@ __global__ __launch_bounds__(ENT) void el3_abl_adj(ElDev d, const float *__restr
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
+// The adjoint on tiles (elastic_tile.hpp): tile height and shots per group.  One workgroup runs per
+// CU; a group's shots follow each other in it, and its gradient sums are read and written once per
+// launch.  If 32-row tiles of single shots all run at once, they are done soonest (122 x 240, 1
+// shot, us per step: 32 rows 10.0, 48 rows 12.1).  Else 48 rows (20 x 52 of 32 x 64 points are
+// stored, 36 x 52 of 48 x 64), and the group size of least rounds * (time per round): a round of
+// groups of g shots measured 15 + 18.7 g us (242 x 680, 32 shots, us per step for g = 1, 2, 4, 8,
+// 16: 200, 157, 135, 161, 150; 362 x 1040, 48 shots: 648, 502, 449, 413, 461; 171 x 373, 8 shots,
+// g = 1, 2, 4: 24.1, 19.6, 31.6; 32-row tiles: 28.5, 28.8, 24.6).
+struct ElAdjTile { int rows, spg, groups; };
+ElAdjTile el_adj_tile_shape(const adfwi_elastic_desc *d) {
+  auto tiles = [&](int rows) {
+    const int oz = rows - 12, ox = 52;   // stored rows and columns
+    return (long long)((d->nx - 4 + ox - 1) / ox) * ((d->nz - 4 + oz - 1) / oz);
+  };
+  constexpr long long CUS = 256;
+  const int S = d->nshots;
+  if (tiles(32) * S <= CUS) return {32, 1, S};
+  ElAdjTile best{48, 1, S};
+  double least = 0;
+  for (int g = 1; g <= 16 && g <= S; ++g) {
+    const long long groups = (S + g - 1) / g, rounds = (tiles(48) * groups + CUS - 1) / CUS;
+    const double cost = (double)rounds * (15 + 18.7 * g);
+    if (g == 1 || cost < least) { best = {48, g, (int)groups}; least = cost; }
+  }
+  return best;
+}
+
 int el_layout(const adfwi_elastic_desc *d, adfwi_layout *L) {
   if (!d) { adfwi::set_error("null descriptor"); return ADFWI_E_ARG; }
   if (d->abi_version != ADFWI_ABI_VERSION || d->struct_size != (int32_t)sizeof(adfwi_elastic_desc)) {
@@ -2381,7 +2379,11 @@ int el_layout(const adfwi_elastic_desc *d, adfwi_layout *L) {
                   "grid of %d x %d (pitch %d) exceeds the 2 GiB of one set of gradient planes",
                   d->nz, d->nx, d->pitch);
   L->state_floats = nf * L->field_floats;
-  L->accum_floats = (int64_t)L->ngroups * NCOEF * d->nz * d->pitch;
+  // gradient planes: a set per group of the adjoint that may run (step kernels or tiles)
+  int sets = L->ngroups;
+  if (nn == 2 && !d->damping && !d->aniso && d->shots_per_wave == 0 && d->tile_z == 0)
+    sets = max(sets, el_adj_tile_shape(d).groups);
+  L->accum_floats = (int64_t)sets * NCOEF * d->nz * d->pitch;
   return ADFWI_OK;
 }
 
@@ -2436,6 +2438,21 @@ void launch_el_fwd_tile(const ElDev &v, hipStream_t st, const tile::FwdIO &io) {
   if (count(32) > CUS && count(48) <= CUS) launch_el_fwd_tile_c<4, 12>(v, st, io);
   else if (count(32) > CUS && count(64) <= CUS) launch_el_fwd_tile_c<4, 16>(v, st, io);
   else launch_el_fwd_tile_c<4, 8>(v, st, io);
+}
+
+template <int NR, int NW>
+void launch_el_adj_tile_c(const ElDev &v, hipStream_t st, const tile::AdjIO &io, int groups) {
+  constexpr int oz = tile::out_rows(NR * NW);
+  tile::Grid g;
+  g.ntx = (v.X - 4 + tile::OX - 1) / tile::OX;
+  g.ntz = (v.Z - 4 + oz - 1) / oz;
+  hipLaunchKernelGGL((tile::el_adj_tile<NR, NW>), dim3((unsigned)(g.ntx * g.ntz * groups)), dim3(NW * WAVE), 0, st, v, g, io);
+}
+
+void launch_el_adj_tile(const ElDev &v, hipStream_t st, const tile::AdjIO &io, const ElAdjTile &sh) {
+  static_assert(tile::OX == 52 && tile::out_rows(32) == 32 - 12, "el_adj_tile_shape counts these");
+  if (sh.rows == 32) launch_el_adj_tile_c<4, 8>(v, st, io, sh.groups);
+  else launch_el_adj_tile_c<4, 12>(v, st, io, sh.groups);
 }
 
 }  // namespace
@@ -2573,9 +2590,9 @@ static int elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *
   const bool recs = a->grad_rec[0] || a->grad_rec[1] || a->grad_rec[2] || a->grad_rec[3] || a->grad_rec[4];
   if (recs && d->nrec > 0) ADFWI_CHECK_ARG(d->rcv_z && d->rcv_x, "null receiver table pointer");
   ElDev v = el_dev(d, L);
-  ADFWI_CHECK_ARG(!totals || (!d->damping && v.nn == 2 && !d->aniso),
-                  "a trace of totals belongs to the 4th-order PML scheme without C15 / C35");
-  const long long slot = totals ? NFIELD5 * L.field_floats : L.state_floats;
+  ADFWI_CHECK_ARG(!totals || el_tile_ok(d, v, L, recs && d->nrec > 0),
+                  "a trace of totals needs the tile kernels (4th-order PML without C15 / C35, library tiling, a "
+                  "receiver map for record adjoints, state sets under 2 GiB)");
   // the free-surface transposes need rows 0..3 inside the first strip (every strip height here
   // is at least 8)
   // (damping scheme: strips of ETZA rows, so that no strip but the first reaches the
@@ -2616,6 +2633,32 @@ static int elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *
     for (int q = 0; q < 5; ++q) ij.g[q] = a->grad_rec[q];
   }
   float *cur = a->lam_in;
+  if (totals) {
+    const ElAdjTile sh = el_adj_tile_shape(d);
+    const long long slot = NFIELD5 * L.field_floats;
+    for (int i = a->nsteps - 1; i >= 0;) {   // two steps per launch, the last launch the odd one
+      tile::AdjIO io;
+      io.t = t_lo + i;
+      io.n = min(tile::TK, i + 1);
+      for (int j = 0; j < tile::TK; ++j) {
+        const int q = max(i - j, 0);
+        io.fv[j] = q == 0 ? a->fwd0 : a->trace + (long long)(q - 1) * slot;
+        io.fs[j] = a->trace + (long long)q * slot;
+      }
+      io.lin = cur;
+      io.lout = (cur == a->work[0]) ? a->work[1] : a->work[0];
+      io.spg = sh.spg;
+      io.gacc = a->grad_coef;
+      io.gsrc = a->grad_src;
+      io.inj = ij;
+      launch_el_adj_tile(v, st, io, sh);
+      if ((rc = adfwi::check_launch("el_adj_tile"))) return rc;
+      cur = io.lout;
+      i -= io.n;
+    }
+    a->lam_out = cur;
+    return ADFWI_OK;
+  }
   for (int i = a->nsteps - 1; i >= 0; --i) {
     const int t = t_lo + i;
     if (recs && ng > 0 && !fused) {
@@ -2627,8 +2670,8 @@ static int elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *
                            a->grad_rec[2], a->grad_rec[3], a->grad_rec[4], t);
       if ((rc = adfwi::check_launch("el_inject"))) return rc;
     }
-    const float *fv = i == 0 ? a->fwd0 : a->trace + (long long)(i - 1) * slot;
-    const float *fsn = a->trace + (long long)i * slot;
+    const float *fv = i == 0 ? a->fwd0 : a->trace + (long long)(i - 1) * L.state_floats;
+    const float *fsn = a->trace + (long long)i * L.state_floats;
     float *nxt = (cur == a->work[0]) ? a->work[1] : a->work[0];
     if (d->damping && v.nn > 2) {
       if (d->aniso)
@@ -2650,11 +2693,7 @@ static int elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *
       if ((rc = adfwi::check_launch("el3_adj_step"))) return rc;
     } else {
       float *gc = a->grad_coef, *gs = a->grad_src;
-      if (totals && fused)
-        hipLaunchKernelGGL(el_adj_totals<true>, grid, block, 0, st, v, cur, nxt, fv, fsn, t, gc, gs, ij);
-      else if (totals)
-        hipLaunchKernelGGL(el_adj_totals<false>, grid, block, 0, st, v, cur, nxt, fv, fsn, t, gc, gs, ij);
-      else if (d->aniso && fused)
+      if (d->aniso && fused)
         hipLaunchKernelGGL((el_adj_step<true, true>), grid, block, 0, st, v, cur, nxt, fv, fsn, t, gc, gs, ij);
       else if (d->aniso)
         hipLaunchKernelGGL((el_adj_step<true, false>), grid, block, 0, st, v, cur, nxt, fv, fsn, t, gc, gs, ij);
@@ -2662,7 +2701,7 @@ static int elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *
         hipLaunchKernelGGL((el_adj_step<false, true>), grid, block, 0, st, v, cur, nxt, fv, fsn, t, gc, gs, ij);
       else
         hipLaunchKernelGGL((el_adj_step<false, false>), grid, block, 0, st, v, cur, nxt, fv, fsn, t, gc, gs, ij);
-      if ((rc = adfwi::check_launch(totals ? "el_adj_totals" : "el_adj_step"))) return rc;
+      if ((rc = adfwi::check_launch("el_adj_step"))) return rc;
     }
     cur = nxt;
   }

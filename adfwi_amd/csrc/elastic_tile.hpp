@@ -287,4 +287,319 @@ __global__ __launch_bounds__(NW *WAVE) void el_fwd_tile(ElDev d, Grid g, FwdIO i
   }
 }
 
+struct AdjIO {
+  const float *lin;
+  float *lout;
+  int t, n;              // latest step and number of steps (1 .. TK), going down
+  int spg;               // shots per group
+  const float *fv[TK];   // totals [5][S][Z][pitch] before each step (velocities) ...
+  const float *fs[TK];   // ... and after it (stresses)
+  float *gacc, *gsrc;    // [groups][NCOEF][Z][pitch] gradient sums; [S][nt] or NULL
+  ElInj inj;             // inj.map NULL: no record adjoints
+};
+
+// forms the values where this stands: left to itself the compiler moves a sum whose only use lies
+// past a later branch there, and holds its terms till then (50 registers in the kernel below)
+__device__ __forceinline__ void pin(float &a, float &b) { asm volatile("" : "+v"(a), "+v"(b)); }
+__device__ __forceinline__ float keep(int m, float v) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(int, v) & m);
+}
+__device__ __forceinline__ float pick(int m, float a, float b) {   // bits of a where m is set, else of b
+  return __builtin_bit_cast(float, (__builtin_bit_cast(int, a) & m) | (__builtin_bit_cast(int, b) & ~m));
+}
+
+// The adjoint (el_adj_step lists the transposes) over the same tiles.  A workgroup takes the shots
+// of a group one after the other and keeps their gradient sums of its points in registers: one
+// read and write of the gradient planes per launch.  Per point and step that is 40 B of splits, 20 B
+// of totals and 24 / shots B of gradients, against 80 + 20 + 12 for a step at a time; the halo's
+// re-reads come from the L2.  A tile's loads, its arithmetic (about 200 VALU operations a row and
+// step, 24 of them wavefront shifts) and its stores follow each other with one workgroup per CU; at
+// 48 rows the traffic alone is two thirds of the time.  All of it has to stay within 168 registers,
+// three wavefronts per SIMD: with 224 (two) 150 us per step against 135 on 242 x 680 with 32 shots,
+// and el_adj_step took 251; 362 x 1040, 48 shots: 474, 409, 779.  Adjoint splits outside the window, which
+// el_adj_step keeps at zero, take values here, but nothing reads them: the coefficients there are
+// zero, and they are not stored.
+template <int NR, int NW>
+__global__ __launch_bounds__(NW *WAVE, NW / 4) void el_adj_tile(ElDev d, Grid g, AdjIO io) {
+  static_assert(NR == 4 && H == 6, "rows 0 .. 3, which the free surface ties together, are wavefront 1 of the first tiles");
+  constexpr int OZ = out_rows(NR * NW);
+  __shared__ float sv[NW + 2][18][WAVE], ss[NW + 2][6][WAVE];
+  int tx, tzi, grp;
+  place(g, tx, tzi, grp);
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+  if (wv == 0) {
+#pragma unroll
+    for (int q = 0; q < 18; ++q) sv[0][q][lane] = sv[NW + 1][q][lane] = 0.f;
+#pragma unroll
+    for (int q = 0; q < 6; ++q) ss[0][q][lane] = ss[NW + 1][q][lane] = 0.f;
+  }
+  const int x0 = 2 + tx * OX, z0 = 2 + tzi * OZ;
+  const int c = x0 - H + lane, zt = z0 - H + wv * NR;
+  const int zw1 = d.Z - 3;
+  const unsigned rowb = 4u * (unsigned)d.pitch, planeb = 4u * (unsigned)d.plane, fieldb = 4u * (unsigned)d.field;
+  const bool own = c >= x0 && c < min(x0 + OX, d.X - 2);
+  const bool cwin = c >= 2 && c <= d.X - 3;
+  auto bits = [&](int lo, int hi) -> unsigned {   // rows lo .. hi-1 of this wavefront
+    const int a = min(max(lo - zt, 0), NR), b = min(max(hi - zt, 0), NR);
+    return b > a ? ((1u << b) - 1u) & ~((1u << a) - 1u) : 0u;
+  };
+  const unsigned ownbits = bits(z0, min(z0 + OZ, zw1 + 1));
+  // byte offset of this lane's point of row r in a plane (outside the grid: none, loads return 0),
+  // and the same where the workgroup stores the point
+  unsigned vi[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r)
+    vi[r] = c >= 0 && c < d.X && zt + r >= 0 && zt + r < d.Z ? (unsigned)(zt + r) * rowb + 4u * (unsigned)c : DROP;
+  auto vo = [&](int r) -> unsigned { return own && ((ownbits >> r) & 1u) ? vi[r] : DROP; };
+  const float c0 = d.c0, c1 = d.c1;
+  float C[4][NR], bx[NR], bz[NR];
+  {
+    const rsrc_t rC = rsrc(d.coef, (unsigned)NCOEF * planeb);
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const unsigned v = cwin && zt + r >= 2 && zt + r <= zw1 ? vi[r] : DROP;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) C[q][r] = bld(rC, v, (unsigned)q * planeb);
+      bx[r] = bld(rC, v, BX * planeb);
+      bz[r] = bld(rC, v, BZ * planeb);
+    }
+  }
+  // absorbing-boundary factors: per column, and per row in scalar registers
+  const int cc = min(max(c, 0), d.X - 1);
+  const float pxn = d.pml_x[cc], pxd = d.pml_x[d.pitch + cc], pxi = d.pml_x[2 * d.pitch + cc];
+  const float sx_keep = pxn * pxi, sx_a = d.dt_dx * pxi, vx_keep = pxn / pxd, vx_w = d.dt / (d.dx * pxd);
+  auto uni = [](float v) -> float {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+  };
+  float sz_keep[NR], sz_a[NR], vz_keep[NR], vz_w[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const int row = min(max(zt + r, 0), d.Z - 1);
+    const float pzn = scalar_ld(d.pml_z + row), pzd = scalar_ld(d.pml_z + d.Z + row), pzi = scalar_ld(d.pml_z + 2 * d.Z + row);
+    sz_keep[r] = uni(pzn * pzi); sz_a[r] = uni(d.dt_dz * pzi);
+    vz_keep[r] = uni(pzn / pzd); vz_w[r] = uni(d.dt / (d.dz * pzd));
+  }
+  // masks: the free surface's wavefront (rows 0 .. 3), window columns c, c + 1 and c - 1
+  int mfs = __builtin_amdgcn_readfirstlane(d.fsurf && tzi == 0 && wv == 1 ? -1 : 0);
+  asm volatile("" : "+s"(mfs));
+  auto in_win = [&](int x) -> int { int m = x >= 2 && x <= d.X - 3 ? -1 : 0; asm volatile("" : "+v"(m)); return m; };
+  const int mcw = in_win(c), mj1 = in_win(c + 1), mm1 = in_win(c - 1), mfc = mfs & mcw;
+  unsigned rbits = 0;   // rows with receivers: of the halo, too
+  if (io.inj.map) {
+    const bool mine = lane < NR && zt + lane >= 2 && zt + lane <= zw1;
+    rbits = (unsigned)__ballot(mine && io.inj.map[mine ? zt + lane : 0] > 0);
+  }
+  float G[6][NR];
+#pragma unroll
+  for (int q = 0; q < 6; ++q)
+#pragma unroll
+    for (int r = 0; r < NR; ++r) G[q][r] = 0.f;
+
+  const int s_end = min((grp + 1) * io.spg, d.S);
+#pragma unroll 1
+  for (int s = grp * io.spg; s < s_end; ++s) {
+    const int zs = scalar_ld(d.src_z + s), xs = scalar_ld(d.src_x + s);
+    const bool src_here = io.gsrc && zs >= zt && zs < zt + NR && ((ownbits >> (zs - zt)) & 1u) && xs >= x0 && xs < x0 + OX;
+    float f[NFIELD][NR];
+    {
+      const rsrc_t rIn = rsrc(io.lin + (long long)s * d.plane, (NFIELD - 1) * fieldb + planeb);
+#pragma unroll
+      for (int r = 0; r < NR; ++r)
+#pragma unroll
+        for (int q = 0; q < NFIELD; ++q) f[q][r] = bld(rIn, vi[r], (unsigned)q * fieldb);
+    }
+#pragma unroll 1
+    for (int i = 0; i < io.n; ++i) {
+      const int t = io.t - i;
+      float vx[NR], vz[NR], xx[NR], zz[NR], xz[NR];
+      {
+        const rsrc_t rV = rsrc(io.fv[i] + (long long)s * d.plane, (NFIELD5 - 1) * fieldb + planeb);
+        const rsrc_t rS = rsrc(io.fs[i] + (long long)s * d.plane, (NFIELD5 - 1) * fieldb + planeb);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          vx[r] = bld(rV, vi[r], VX * fieldb);
+          vz[r] = bld(rV, vi[r], VZ * fieldb);
+        }
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          xx[r] = bld(rS, vi[r], TXX * fieldb);
+          zz[r] = bld(rS, vi[r], TZZ * fieldb);
+          xz[r] = bld(rS, vi[r], TXZ * fieldb);
+        }
+      }
+      if (rbits) {   // record adjoints of step t, to both splits
+        const long long ro = ((long long)s * d.nt + t) * d.nrec;
+        auto adj = [&](int q, unsigned v) -> float {
+          const float *p = io.inj.g[q];
+          return bld(rsrc(p ? p + ro : nullptr, p ? 4u * (unsigned)d.nrec : 0u), v, 0u);
+        };
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          if ((rbits >> r) & 1u) {
+            const int m = __builtin_bit_cast(int, bld(rsrc(io.inj.map + d.Z, planeb), vi[r], 0u));
+            const unsigned v = cwin && m >= 0 ? 4u * (unsigned)m : DROP;
+            const float axx = adj(TXX, v), azz = adj(TZZ, d.fsurf && zt + r == 2 ? DROP : v), axz = adj(TXZ, v);
+            const float avx = adj(VX, v), avz = adj(VZ, v);
+            f[TXX_X][r] += axx; f[TXX_Z][r] += axx; f[TZZ_X][r] += azz; f[TZZ_Z][r] += azz;
+            f[TXZ_X][r] += axz; f[TXZ_Z][r] += axz; f[VX_X][r] += avx; f[VX_Z][r] += avx;
+            f[VZ_X][r] += avz; f[VZ_Z][r] += avz;
+          }
+      }
+      float eb[NR], ed[NR];
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        asm volatile("" : "+v"(bx[r]), "+v"(bz[r]));   // (the products below, kept over the loops, would cost 8 registers)
+        eb[r] = f[VX_Z][r] * (vz_w[r] * bx[r]);
+        ed[r] = f[VZ_Z][r] * (vz_w[r] * bz[r]);
+      }
+      // forward free surface: velocity rows 0 and 1 from rows 2 and 3, stress rows 0 .. 2.  Bit
+      // masks, not branches, here and below: the sides of a branch (or of a select, which becomes
+      // one) share terms with what follows, and holding those cost 90 registers
+      {
+        const float vz2n = from_right(vz[2]);
+        const float vz1m_n = keep(mj1, vz2n);
+        const float vz1m = pick(mcw, vz[2], vz[1]);
+        const float nx1 = (((vz1m_n - vz1m) + vz2n) - vz[2]) + vx[3];
+        vx[1] = pick(mfc, nx1, vx[1]);
+        vz[0] = pick(mfc, vz1m, vz[0]);
+        vz[1] = pick(mfs, vz1m, vz[1]);
+        zz[1] = pick(mfs, -zz[3], zz[1]); zz[2] = keep(~mfs, zz[2]);
+        xz[1] = pick(mfs, -xz[2], xz[1]); xz[0] = pick(mfs, -xz[3], xz[0]);
+      }
+      sv[wv + 1][0][lane] = eb[0]; sv[wv + 1][1][lane] = eb[1]; sv[wv + 1][2][lane] = eb[NR - 1];
+      sv[wv + 1][3][lane] = ed[0]; sv[wv + 1][4][lane] = ed[NR - 2]; sv[wv + 1][5][lane] = ed[NR - 1];
+      sv[wv + 1][6][lane] = vx[0]; sv[wv + 1][7][lane] = vx[1]; sv[wv + 1][8][lane] = vx[NR - 1];
+      sv[wv + 1][9][lane] = vz[0]; sv[wv + 1][10][lane] = vz[NR - 2]; sv[wv + 1][11][lane] = vz[NR - 1];
+      sv[wv + 1][12][lane] = zz[0]; sv[wv + 1][13][lane] = zz[1]; sv[wv + 1][14][lane] = zz[NR - 1];
+      sv[wv + 1][15][lane] = xz[0]; sv[wv + 1][16][lane] = xz[NR - 2]; sv[wv + 1][17][lane] = xz[NR - 1];
+      lds_barrier();
+      {   // buoyancy gradients: velocity adjoints as they are now, forward stress derivatives
+        const float za = sv[wv][14][lane], zb1 = sv[wv + 2][12][lane], zb2 = sv[wv + 2][13][lane];
+        const float xa2 = sv[wv][16][lane], xa1 = sv[wv][17][lane], xb = sv[wv + 2][15][lane];
+        auto ZZr = [&](int r) { return r < 0 ? za : r == NR ? zb1 : r > NR ? zb2 : zz[r]; };
+        auto XZr = [&](int r) { return r == -2 ? xa2 : r == -1 ? xa1 : r >= NR ? xb : xz[r]; };
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          __builtin_amdgcn_sched_barrier(0);
+          const float tl1 = from_left(xx[r]), tr1 = from_right(xx[r]), tr2 = from_right(tr1);
+          const float ul1 = from_left(xz[r]), ul2 = from_left(ul1), ur1 = from_right(xz[r]);
+          const float dxf_txx = c0 * (tr1 - xx[r]) + c1 * (tr2 - tl1);
+          const float dzb_txz = c0 * (xz[r] - XZr(r - 1)) + c1 * (XZr(r + 1) - XZr(r - 2));
+          const float dxb_txz = c0 * (xz[r] - ul1) + c1 * (ur1 - ul2);
+          const float dzf_tzz = c0 * (ZZr(r + 1) - zz[r]) + c1 * (ZZr(r + 2) - ZZr(r - 1));
+          G[4][r] += f[VX_X][r] * (vx_w * dxf_txx) + f[VX_Z][r] * (vz_w[r] * dzb_txz);
+          G[5][r] += f[VZ_X][r] * (vx_w * dxb_txz) + f[VZ_Z][r] * (vz_w[r] * dzf_tzz);
+          pin(G[4][r], G[5][r]);
+        }
+      }
+      float P1[NR], Q2[NR], Q3[NR], P4[NR];
+      {
+        const float eba = sv[wv][2][lane], ebb1 = sv[wv + 2][0][lane], ebb2 = sv[wv + 2][1][lane];
+        const float eda2 = sv[wv][4][lane], eda1 = sv[wv][5][lane], edb = sv[wv + 2][3][lane];
+        const float xa = sv[wv][8][lane], xb1 = sv[wv + 2][6][lane], xb2 = sv[wv + 2][7][lane];
+        const float za2 = sv[wv][10][lane], za1 = sv[wv][11][lane], zb = sv[wv + 2][9][lane];
+        auto EB = [&](int r) { return r < 0 ? eba : r == NR ? ebb1 : r > NR ? ebb2 : eb[r]; };
+        auto ED = [&](int r) { return r == -2 ? eda2 : r == -1 ? eda1 : r >= NR ? edb : ed[r]; };
+        auto VXr = [&](int r) { return r < 0 ? xa : r == NR ? xb1 : r > NR ? xb2 : vx[r]; };
+        auto VZr = [&](int r) { return r == -2 ? za2 : r == -1 ? za1 : r >= NR ? zb : vz[r]; };
+        float ltxz0 = 0.f, ltxz1 = 0.f, ltzz1 = 0.f;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          __builtin_amdgcn_sched_barrier(0);
+          const float ea = f[VX_X][r] * (vx_w * bx[r]), ec = f[VZ_X][r] * (vx_w * bz[r]);
+          const float e1m1 = from_left(ea), e1m2 = from_left(e1m1), e1p1 = from_right(ea);
+          const float e3p1 = from_right(ec), e3m1 = from_left(ec), e3p2 = from_right(e3p1);
+          const float lt_xx = c0 * (e1m1 - ea) + c1 * (e1m2 - e1p1);
+          float lt_xz = (c0 * (eb[r] - EB(r + 1)) + c1 * (EB(r - 1) - EB(r + 2))) + (c0 * (ec - e3p1) + c1 * (e3m1 - e3p2));
+          float lt_zz = c0 * (ED(r - 1) - ed[r]) + c1 * (ED(r - 2) - ED(r + 1));
+          // stress free surface transposed
+          if (r == 0) ltxz0 = keep(mfs, lt_xz);
+          if (r == 1) { ltzz1 = keep(mfs, lt_zz); ltxz1 = keep(mfs, lt_xz); }
+          if (r == 2) { lt_zz = keep(~mfs, lt_zz); lt_xz = lt_xz - ltxz1; }
+          if (r == 3) { lt_zz = lt_zz - ltzz1; lt_xz = lt_xz - ltxz0; }
+          f[TXX_X][r] += lt_xx; f[TXX_Z][r] += lt_xx;
+          f[TZZ_X][r] += lt_zz; f[TZZ_Z][r] += lt_zz;
+          f[TXZ_X][r] += lt_xz; f[TXZ_Z][r] += lt_xz;
+          const float lxx_x = f[TXX_X][r], lxx_z = f[TXX_Z][r];
+          const float lzz_x = f[TZZ_X][r], lzz_z = f[TZZ_Z][r];
+          const float lxz_x = f[TXZ_X][r], lxz_z = f[TXZ_Z][r];
+          const float axx_x = sx_a * lxx_x, axx_z = sz_a[r] * lxx_z;
+          const float azz_x = sx_a * lzz_x, azz_z = sz_a[r] * lzz_z;
+          const float axz_x = sx_a * lxz_x, axz_z = sz_a[r] * lxz_z;
+          P1[r] = C[0][r] * axx_x + C[1][r] * azz_x;
+          Q2[r] = C[1][r] * axx_z + C[2][r] * azz_z;
+          Q3[r] = C[3][r] * axz_x;
+          P4[r] = C[3][r] * axz_z;
+          const float xl1 = from_left(vx[r]), xl2 = from_left(xl1), xr1 = from_right(vx[r]);
+          const float zl1 = from_left(vz[r]), zr1 = from_right(vz[r]), zr2 = from_right(zr1);
+          const float dxb_vx = c0 * (vx[r] - xl1) + c1 * (xr1 - xl2);
+          const float dzb_vz = c0 * (vz[r] - VZr(r - 1)) + c1 * (VZr(r + 1) - VZr(r - 2));
+          const float dxf_vz = c0 * (zr1 - vz[r]) + c1 * (zr2 - zl1);
+          const float dzf_vx = c0 * (VXr(r + 1) - vx[r]) + c1 * (VXr(r + 2) - VXr(r - 1));
+          G[0][r] += axx_x * dxb_vx;
+          G[1][r] += axx_z * dzb_vz + azz_x * dxb_vx;
+          G[2][r] += azz_z * dzb_vz;
+          G[3][r] += axz_x * dxf_vz + axz_z * dzf_vx;
+          pin(G[0][r], G[1][r]); pin(G[2][r], G[3][r]);
+          pin(P1[r], Q2[r]); pin(Q3[r], P4[r]);
+        }
+      }
+      ss[wv + 1][0][lane] = Q2[0]; ss[wv + 1][1][lane] = Q2[1]; ss[wv + 1][2][lane] = Q2[NR - 1];
+      ss[wv + 1][3][lane] = P4[0]; ss[wv + 1][4][lane] = P4[NR - 2]; ss[wv + 1][5][lane] = P4[NR - 1];
+      if (src_here) {
+        const float mxx = d.src_m[3 * s], mzz = d.src_m[3 * s + 1], mxz = d.src_m[3 * s + 2];
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          if (zs == zt + r && c == xs) {
+            float gm = (mxx * (f[TXX_X][r] + f[TXX_Z][r]) + mzz * (f[TZZ_X][r] + f[TZZ_Z][r])) +
+                       mxz * (f[TXZ_X][r] + f[TXZ_Z][r]);
+            if (d.src_fz) gm = gm + 0.5f * (d.src_fz[s] * (f[VZ_X][r] + f[VZ_Z][r]));
+            io.gsrc[(long long)s * d.nt + t] = gm;
+          }
+      }
+      lds_barrier();
+      {
+        const float qa = ss[wv][2][lane], qb1 = ss[wv + 2][0][lane], qb2 = ss[wv + 2][1][lane];
+        const float pa2 = ss[wv][4][lane], pa1 = ss[wv][5][lane], pb = ss[wv + 2][3][lane];
+        auto Q2r = [&](int r) { return r < 0 ? qa : r == NR ? qb1 : r > NR ? qb2 : Q2[r]; };
+        auto P4r = [&](int r) { return r == -2 ? pa2 : r == -1 ? pa1 : r >= NR ? pb : P4[r]; };
+        float lvz0 = 0.f, lvz1 = 0.f, lvx1 = 0.f;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          __builtin_amdgcn_sched_barrier(0);
+          const float p1p1 = from_right(P1[r]), p1p2 = from_right(p1p1), p1m1 = from_left(P1[r]);
+          const float q3m1 = from_left(Q3[r]), q3m2 = from_left(q3m1), q3p1 = from_right(Q3[r]);
+          float lvx = (c0 * (P1[r] - p1p1) + c1 * (p1m1 - p1p2)) + (c0 * (P4r(r - 1) - P4[r]) + c1 * (P4r(r - 2) - P4r(r + 1)));
+          float lvz = (c0 * (Q2[r] - Q2r(r + 1)) + c1 * (Q2r(r - 1) - Q2r(r + 2))) + (c0 * (q3m1 - Q3[r]) + c1 * (q3m2 - q3p1));
+          if (r == 0) lvz0 = lvz;
+          if (r == 1) { lvz1 = lvz; lvx1 = lvx; }
+          if (r == 2) lvz = lvz + keep(mfs, ((lvz1 + lvz0) - 2.0f * lvx1) + keep(mm1, 2.0f * from_left(lvx1)));
+          if (r == 3) lvx = lvx + keep(mfs, lvx1);
+          const float l1 = f[VX_X][r], l2 = f[VX_Z][r], l3 = f[VZ_X][r], l4 = f[VZ_Z][r];
+          f[TXX_X][r] = sx_keep * f[TXX_X][r]; f[TXX_Z][r] = sz_keep[r] * f[TXX_Z][r];
+          f[TZZ_X][r] = sx_keep * f[TZZ_X][r]; f[TZZ_Z][r] = sz_keep[r] * f[TZZ_Z][r];
+          f[TXZ_X][r] = sx_keep * f[TXZ_X][r]; f[TXZ_Z][r] = sz_keep[r] * f[TXZ_Z][r];
+          f[VX_X][r] = vx_keep * l1 + lvx; f[VX_Z][r] = vz_keep[r] * l2 + lvx;
+          f[VZ_X][r] = vx_keep * l3 + lvz; f[VZ_Z][r] = vz_keep[r] * l4 + lvz;
+        }
+      }
+    }
+    const rsrc_t rOut = rsrc(io.lout + (long long)s * d.plane, (NFIELD - 1) * fieldb + planeb);
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const unsigned v = vo(r);
+#pragma unroll
+      for (int q = 0; q < NFIELD; ++q) bst(f[q][r], rOut, v, (unsigned)q * fieldb);
+    }
+  }
+  const rsrc_t rG = rsrc(io.gacc + (long long)grp * NCOEF * d.Z * d.pitch, (unsigned)NCOEF * planeb);
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const unsigned v = vo(r);
+#pragma unroll
+    for (int q = 0; q < 6; ++q) bst(bld(rG, v, (unsigned)q * planeb) + G[q][r], rG, v, (unsigned)q * planeb);
+  }
+}
+
 }  // namespace tile

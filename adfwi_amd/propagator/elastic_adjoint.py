@@ -94,8 +94,9 @@ def run_backward(geom, coef: torch.Tensor, src: torch.Tensor, pml_x: Optional[to
             aa.grad_rec[i] = None if g[i] is None else g[i].data_ptr()
         aa.grad_coef = gacc.data_ptr()
         aa.grad_src = gsrc.data_ptr()
-        TIMELINE.call("adjoint", "el_adj_totals" if totals else geom.kernel_names[1], n, dev, lambda: nat.check(
-            adjoint(ctypes.byref(d), ctypes.byref(aa), stream), "adfwi_elastic_adjoint"))
+        TIMELINE.call("adjoint", "el_adj_tile" if totals else geom.kernel_names[1],
+                      tile_launches(0, n, 0, TILE_STEPS) if totals else n, dev, lambda: nat.check(
+            adjoint(ctypes.byref(d), ctypes.byref(aa), stream), "adfwi_elastic_adjoint"), steps=n)
         cur = lam[0] if aa.lam_out == lam[0].data_ptr() else lam[1]
         traces.pop(seg, None)              # done; segment seg + 1, which read its last state, too
         seg_trace = fwd0 = None

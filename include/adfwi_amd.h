@@ -224,7 +224,8 @@ typedef struct adfwi_elastic_desc {
 /* Tiling and buffer sizes; layout.nfields = 10 (PML split fields) or 5 (damping), layout.reserved = shots per
  * wavefront, layout.shots_per_block = shots per workgroup, layout.ngroups = workgroups along
  * the shots, layout.accum_floats = size of the gradient accumulator of the adjoint,
- * [ngroups][8][nz][pitch] (one set of planes per workgroup's shots). */
+ * [sets][8][nz][pitch] (one set of planes per workgroup's shots; layout.accum_floats gives the
+ * sets, at least ngroups), their sum over the sets. */
 int adfwi_elastic_get_layout(const adfwi_elastic_desc *d, adfwi_layout *out);
 
 typedef struct adfwi_elastic_fwd_args {
@@ -271,8 +272,9 @@ int adfwi_elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a
 
 /* The same from a trace of totals (adfwi_elastic_fwd_args.trace_totals): a->trace holds
  * [nsteps][5][S][Z][pitch] and a->fwd0 the totals before step t_hi-nsteps, [5][S][Z][pitch] (vx and
- * vz are read).  Half the bytes of the forward wavefield; the gradients are the same bit for bit.
- * 4th-order PML scheme with aniso 0. */
+ * vz are read).  Half the bytes of the forward wavefield, and two steps per launch; the gradients
+ * are the same to rounding (their terms are added in another order), the adjoint states and the
+ * wavelet gradient bit for bit.  For what adfwi_elastic_fwd_args.trace_totals takes. */
 int adfwi_elastic_adjoint_totals(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a, adfwi_stream_t stream);
 
 /* ------------------------------------------------------------------------ */

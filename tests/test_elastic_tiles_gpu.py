@@ -1,11 +1,16 @@
 """The elastic tile kernels (up to two steps per launch on register tiles, a trace of five totals)
 against the one-step kernels (explicit tiling, a trace of the ten splits): records, checkpoints,
-final states and gradients are all formed by the same operations in the same order, so they are
-equal bit for bit.
+final states and the wavelet gradient are formed by the same operations in the same order, so they
+are equal bit for bit; the terms of the coefficient gradients are added in another order.
 
 The grids pick every tile height (32, 48 and 64 rows, which store 20, 36 and 52) and end at, one
 short of and one past a tile's edge each way (52 columns, from column 2); one grid is the smallest
-the library takes; steps and checkpoint cuts leave launches of one and of two steps.
+the library takes; steps and checkpoint cuts leave launches of one and of two steps.  The adjoint takes 32 rows and
+single shots in the first five, 48 rows and groups of 1, 2 and more shots, the last of them smaller,
+in the others.
+
+Tolerance of the reordered sums: N = shots * steps terms per point, at most 80 * 13 = 1040, each
+addition rounding to 2^-24: sqrt(N) * 2^-24 = 1.9e-6; 5e-6 leaves room for cancellation.
 """
 import numpy as np
 import pytest
@@ -69,5 +74,6 @@ def test_tiles_equal_one_step_kernels(Z, X, S, fs, force):
     torch.cuda.synchronize()
     for i in range(6):
         assert grads[1][0][i].abs().max() > 0
-        assert torch.equal(grads[0][0][i], grads[1][0][i]), ("gradient", i)
+        err = rel_l2(grads[0][0][i].cpu().numpy(), grads[1][0][i].cpu().numpy())
+        assert err <= 5e-6, ("gradient", i, err)
     assert torch.equal(grads[0][1], grads[1][1])
