@@ -2292,7 +2292,8 @@ __global__ __launch_bounds__(ENT) void el3_abl_adj(ElDev d, const float *__restr
 // ---------------------------------------------------------------------------
 // The adjoint on tiles (elastic_tile.hpp): tile height and shots per group.  One workgroup runs per
 // CU; a group's shots follow each other in it, and its gradient sums are read and written once per
-// launch.  If 32-row tiles of single shots all run at once, they are done soonest (122 x 240, 1
+// launch.  (Three-term differences, a step per launch: the same rule; 214 x 393, 8 shots: 48 rows,
+// g = 1, 2, 4: 47, 37, 55.)  If 32-row tiles of single shots all run at once, they are done soonest (122 x 240, 1
 // shot, us per step: 32 rows 10.0, 48 rows 12.1).  Else 48 rows (20 x 52 of 32 x 64 points are
 // stored, 36 x 52 of 48 x 64), and the group size of least rounds * (time per round): a round of
 // groups of g shots measured 15 + 18.7 g us (242 x 680, 32 shots, us per step for g = 1, 2, 4, 8,
@@ -2300,9 +2301,10 @@ __global__ __launch_bounds__(ENT) void el3_abl_adj(ElDev d, const float *__restr
 // g = 1, 2, 4: 24.1, 19.6, 31.6; 32-row tiles: 28.5, 28.8, 24.6).
 struct ElAdjTile { int rows, spg, groups; };
 ElAdjTile el_adj_tile_shape(const adfwi_elastic_desc *d) {
+  const int nn = d->nn == 0 ? 2 : d->nn;
   auto tiles = [&](int rows) {
     const int oz = rows - 12, ox = 52;   // stored rows and columns
-    return (long long)((d->nx - 4 + ox - 1) / ox) * ((d->nz - 4 + oz - 1) / oz);
+    return (long long)((d->nx - 2 * nn + ox - 1) / ox) * ((d->nz - 2 * nn + oz - 1) / oz);
   };
   constexpr long long CUS = 256;
   const int S = d->nshots;
@@ -2381,7 +2383,7 @@ int el_layout(const adfwi_elastic_desc *d, adfwi_layout *L) {
   L->state_floats = nf * L->field_floats;
   // gradient planes: a set per group of the adjoint that may run (step kernels or tiles)
   int sets = L->ngroups;
-  if (nn == 2 && !d->damping && !d->aniso && d->shots_per_wave == 0 && d->tile_z == 0)
+  if (!d->damping && !d->aniso && d->shots_per_wave == 0 && d->tile_z == 0)
     sets = max(sets, el_adj_tile_shape(d).groups);
   L->accum_floats = (int64_t)sets * NCOEF * d->nz * d->pitch;
   return ADFWI_OK;
@@ -2404,55 +2406,67 @@ ElDev el_dev(const adfwi_elastic_desc *d, const adfwi_layout &L) {
   return v;
 }
 
-// ---- tiles (elastic_tile.hpp): up to two steps per launch of the 4th-order PML scheme without
-// C15 / C35, where the caller left the layout to the library, records (if any) go through the
-// receiver map, and a state set stays under the 2 GiB that dropped buffer accesses need
+// ---- tiles (elastic_tile.hpp): the PML scheme without C15 / C35, where the caller left the layout
+// to the library, records (if any) go through the receiver map, and a state set stays under the
+// 2 GiB that dropped buffer accesses need.  Two steps per launch at 4th order.  With three-term
+// differences it is one, the halo's price is not halved, and what the tiles gain is that no lane
+// marches down a strip: up to three rounds of 64-row tiles.  Measured, us per step, step kernels ->
+// tiles, forward with records / with a trace / adjoint: 163 x 341, 3 shots 20 -> 10 / 19 -> 11 / 36 ->
+// 17; 214 x 393, 8 shots (256 tiles) 25 -> 18 / 29 -> 20 / 46 -> 37; 24 shots (768) 49 -> 50 / 63 -> 55 /
+// 111 -> 78; 32 shots 59 -> 66 / 78 -> 81 / 150 -> 113; 243 x 680, 32 shots 151 -> 158 / 152 -> 191 /
+// 268 -> 224.
+constexpr long long EL3_TILES = 768;
 bool el_tile_ok(const adfwi_elastic_desc *d, const ElDev &v, const adfwi_layout &L, bool recs) {
-  return !d->damping && v.nn == 2 && !d->aniso && d->shots_per_wave == 0 && d->tile_z == 0 &&
+  const long long tiles64 = (long long)((v.X - 2 * v.nn + 51) / 52) * ((v.Z - 2 * v.nn + 51) / 52) * v.S;
+  return !d->damping && !d->aniso && d->shots_per_wave == 0 && d->tile_z == 0 && (v.nn == 2 || tiles64 <= EL3_TILES) &&
          (!recs || d->rcv_map) && L.state_floats * 4 < ((int64_t)1 << 31) &&
          (int64_t)NCOEF * d->nz * d->pitch * 4 < ((int64_t)1 << 31);
 }
 
-template <int NR, int NW>
+template <int NW>
+tile::Grid el_tile_grid(const ElDev &v) {
+  constexpr int oz = tile::out_rows(4 * NW);
+  return {(v.X - 2 * v.nn + tile::OX - 1) / tile::OX, (v.Z - 2 * v.nn + oz - 1) / oz};
+}
+
+template <int NW>
 void launch_el_fwd_tile_c(const ElDev &v, hipStream_t st, const tile::FwdIO &io) {
-  constexpr int oz = tile::out_rows(NR * NW);
-  tile::Grid g;
-  g.ntx = (v.X - 4 + tile::OX - 1) / tile::OX;
-  g.ntz = (v.Z - 4 + oz - 1) / oz;
-  hipLaunchKernelGGL((tile::el_fwd_tile<NR, NW>), dim3((unsigned)(g.ntx * g.ntz * v.S)), dim3(NW * WAVE), 0, st, v, g, io);
+  const tile::Grid g = el_tile_grid<NW>(v);
+  const dim3 grid((unsigned)(g.ntx * g.ntz * v.S)), block(NW * WAVE);
+  if (v.nn == 2) hipLaunchKernelGGL((tile::el_fwd_tile<2, 4, NW>), grid, block, 0, st, v, g, io);
+  else hipLaunchKernelGGL((tile::el_fwd_tile<3, 4, NW>), grid, block, 0, st, v, g, io);
 }
 
 // Tile heights: 32, 48 and 64 rows (20, 36 and 52 stored).  A launch whose workgroups all run at
 // once lasts as long as one of them, and a lower tile is done sooner: the lowest that gives at most
 // one workgroup per CU.  Above that, 32 rows again: two such workgroups fit a CU and overlap each
 // other's loads, stores and arithmetic, which outweighs their larger halo.  Measured, forward with
-// records, us per step, 32 / 48 / 64 rows: 122 x 240, 1 shot 6.1 / 7.9 / 9.4; 142 x 341, 6 shots
-// (294 / 168 / 126 workgroups) 10.4 / 8.6 / 10.2; 171 x 373, 8 shots (576 / 320 / 256) 14.2 / 15.3 /
-// 11.0; 242 x 680, 32 shots 81 / 119 / 106; 362 x 1040, 48 shots 267 / 390 / 336.
+// records, us per step, 32 / 48 / 64 rows: 122 x 240, 1 shot 5.5 / 7.9 / 9.4; 142 x 341, 6 shots
+// (294 / 168 / 126 workgroups) 10.4 / 7.5 / 10.2; 171 x 373, 8 shots (576 / 320 / 256) 14.2 / 15.3 /
+// 9.7; 242 x 680, 32 shots 80 / 119 / 106; 362 x 1040, 48 shots 271 / 390 / 336.  With three-term
+// differences a launch is one step and the smaller halo counts for more: 64 rows then (214 x 393,
+// 16 shots 37 / 40 / 34; 24 shots 52 / 62 / 50).
 void launch_el_fwd_tile(const ElDev &v, hipStream_t st, const tile::FwdIO &io) {
-  auto count = [&](int rows) {
-    const int oz = tile::out_rows(rows);
-    return (long long)((v.X - 4 + tile::OX - 1) / tile::OX) * ((v.Z - 4 + oz - 1) / oz) * v.S;
-  };
+  auto count = [&](const tile::Grid &g) { return (long long)g.ntx * g.ntz * v.S; };
   constexpr long long CUS = 256;
-  if (count(32) > CUS && count(48) <= CUS) launch_el_fwd_tile_c<4, 12>(v, st, io);
-  else if (count(32) > CUS && count(64) <= CUS) launch_el_fwd_tile_c<4, 16>(v, st, io);
-  else launch_el_fwd_tile_c<4, 8>(v, st, io);
+  if (count(el_tile_grid<8>(v)) <= CUS) launch_el_fwd_tile_c<8>(v, st, io);
+  else if (count(el_tile_grid<12>(v)) <= CUS) launch_el_fwd_tile_c<12>(v, st, io);
+  else if (v.nn > 2 || count(el_tile_grid<16>(v)) <= CUS) launch_el_fwd_tile_c<16>(v, st, io);
+  else launch_el_fwd_tile_c<8>(v, st, io);
 }
 
-template <int NR, int NW>
+template <int NW>
 void launch_el_adj_tile_c(const ElDev &v, hipStream_t st, const tile::AdjIO &io, int groups) {
-  constexpr int oz = tile::out_rows(NR * NW);
-  tile::Grid g;
-  g.ntx = (v.X - 4 + tile::OX - 1) / tile::OX;
-  g.ntz = (v.Z - 4 + oz - 1) / oz;
-  hipLaunchKernelGGL((tile::el_adj_tile<NR, NW>), dim3((unsigned)(g.ntx * g.ntz * groups)), dim3(NW * WAVE), 0, st, v, g, io);
+  const tile::Grid g = el_tile_grid<NW>(v);
+  const dim3 grid((unsigned)(g.ntx * g.ntz * groups)), block(NW * WAVE);
+  if (v.nn == 2) hipLaunchKernelGGL((tile::el_adj_tile<2, 4, NW>), grid, block, 0, st, v, g, io);
+  else hipLaunchKernelGGL((tile::el_adj_tile<3, 4, NW>), grid, block, 0, st, v, g, io);
 }
 
 void launch_el_adj_tile(const ElDev &v, hipStream_t st, const tile::AdjIO &io, const ElAdjTile &sh) {
   static_assert(tile::OX == 52 && tile::out_rows(32) == 32 - 12, "el_adj_tile_shape counts these");
-  if (sh.rows == 32) launch_el_adj_tile_c<4, 8>(v, st, io, sh.groups);
-  else launch_el_adj_tile_c<4, 12>(v, st, io, sh.groups);
+  if (sh.rows == 32) launch_el_adj_tile_c<8>(v, st, io, sh.groups);
+  else launch_el_adj_tile_c<12>(v, st, io, sh.groups);
 }
 
 }  // namespace
@@ -2490,20 +2504,20 @@ int adfwi_elastic_forward(const adfwi_elastic_desc *d, adfwi_elastic_fwd_args *a
   const dim3 ggrid((unsigned)((ng + 255) / 256)), gblock(256);
   // the 4th-order PML step takes its records itself when the receiver map is given
   const bool fused = recs && ng > 0 && d->rcv_map && !d->damping && v.nn == 2;
+  const float *cur = a->state_in;
+  const bool tiles = el_tile_ok(d, v, L, recs && ng > 0);
   ElRec rk{};
-  if (fused) {
+  if (fused || (tiles && recs && ng > 0)) {
     rk.map = d->rcv_map;
     for (int q = 0; q < 5; ++q) rk.r[q] = a->rec[q];
   }
-  const float *cur = a->state_in;
-  const bool tiles = el_tile_ok(d, v, L, recs && ng > 0);
   ADFWI_CHECK_ARG(!a->trace_totals || (a->trace && tiles),
-                  "a trace of totals needs a trace buffer and the tile kernels (4th-order PML without C15 / C35, "
+                  "a trace of totals needs a trace buffer and the tile kernels (PML without C15 / C35, "
                   "library tiling, a receiver map for records, state sets under 2 GiB)");
   if (tiles && (!a->trace || a->trace_totals)) {
     for (int k = 0; k < a->nsteps;) {
       const int t = a->t0 + k;
-      int n = min(tile::TK, a->nsteps - k);
+      int n = min(tile::steps_of(v.nn), a->nsteps - k);
       if (a->ckpt) n = min(n, a->ckpt_every - t % a->ckpt_every);   // up to the next checkpoint
       float *nxt = (cur == a->work[0]) ? a->work[1] : a->work[0];
       if (a->ckpt && (t + n) % a->ckpt_every == 0 && t + n < d->nt)
@@ -2591,7 +2605,7 @@ static int elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *
   if (recs && d->nrec > 0) ADFWI_CHECK_ARG(d->rcv_z && d->rcv_x, "null receiver table pointer");
   ElDev v = el_dev(d, L);
   ADFWI_CHECK_ARG(!totals || el_tile_ok(d, v, L, recs && d->nrec > 0),
-                  "a trace of totals needs the tile kernels (4th-order PML without C15 / C35, library tiling, a "
+                  "a trace of totals needs the tile kernels (PML without C15 / C35, library tiling, a "
                   "receiver map for record adjoints, state sets under 2 GiB)");
   // the free-surface transposes need rows 0..3 inside the first strip (every strip height here
   // is at least 8)
@@ -2628,7 +2642,7 @@ static int elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *
   // the 4th-order PML adjoint step adds the record adjoints itself when the receiver map is given
   const bool fused = recs && ng > 0 && d->rcv_map && !d->damping && v.nn == 2;
   ElInj ij{};
-  if (fused) {
+  if (fused || (totals && recs && ng > 0)) {
     ij.map = d->rcv_map;
     for (int q = 0; q < 5; ++q) ij.g[q] = a->grad_rec[q];
   }
@@ -2639,7 +2653,7 @@ static int elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *
     for (int i = a->nsteps - 1; i >= 0;) {   // two steps per launch, the last launch the odd one
       tile::AdjIO io;
       io.t = t_lo + i;
-      io.n = min(tile::TK, i + 1);
+      io.n = min(tile::steps_of(v.nn), i + 1);
       for (int j = 0; j < tile::TK; ++j) {
         const int q = max(i - j, 0);
         io.fv[j] = q == 0 ? a->fwd0 : a->trace + (long long)(q - 1) * slot;

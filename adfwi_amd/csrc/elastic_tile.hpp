@@ -1,10 +1,10 @@
-// Several steps of the isotropic / VTI 4th-order PML scheme per launch on register tiles
-// (included by elastic.hip; el_fwd_step states one step).
+// The isotropic / VTI PML scheme on register tiles (included by elastic.hip; el_fwd_step and
+// el3_fwd_step state one step): at 4th order two steps per launch, at 6th to 10th one.
 //
 // A workgroup of NW wavefronts holds a tile of NW*NR rows x 64 columns of one shot in registers
-// (NR rows x 1 column per lane: the ten splits and six coefficients), advances it up to TK = 2
-// steps and stores the points whose stencils never left the tile: a step reaches 3 points in each
-// direction (the free-surface rows 2), so 6 points on every side are halo.  x-neighbours come
+// (NR rows x 1 column per lane: the ten splits and six coefficients), advances it and stores the
+// points whose stencils never left the tile: a step reaches 3 points in each direction with
+// two-term differences and 5 with three, so 6 points on every side are halo.  x-neighbours come
 // from the adjacent lanes (DPP wavefront shifts), z-neighbours from registers and, between
 // wavefronts, through LDS: the edge rows of the velocity totals before the stress update, those
 // of the stress totals before the velocity update.  Outside the update window the coefficients
@@ -15,8 +15,10 @@
 // launch's steps.
 namespace tile {
 
-constexpr int TK = 2;              // steps per launch (at most)
-constexpr int H = 3 * TK;          // halo points per side
+// Differences of ORD terms: 2 (4th order) or 3 (6th to 10th)
+__host__ __device__ constexpr int steps_of(int ord) { return ord == 2 ? 2 : 1; }   // steps per launch (at most)
+constexpr int TK = steps_of(2);
+constexpr int H = 6;               // halo points per side: 3 per step with 2 terms, 5 with 3
 constexpr int OX = WAVE - 2 * H;   // stored columns
 constexpr int out_rows(int rows) { return rows - 2 * H; }
 constexpr unsigned DROP = 0x80000000u;   // a lane offset past every buffer (all under 2 GiB): access dropped
@@ -48,6 +50,73 @@ __device__ __forceinline__ T scalar_ld(const T *p) {
 
 struct Grid { int ntx, ntz; };
 
+// the ORD-term staggered differences and their transposes: along x by wavefront shifts, along z
+// about row r of an accessor
+template <int ORD>
+struct Fd {
+  float c0, c1, c2;
+  __device__ __forceinline__ float dxf(float v) const {
+    const float l1 = from_left(v), r1 = from_right(v), r2 = from_right(r1);
+    const float s = c0 * (r1 - v) + c1 * (r2 - l1);
+    return ORD == 2 ? s : s + c2 * (from_right(r2) - from_left(l1));
+  }
+  __device__ __forceinline__ float dxb(float v) const {
+    const float l1 = from_left(v), l2 = from_left(l1), r1 = from_right(v);
+    const float s = c0 * (v - l1) + c1 * (r1 - l2);
+    return ORD == 2 ? s : s + c2 * (from_right(r1) - from_left(l2));
+  }
+  __device__ __forceinline__ float dxfT(float v) const {
+    const float l1 = from_left(v), l2 = from_left(l1), r1 = from_right(v);
+    const float s = c0 * (l1 - v) + c1 * (l2 - r1);
+    return ORD == 2 ? s : s + c2 * (from_left(l2) - from_right(r1));
+  }
+  __device__ __forceinline__ float dxbT(float v) const {
+    const float l1 = from_left(v), r1 = from_right(v), r2 = from_right(r1);
+    const float s = c0 * (v - r1) + c1 * (l1 - r2);
+    return ORD == 2 ? s : s + c2 * (from_left(l1) - from_right(r2));
+  }
+  template <class W> __device__ __forceinline__ float dzf(const W &w, int r) const {
+    const float s = c0 * (w(r + 1) - w(r)) + c1 * (w(r + 2) - w(r - 1));
+    return ORD == 2 ? s : s + c2 * (w(r + 3) - w(r - 2));
+  }
+  template <class W> __device__ __forceinline__ float dzb(const W &w, int r) const {
+    const float s = c0 * (w(r) - w(r - 1)) + c1 * (w(r + 1) - w(r - 2));
+    return ORD == 2 ? s : s + c2 * (w(r + 2) - w(r - 3));
+  }
+  template <class W> __device__ __forceinline__ float dzfT(const W &w, int r) const {
+    const float s = c0 * (w(r - 1) - w(r)) + c1 * (w(r - 2) - w(r + 1));
+    return ORD == 2 ? s : s + c2 * (w(r - 3) - w(r + 2));
+  }
+  template <class W> __device__ __forceinline__ float dzbT(const W &w, int r) const {
+    const float s = c0 * (w(r) - w(r + 1)) + c1 * (w(r - 1) - w(r + 2));
+    return ORD == 2 ? s : s + c2 * (w(r - 2) - w(r + 3));
+  }
+};
+
+// A wavefront's NR rows with the A rows above and the B below them from its neighbours, through an
+// LDS buffer of A + B rows per wavefront (its first B and its last A), written by put before a
+// barrier and read by get after it.  dzb and dzfT take A = ORD, B = ORD - 1, dzf and dzbT the reverse.
+template <int A, int B, int NR>
+struct Rows {
+  const float (&v)[NR];
+  float a[A], b[B];
+  template <int Q>
+  static __device__ __forceinline__ void put(float (*buf)[Q][WAVE], int wv, int slot, int lane, const float (&v)[NR]) {
+#pragma unroll
+    for (int j = 0; j < B; ++j) buf[wv + 1][slot + j][lane] = v[j];
+#pragma unroll
+    for (int j = 0; j < A; ++j) buf[wv + 1][slot + B + j][lane] = v[NR - A + j];
+  }
+  template <int Q>
+  __device__ __forceinline__ Rows(const float (*buf)[Q][WAVE], int wv, int slot, int lane, const float (&v_)[NR]) : v(v_) {
+#pragma unroll
+    for (int j = 0; j < A; ++j) a[j] = buf[wv][slot + B + j][lane];
+#pragma unroll
+    for (int j = 0; j < B; ++j) b[j] = buf[wv + 2][slot + j][lane];
+  }
+  __device__ __forceinline__ float operator()(int r) const { return r < 0 ? a[r + A] : r >= NR ? b[r - NR] : v[r]; }
+};
+
 struct FwdIO {
   const float *in;
   float *out;
@@ -72,34 +141,39 @@ __device__ __forceinline__ void place(const Grid &g, int &tx, int &tz, int &s) {
   tx = tl - tz * g.ntx;
 }
 
-template <int NR, int NW>
-__global__ __launch_bounds__(NW *WAVE) void el_fwd_tile(ElDev d, Grid g, FwdIO io) {
-  static_assert(NR == 4 && H == 6, "rows 0 .. 3, which the free surface ties together, are wavefront 1 of the first tiles");
+template <int ORD, int NR, int NW>
+__global__ __launch_bounds__(NW *WAVE, 4) void el_fwd_tile(ElDev d, Grid g, FwdIO io) {
+  static_assert(NR == 4 && H == 6, "rows nn-2 .. nn+1, which the free surface ties together, are wavefront 1 of the first tiles");
+  using Up = Rows<ORD, ORD - 1, NR>;
+  using Dn = Rows<ORD - 1, ORD, NR>;
+  constexpr int Q = 2 * ORD - 1;   // LDS rows of either
+  const int nn = ORD == 2 ? 2 : d.nn;
   constexpr int OZ = out_rows(NR * NW);
-  __shared__ float sv[NW + 2][6][WAVE], ss[NW + 2][6][WAVE];
+  constexpr int QN = 2 * (2 * ORD - 1);
+  __shared__ float sv[NW + 2][QN][WAVE], ss[NW + 2][QN][WAVE];
   int tx, tzi, s;
   place(g, tx, tzi, s);
   const int lane = threadIdx.x & (WAVE - 1);
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
   if (wv == 0) {
 #pragma unroll
-    for (int q = 0; q < 6; ++q) sv[0][q][lane] = sv[NW + 1][q][lane] = ss[0][q][lane] = ss[NW + 1][q][lane] = 0.f;
+    for (int q = 0; q < QN; ++q) sv[0][q][lane] = sv[NW + 1][q][lane] = ss[0][q][lane] = ss[NW + 1][q][lane] = 0.f;
   }
-  const int x0 = 2 + tx * OX, z0 = 2 + tzi * OZ;            // first stored column and row
+  const int x0 = nn + tx * OX, z0 = nn + tzi * OZ;            // first stored column and row
   const int c = x0 - H + lane, zt = z0 - H + wv * NR;       // this lane's column, this wavefront's first row
-  const int zw1 = d.Z - 3;
+  const int zw1 = d.Z - nn - 1, xw1 = d.X - nn - 1;   // the window's last row and column
   const unsigned rowb = 4u * (unsigned)d.pitch, planeb = 4u * (unsigned)d.plane, fieldb = 4u * (unsigned)d.field;
   const unsigned vin = c >= 0 && c < d.X ? 4u * (unsigned)c : DROP;
-  const bool own = c >= x0 && c < min(x0 + OX, d.X - 2);
+  const bool own = c >= x0 && c < min(x0 + OX, xw1 + 1);
   const unsigned vout = own ? 4u * (unsigned)c : DROP;
-  const bool cwin = c >= 2 && c <= d.X - 3;
+  const bool cwin = c >= nn && c <= xw1;
   auto bits = [&](int lo, int hi) -> unsigned {   // rows lo .. hi-1 of this wavefront
     const int a = min(max(lo - zt, 0), NR), b = min(max(hi - zt, 0), NR);
     return b > a ? ((1u << b) - 1u) & ~((1u << a) - 1u) : 0u;
   };
   const unsigned ownbits = bits(z0, min(z0 + OZ, zw1 + 1));
   auto off = [&](int row) -> unsigned { return (unsigned)min(max(row, 0), d.Z - 1) * rowb; };
-  const float c0 = d.c0, c1 = d.c1;
+  const Fd<ORD> D{d.c0, d.c1, ORD == 2 ? 0.f : d.c2};
 
   // ten splits; rows outside the grid repeat an edge row, whose splits are zero as theirs would be
   float f[NFIELD][NR];
@@ -115,7 +189,7 @@ __global__ __launch_bounds__(NW *WAVE) void el_fwd_tile(ElDev d, Grid g, FwdIO i
     const rsrc_t rC = rsrc(d.coef, (unsigned)NCOEF * planeb);
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
-      const unsigned v = cwin && zt + r >= 2 && zt + r <= zw1 ? vin : DROP;   // (dropped loads return 0)
+      const unsigned v = cwin && zt + r >= nn && zt + r <= zw1 ? vin : DROP;   // (dropped loads return 0)
 #pragma unroll
       for (int q = 0; q < 4; ++q) C[q][r] = bld(rC, v, (unsigned)q * planeb + off(zt + r));
       bx[r] = bld(rC, v, BX * planeb + off(zt + r));
@@ -131,7 +205,7 @@ __global__ __launch_bounds__(NW *WAVE) void el_fwd_tile(ElDev d, Grid g, FwdIO i
   for (int r = 0; r < NR; ++r) rpz[r] = 1.0 / (double)pz(1, r);
   const int zs = scalar_ld(d.src_z + s), xs = scalar_ld(d.src_x + s);
   const bool src_here = zs >= zt && zs < zt + NR;
-  const bool fsw = d.fsurf && tzi == 0 && wv == 1;          // this wavefront's rows are 0 .. 3
+  const bool fsw = d.fsurf && tzi == 0 && wv == 1;          // this wavefront's rows are nn-2 .. nn+1
   unsigned rbits = 0;
   if (io.rec.map) {
     const bool mine = lane < NR && ((ownbits >> (lane & 31)) & 1u);
@@ -147,12 +221,12 @@ __global__ __launch_bounds__(NW *WAVE) void el_fwd_tile(ElDev d, Grid g, FwdIO i
 #pragma unroll 1
   for (int i = 0; i < io.n; ++i) {
     const float wsrc = src_here ? scalar_ld(d.src + (long long)s * d.nt + io.t + i) : 0.f;
-    // velocity totals, the free-surface rows 0 and 1 from rows 2 and 3
+    // velocity totals, the free-surface rows nn-2 and nn-1 from rows nn and nn+1
     float vx[NR], vz[NR];
 #pragma unroll
     for (int r = 0; r < NR; ++r) { vx[r] = f[VX_X][r] + f[VX_Z][r]; vz[r] = f[VZ_X][r] + f[VZ_Z][r]; }
     if (fsw) {
-      const bool jj1 = c + 1 >= 2 && c + 1 <= d.X - 3;
+      const bool jj1 = c + 1 >= nn && c + 1 <= xw1;
       const float vz2n = from_right(vz[2]);
       const float vz1m_n = jj1 ? vz2n : 0.0f;
       const float vz1m = cwin ? vz[2] : vz[1];
@@ -162,23 +236,17 @@ __global__ __launch_bounds__(NW *WAVE) void el_fwd_tile(ElDev d, Grid g, FwdIO i
       }
       vz[1] = vz1m;
     }
-    sv[wv + 1][0][lane] = vx[0]; sv[wv + 1][1][lane] = vx[1]; sv[wv + 1][2][lane] = vx[NR - 1];
-    sv[wv + 1][3][lane] = vz[0]; sv[wv + 1][4][lane] = vz[NR - 2]; sv[wv + 1][5][lane] = vz[NR - 1];
+    Dn::put(sv, wv, 0, lane, vx);
+    Up::put(sv, wv, Q, lane, vz);
     lds_barrier();
     {
-      const float xa = sv[wv][2][lane], xb1 = sv[wv + 2][0][lane], xb2 = sv[wv + 2][1][lane];
-      const float za2 = sv[wv][4][lane], za1 = sv[wv][5][lane], zb = sv[wv + 2][3][lane];
-      auto VXr = [&](int r) { return r < 0 ? xa : r == NR ? xb1 : r > NR ? xb2 : vx[r]; };
-      auto VZr = [&](int r) { return r == -2 ? za2 : r == -1 ? za1 : r >= NR ? zb : vz[r]; };
+      const Dn VXr(sv, wv, 0, lane, vx);
+      const Up VZr(sv, wv, Q, lane, vz);
 #pragma unroll
       for (int r = 0; r < NR; ++r) {
         __builtin_amdgcn_sched_barrier(0);
-        const float xl1 = from_left(vx[r]), xl2 = from_left(xl1), xr1 = from_right(vx[r]);
-        const float zl1 = from_left(vz[r]), zr1 = from_right(vz[r]), zr2 = from_right(zr1);
-        const float dxb_vx = c0 * (vx[r] - xl1) + c1 * (xr1 - xl2);
-        const float dzb_vz = c0 * (vz[r] - VZr(r - 1)) + c1 * (VZr(r + 1) - VZr(r - 2));
-        const float dxf_vz = c0 * (zr1 - vz[r]) + c1 * (zr2 - zl1);
-        const float dzf_vx = c0 * (VXr(r + 1) - vx[r]) + c1 * (VXr(r + 2) - VXr(r - 1));
+        const float dxb_vx = D.dxb(vx[r]), dzb_vz = D.dzb(VZr, r);
+        const float dxf_vz = D.dxf(vz[r]), dzf_vx = D.dzf(VXr, r);
         const float pzn = pz(0, r), pzi = pz(2, r);
         f[TXX_X][r] = (pxn * f[TXX_X][r] + d.dt_dx * (C[0][r] * dxb_vx)) * pxi;
         f[TXX_Z][r] = (pzn * f[TXX_Z][r] + d.dt_dz * (C[1][r] * dzb_vz)) * pzi;
@@ -216,7 +284,7 @@ __global__ __launch_bounds__(NW *WAVE) void el_fwd_tile(ElDev d, Grid g, FwdIO i
         if ((rbits >> r) & 1u) {
           const unsigned v = rec_off(r);
           bst(xx[r], rsrc(io.rec.r[TXX] + ro, rbytes), v, 0u);
-          bst(d.fsurf && zt + r == 2 ? 0.0f : zz[r], rsrc(io.rec.r[TZZ] + ro, rbytes), v, 0u);
+          bst(d.fsurf && zt + r == nn ? 0.0f : zz[r], rsrc(io.rec.r[TZZ] + ro, rbytes), v, 0u);
           bst(xz[r], rsrc(io.rec.r[TXZ] + ro, rbytes), v, 0u);
         }
     }
@@ -235,23 +303,17 @@ __global__ __launch_bounds__(NW *WAVE) void el_fwd_tile(ElDev d, Grid g, FwdIO i
       zz[1] = -zz[3]; zz[2] = 0.0f;
       xz[1] = -xz[2]; xz[0] = -xz[3];
     }
-    ss[wv + 1][0][lane] = zz[0]; ss[wv + 1][1][lane] = zz[1]; ss[wv + 1][2][lane] = zz[NR - 1];
-    ss[wv + 1][3][lane] = xz[0]; ss[wv + 1][4][lane] = xz[NR - 2]; ss[wv + 1][5][lane] = xz[NR - 1];
+    Dn::put(ss, wv, 0, lane, zz);
+    Up::put(ss, wv, Q, lane, xz);
     lds_barrier();
     {
-      const float za = ss[wv][2][lane], zb1 = ss[wv + 2][0][lane], zb2 = ss[wv + 2][1][lane];
-      const float xa2 = ss[wv][4][lane], xa1 = ss[wv][5][lane], xb = ss[wv + 2][3][lane];
-      auto ZZr = [&](int r) { return r < 0 ? za : r == NR ? zb1 : r > NR ? zb2 : zz[r]; };
-      auto XZr = [&](int r) { return r == -2 ? xa2 : r == -1 ? xa1 : r >= NR ? xb : xz[r]; };
+      const Dn ZZr(ss, wv, 0, lane, zz);
+      const Up XZr(ss, wv, Q, lane, xz);
 #pragma unroll
       for (int r = 0; r < NR; ++r) {
         __builtin_amdgcn_sched_barrier(0);
-        const float tl1 = from_left(xx[r]), tr1 = from_right(xx[r]), tr2 = from_right(tr1);
-        const float ul1 = from_left(xz[r]), ul2 = from_left(ul1), ur1 = from_right(xz[r]);
-        const float dxf_txx = c0 * (tr1 - xx[r]) + c1 * (tr2 - tl1);
-        const float dzb_txz = c0 * (xz[r] - XZr(r - 1)) + c1 * (XZr(r + 1) - XZr(r - 2));
-        const float dxb_txz = c0 * (xz[r] - ul1) + c1 * (ur1 - ul2);
-        const float dzf_tzz = c0 * (ZZr(r + 1) - zz[r]) + c1 * (ZZr(r + 2) - ZZr(r - 1));
+        const float dxf_txx = D.dxf(xx[r]), dzb_txz = D.dzb(XZr, r);
+        const float dxb_txz = D.dxb(xz[r]), dzf_tzz = D.dzf(ZZr, r);
         const float pzn = pz(0, r);
         f[VX_X][r] = quot(pxn * f[VX_X][r] + quot((d.dt * bx[r]) * dxf_txx, rdx), rpx);
         f[VX_Z][r] = quot(pzn * f[VX_Z][r] + quot((d.dt * bx[r]) * dzb_txz, rdz), rpz[r]);
@@ -329,27 +391,31 @@ __device__ __forceinline__ float pick(int m, float a, float b) {   // bits of a 
 // and el_adj_step took 251; 362 x 1040, 48 shots: 474, 409, 779.  Adjoint splits outside the window, which
 // el_adj_step keeps at zero, take values here, but nothing reads them: the coefficients there are
 // zero, and they are not stored.
-template <int NR, int NW>
+template <int ORD, int NR, int NW>
 __global__ __launch_bounds__(NW *WAVE, NW / 4) void el_adj_tile(ElDev d, Grid g, AdjIO io) {
-  static_assert(NR == 4 && H == 6, "rows 0 .. 3, which the free surface ties together, are wavefront 1 of the first tiles");
+  static_assert(NR == 4 && H == 6, "rows nn-2 .. nn+1, which the free surface ties together, are wavefront 1 of the first tiles");
+  using Up = Rows<ORD, ORD - 1, NR>;
+  using Dn = Rows<ORD - 1, ORD, NR>;
+  constexpr int Q = 2 * ORD - 1;   // LDS rows of either
+  const int nn = ORD == 2 ? 2 : d.nn;
   constexpr int OZ = out_rows(NR * NW);
-  __shared__ float sv[NW + 2][18][WAVE], ss[NW + 2][6][WAVE];
+  __shared__ float sv[NW + 2][6 * (2 * ORD - 1)][WAVE], ss[NW + 2][2 * (2 * ORD - 1)][WAVE];
   int tx, tzi, grp;
   place(g, tx, tzi, grp);
   const int lane = threadIdx.x & (WAVE - 1);
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
   if (wv == 0) {
 #pragma unroll
-    for (int q = 0; q < 18; ++q) sv[0][q][lane] = sv[NW + 1][q][lane] = 0.f;
+    for (int q = 0; q < 6 * Q; ++q) sv[0][q][lane] = sv[NW + 1][q][lane] = 0.f;
 #pragma unroll
-    for (int q = 0; q < 6; ++q) ss[0][q][lane] = ss[NW + 1][q][lane] = 0.f;
+    for (int q = 0; q < 2 * Q; ++q) ss[0][q][lane] = ss[NW + 1][q][lane] = 0.f;
   }
-  const int x0 = 2 + tx * OX, z0 = 2 + tzi * OZ;
+  const int x0 = nn + tx * OX, z0 = nn + tzi * OZ;
   const int c = x0 - H + lane, zt = z0 - H + wv * NR;
-  const int zw1 = d.Z - 3;
+  const int zw1 = d.Z - nn - 1, xw1 = d.X - nn - 1;   // the window's last row and column
   const unsigned rowb = 4u * (unsigned)d.pitch, planeb = 4u * (unsigned)d.plane, fieldb = 4u * (unsigned)d.field;
-  const bool own = c >= x0 && c < min(x0 + OX, d.X - 2);
-  const bool cwin = c >= 2 && c <= d.X - 3;
+  const bool own = c >= x0 && c < min(x0 + OX, xw1 + 1);
+  const bool cwin = c >= nn && c <= xw1;
   auto bits = [&](int lo, int hi) -> unsigned {   // rows lo .. hi-1 of this wavefront
     const int a = min(max(lo - zt, 0), NR), b = min(max(hi - zt, 0), NR);
     return b > a ? ((1u << b) - 1u) & ~((1u << a) - 1u) : 0u;
@@ -362,13 +428,13 @@ __global__ __launch_bounds__(NW *WAVE, NW / 4) void el_adj_tile(ElDev d, Grid g,
   for (int r = 0; r < NR; ++r)
     vi[r] = c >= 0 && c < d.X && zt + r >= 0 && zt + r < d.Z ? (unsigned)(zt + r) * rowb + 4u * (unsigned)c : DROP;
   auto vo = [&](int r) -> unsigned { return own && ((ownbits >> r) & 1u) ? vi[r] : DROP; };
-  const float c0 = d.c0, c1 = d.c1;
+  const Fd<ORD> D{d.c0, d.c1, ORD == 2 ? 0.f : d.c2};
   float C[4][NR], bx[NR], bz[NR];
   {
     const rsrc_t rC = rsrc(d.coef, (unsigned)NCOEF * planeb);
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
-      const unsigned v = cwin && zt + r >= 2 && zt + r <= zw1 ? vi[r] : DROP;
+      const unsigned v = cwin && zt + r >= nn && zt + r <= zw1 ? vi[r] : DROP;
 #pragma unroll
       for (int q = 0; q < 4; ++q) C[q][r] = bld(rC, v, (unsigned)q * planeb);
       bx[r] = bld(rC, v, BX * planeb);
@@ -390,14 +456,14 @@ __global__ __launch_bounds__(NW *WAVE, NW / 4) void el_adj_tile(ElDev d, Grid g,
     sz_keep[r] = uni(pzn * pzi); sz_a[r] = uni(d.dt_dz * pzi);
     vz_keep[r] = uni(pzn / pzd); vz_w[r] = uni(d.dt / (d.dz * pzd));
   }
-  // masks: the free surface's wavefront (rows 0 .. 3), window columns c, c + 1 and c - 1
+  // masks: the free surface's wavefront (rows nn-2 .. nn+1), window columns c, c + 1 and c - 1
   int mfs = __builtin_amdgcn_readfirstlane(d.fsurf && tzi == 0 && wv == 1 ? -1 : 0);
   asm volatile("" : "+s"(mfs));
-  auto in_win = [&](int x) -> int { int m = x >= 2 && x <= d.X - 3 ? -1 : 0; asm volatile("" : "+v"(m)); return m; };
+  auto in_win = [&](int x) -> int { int m = x >= nn && x <= xw1 ? -1 : 0; asm volatile("" : "+v"(m)); return m; };
   const int mcw = in_win(c), mj1 = in_win(c + 1), mm1 = in_win(c - 1), mfc = mfs & mcw;
   unsigned rbits = 0;   // rows with receivers: of the halo, too
   if (io.inj.map) {
-    const bool mine = lane < NR && zt + lane >= 2 && zt + lane <= zw1;
+    const bool mine = lane < NR && zt + lane >= nn && zt + lane <= zw1;
     rbits = (unsigned)__ballot(mine && io.inj.map[mine ? zt + lane : 0] > 0);
   }
   float G[6][NR];
@@ -449,7 +515,7 @@ __global__ __launch_bounds__(NW *WAVE, NW / 4) void el_adj_tile(ElDev d, Grid g,
           if ((rbits >> r) & 1u) {
             const int m = __builtin_bit_cast(int, bld(rsrc(io.inj.map + d.Z, planeb), vi[r], 0u));
             const unsigned v = cwin && m >= 0 ? 4u * (unsigned)m : DROP;
-            const float axx = adj(TXX, v), azz = adj(TZZ, d.fsurf && zt + r == 2 ? DROP : v), axz = adj(TXZ, v);
+            const float axx = adj(TXX, v), azz = adj(TZZ, d.fsurf && zt + r == nn ? DROP : v), axz = adj(TXZ, v);
             const float avx = adj(VX, v), avz = adj(VZ, v);
             f[TXX_X][r] += axx; f[TXX_Z][r] += axx; f[TZZ_X][r] += azz; f[TZZ_Z][r] += azz;
             f[TXZ_X][r] += axz; f[TXZ_Z][r] += axz; f[VX_X][r] += avx; f[VX_Z][r] += avx;
@@ -463,7 +529,7 @@ __global__ __launch_bounds__(NW *WAVE, NW / 4) void el_adj_tile(ElDev d, Grid g,
         eb[r] = f[VX_Z][r] * (vz_w[r] * bx[r]);
         ed[r] = f[VZ_Z][r] * (vz_w[r] * bz[r]);
       }
-      // forward free surface: velocity rows 0 and 1 from rows 2 and 3, stress rows 0 .. 2.  Bit
+      // forward free surface: velocity rows nn-2 and nn-1, stress rows nn-2 .. nn.  Bit
       // masks, not branches, here and below: the sides of a branch (or of a select, which becomes
       // one) share terms with what follows, and holding those cost 90 registers
       {
@@ -477,27 +543,21 @@ __global__ __launch_bounds__(NW *WAVE, NW / 4) void el_adj_tile(ElDev d, Grid g,
         zz[1] = pick(mfs, -zz[3], zz[1]); zz[2] = keep(~mfs, zz[2]);
         xz[1] = pick(mfs, -xz[2], xz[1]); xz[0] = pick(mfs, -xz[3], xz[0]);
       }
-      sv[wv + 1][0][lane] = eb[0]; sv[wv + 1][1][lane] = eb[1]; sv[wv + 1][2][lane] = eb[NR - 1];
-      sv[wv + 1][3][lane] = ed[0]; sv[wv + 1][4][lane] = ed[NR - 2]; sv[wv + 1][5][lane] = ed[NR - 1];
-      sv[wv + 1][6][lane] = vx[0]; sv[wv + 1][7][lane] = vx[1]; sv[wv + 1][8][lane] = vx[NR - 1];
-      sv[wv + 1][9][lane] = vz[0]; sv[wv + 1][10][lane] = vz[NR - 2]; sv[wv + 1][11][lane] = vz[NR - 1];
-      sv[wv + 1][12][lane] = zz[0]; sv[wv + 1][13][lane] = zz[1]; sv[wv + 1][14][lane] = zz[NR - 1];
-      sv[wv + 1][15][lane] = xz[0]; sv[wv + 1][16][lane] = xz[NR - 2]; sv[wv + 1][17][lane] = xz[NR - 1];
+      Dn::put(sv, wv, 0, lane, eb);
+      Up::put(sv, wv, Q, lane, ed);
+      Dn::put(sv, wv, 2 * Q, lane, vx);
+      Up::put(sv, wv, 3 * Q, lane, vz);
+      Dn::put(sv, wv, 4 * Q, lane, zz);
+      Up::put(sv, wv, 5 * Q, lane, xz);
       lds_barrier();
       {   // buoyancy gradients: velocity adjoints as they are now, forward stress derivatives
-        const float za = sv[wv][14][lane], zb1 = sv[wv + 2][12][lane], zb2 = sv[wv + 2][13][lane];
-        const float xa2 = sv[wv][16][lane], xa1 = sv[wv][17][lane], xb = sv[wv + 2][15][lane];
-        auto ZZr = [&](int r) { return r < 0 ? za : r == NR ? zb1 : r > NR ? zb2 : zz[r]; };
-        auto XZr = [&](int r) { return r == -2 ? xa2 : r == -1 ? xa1 : r >= NR ? xb : xz[r]; };
+        const Dn ZZr(sv, wv, 4 * Q, lane, zz);
+        const Up XZr(sv, wv, 5 * Q, lane, xz);
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
           __builtin_amdgcn_sched_barrier(0);
-          const float tl1 = from_left(xx[r]), tr1 = from_right(xx[r]), tr2 = from_right(tr1);
-          const float ul1 = from_left(xz[r]), ul2 = from_left(ul1), ur1 = from_right(xz[r]);
-          const float dxf_txx = c0 * (tr1 - xx[r]) + c1 * (tr2 - tl1);
-          const float dzb_txz = c0 * (xz[r] - XZr(r - 1)) + c1 * (XZr(r + 1) - XZr(r - 2));
-          const float dxb_txz = c0 * (xz[r] - ul1) + c1 * (ur1 - ul2);
-          const float dzf_tzz = c0 * (ZZr(r + 1) - zz[r]) + c1 * (ZZr(r + 2) - ZZr(r - 1));
+          const float dxf_txx = D.dxf(xx[r]), dzb_txz = D.dzb(XZr, r);
+          const float dxb_txz = D.dxb(xz[r]), dzf_tzz = D.dzf(ZZr, r);
           G[4][r] += f[VX_X][r] * (vx_w * dxf_txx) + f[VX_Z][r] * (vz_w[r] * dzb_txz);
           G[5][r] += f[VZ_X][r] * (vx_w * dxb_txz) + f[VZ_Z][r] * (vz_w[r] * dzf_tzz);
           pin(G[4][r], G[5][r]);
@@ -505,24 +565,15 @@ __global__ __launch_bounds__(NW *WAVE, NW / 4) void el_adj_tile(ElDev d, Grid g,
       }
       float P1[NR], Q2[NR], Q3[NR], P4[NR];
       {
-        const float eba = sv[wv][2][lane], ebb1 = sv[wv + 2][0][lane], ebb2 = sv[wv + 2][1][lane];
-        const float eda2 = sv[wv][4][lane], eda1 = sv[wv][5][lane], edb = sv[wv + 2][3][lane];
-        const float xa = sv[wv][8][lane], xb1 = sv[wv + 2][6][lane], xb2 = sv[wv + 2][7][lane];
-        const float za2 = sv[wv][10][lane], za1 = sv[wv][11][lane], zb = sv[wv + 2][9][lane];
-        auto EB = [&](int r) { return r < 0 ? eba : r == NR ? ebb1 : r > NR ? ebb2 : eb[r]; };
-        auto ED = [&](int r) { return r == -2 ? eda2 : r == -1 ? eda1 : r >= NR ? edb : ed[r]; };
-        auto VXr = [&](int r) { return r < 0 ? xa : r == NR ? xb1 : r > NR ? xb2 : vx[r]; };
-        auto VZr = [&](int r) { return r == -2 ? za2 : r == -1 ? za1 : r >= NR ? zb : vz[r]; };
+        const Dn EB(sv, wv, 0, lane, eb), VXr(sv, wv, 2 * Q, lane, vx);
+        const Up ED(sv, wv, Q, lane, ed), VZr(sv, wv, 3 * Q, lane, vz);
         float ltxz0 = 0.f, ltxz1 = 0.f, ltzz1 = 0.f;
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
           __builtin_amdgcn_sched_barrier(0);
           const float ea = f[VX_X][r] * (vx_w * bx[r]), ec = f[VZ_X][r] * (vx_w * bz[r]);
-          const float e1m1 = from_left(ea), e1m2 = from_left(e1m1), e1p1 = from_right(ea);
-          const float e3p1 = from_right(ec), e3m1 = from_left(ec), e3p2 = from_right(e3p1);
-          const float lt_xx = c0 * (e1m1 - ea) + c1 * (e1m2 - e1p1);
-          float lt_xz = (c0 * (eb[r] - EB(r + 1)) + c1 * (EB(r - 1) - EB(r + 2))) + (c0 * (ec - e3p1) + c1 * (e3m1 - e3p2));
-          float lt_zz = c0 * (ED(r - 1) - ed[r]) + c1 * (ED(r - 2) - ED(r + 1));
+          const float lt_xx = D.dxfT(ea);
+          float lt_xz = D.dzbT(EB, r) + D.dxbT(ec), lt_zz = D.dzfT(ED, r);
           // stress free surface transposed
           if (r == 0) ltxz0 = keep(mfs, lt_xz);
           if (r == 1) { ltzz1 = keep(mfs, lt_zz); ltxz1 = keep(mfs, lt_xz); }
@@ -541,12 +592,8 @@ __global__ __launch_bounds__(NW *WAVE, NW / 4) void el_adj_tile(ElDev d, Grid g,
           Q2[r] = C[1][r] * axx_z + C[2][r] * azz_z;
           Q3[r] = C[3][r] * axz_x;
           P4[r] = C[3][r] * axz_z;
-          const float xl1 = from_left(vx[r]), xl2 = from_left(xl1), xr1 = from_right(vx[r]);
-          const float zl1 = from_left(vz[r]), zr1 = from_right(vz[r]), zr2 = from_right(zr1);
-          const float dxb_vx = c0 * (vx[r] - xl1) + c1 * (xr1 - xl2);
-          const float dzb_vz = c0 * (vz[r] - VZr(r - 1)) + c1 * (VZr(r + 1) - VZr(r - 2));
-          const float dxf_vz = c0 * (zr1 - vz[r]) + c1 * (zr2 - zl1);
-          const float dzf_vx = c0 * (VXr(r + 1) - vx[r]) + c1 * (VXr(r + 2) - VXr(r - 1));
+          const float dxb_vx = D.dxb(vx[r]), dzb_vz = D.dzb(VZr, r);
+          const float dxf_vz = D.dxf(vz[r]), dzf_vx = D.dzf(VXr, r);
           G[0][r] += axx_x * dxb_vx;
           G[1][r] += axx_z * dzb_vz + azz_x * dxb_vx;
           G[2][r] += azz_z * dzb_vz;
@@ -555,8 +602,8 @@ __global__ __launch_bounds__(NW *WAVE, NW / 4) void el_adj_tile(ElDev d, Grid g,
           pin(P1[r], Q2[r]); pin(Q3[r], P4[r]);
         }
       }
-      ss[wv + 1][0][lane] = Q2[0]; ss[wv + 1][1][lane] = Q2[1]; ss[wv + 1][2][lane] = Q2[NR - 1];
-      ss[wv + 1][3][lane] = P4[0]; ss[wv + 1][4][lane] = P4[NR - 2]; ss[wv + 1][5][lane] = P4[NR - 1];
+      Dn::put(ss, wv, 0, lane, Q2);
+      Up::put(ss, wv, Q, lane, P4);
       if (src_here) {
         const float mxx = d.src_m[3 * s], mzz = d.src_m[3 * s + 1], mxz = d.src_m[3 * s + 2];
 #pragma unroll
@@ -570,18 +617,13 @@ __global__ __launch_bounds__(NW *WAVE, NW / 4) void el_adj_tile(ElDev d, Grid g,
       }
       lds_barrier();
       {
-        const float qa = ss[wv][2][lane], qb1 = ss[wv + 2][0][lane], qb2 = ss[wv + 2][1][lane];
-        const float pa2 = ss[wv][4][lane], pa1 = ss[wv][5][lane], pb = ss[wv + 2][3][lane];
-        auto Q2r = [&](int r) { return r < 0 ? qa : r == NR ? qb1 : r > NR ? qb2 : Q2[r]; };
-        auto P4r = [&](int r) { return r == -2 ? pa2 : r == -1 ? pa1 : r >= NR ? pb : P4[r]; };
+        const Dn Q2r(ss, wv, 0, lane, Q2);
+        const Up P4r(ss, wv, Q, lane, P4);
         float lvz0 = 0.f, lvz1 = 0.f, lvx1 = 0.f;
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
           __builtin_amdgcn_sched_barrier(0);
-          const float p1p1 = from_right(P1[r]), p1p2 = from_right(p1p1), p1m1 = from_left(P1[r]);
-          const float q3m1 = from_left(Q3[r]), q3m2 = from_left(q3m1), q3p1 = from_right(Q3[r]);
-          float lvx = (c0 * (P1[r] - p1p1) + c1 * (p1m1 - p1p2)) + (c0 * (P4r(r - 1) - P4[r]) + c1 * (P4r(r - 2) - P4r(r + 1)));
-          float lvz = (c0 * (Q2[r] - Q2r(r + 1)) + c1 * (Q2r(r - 1) - Q2r(r + 2))) + (c0 * (q3m1 - Q3[r]) + c1 * (q3m2 - q3p1));
+          float lvx = D.dxbT(P1[r]) + D.dzfT(P4r, r), lvz = D.dzbT(Q2r, r) + D.dxfT(Q3[r]);
           if (r == 0) lvz0 = lvz;
           if (r == 1) { lvz1 = lvz; lvx1 = lvx; }
           if (r == 2) lvz = lvz + keep(mfs, ((lvz1 + lvz0) - 2.0f * lvx1) + keep(mm1, 2.0f * from_left(lvx1)));

@@ -11,7 +11,6 @@ import torch
 
 from .. import _native as nat
 from .acoustic_kernels import TIMELINE, tile_launches
-from .elastic_kernels import TILE_STEPS
 
 NCOEF = 8
 
@@ -75,7 +74,7 @@ def run_backward(geom, coef: torch.Tensor, src: torch.Tensor, pml_x: Optional[to
                 fa.trace_totals = 1
                 fa.work[0], fa.work[1] = rw[0].data_ptr(), rw[1].data_ptr()
             TIMELINE.call("recompute", "el_fwd_tile" if totals else geom.kernel_names[0],
-                          tile_launches(t0, n, 0, TILE_STEPS) if totals else n, dev, lambda: nat.check(
+                          tile_launches(t0, n, 0, geom.tile_steps) if totals else n, dev, lambda: nat.check(
                 lib.adfwi_elastic_forward(ctypes.byref(d), ctypes.byref(fa), stream),
                 "adfwi_elastic_forward (recompute)"), steps=n)
         if totals and seg - 1 not in traces:   # (a resident segment's last totals are there already)
@@ -95,7 +94,7 @@ def run_backward(geom, coef: torch.Tensor, src: torch.Tensor, pml_x: Optional[to
         aa.grad_coef = gacc.data_ptr()
         aa.grad_src = gsrc.data_ptr()
         TIMELINE.call("adjoint", "el_adj_tile" if totals else geom.kernel_names[1],
-                      tile_launches(0, n, 0, TILE_STEPS) if totals else n, dev, lambda: nat.check(
+                      tile_launches(0, n, 0, geom.tile_steps) if totals else n, dev, lambda: nat.check(
             adjoint(ctypes.byref(d), ctypes.byref(aa), stream), "adfwi_elastic_adjoint"), steps=n)
         cur = lam[0] if aa.lam_out == lam[0].data_ptr() else lam[1]
         traces.pop(seg, None)              # done; segment seg + 1, which read its last state, too

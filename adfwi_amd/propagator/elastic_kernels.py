@@ -21,7 +21,6 @@ from .acoustic_kernels import (PITCH_ALIGN, TIMELINE, ResidentSet, checkpoint_in
 
 NAMES = ("txx", "tzz", "txz", "vx", "vz")
 NFIELD = 10
-TILE_STEPS = 2    # steps per launch of the tile kernels
 
 
 def DiffCoef(order: int, grid_scheme: str) -> torch.Tensor:
@@ -114,14 +113,20 @@ class ElasticGeometry:
 
     @property
     def tiled(self) -> bool:
-        """Whether the forward runs on the tile kernels (two steps per launch; a trace then holds
-        the five totals of a step instead of its ten splits): the 4th-order PML scheme without
-        C15 / C35, library tiling, a receiver map if there are receivers, state sets and
-        coefficients under 2 GiB."""
+        """Whether the tile kernels run (tile_steps per launch; a trace then holds the five totals of
+        a step instead of its ten splits): the PML scheme without C15 / C35, library tiling, a
+        receiver map if there are receivers, state sets and coefficients under 2 GiB, at 6th to
+        10th order no more than three rounds of tiles (el_tile_ok's rule)."""
         plane = 4 * self.Z * self.pitch
-        return (not self.damping and self.nn == 2 and not self.aniso and not self.shots_per_wave and not self.tile_z
+        tiles64 = -(-(self.X - 2 * self.nn) // 52) * -(-(self.Z - 2 * self.nn) // 52) * self.S
+        return (not self.damping and (self.nn == 2 or tiles64 <= 768) and not self.aniso and not self.shots_per_wave and not self.tile_z
                 and (self.R == 0 or self.rcv_map is not None) and self.nfield * self.S * plane < 1 << 31
                 and 8 * plane < 1 << 31)
+
+    @property
+    def tile_steps(self) -> int:
+        """Steps per launch of the tile kernels (at most)."""
+        return 2 if self.nn == 2 else 1
 
     def trace_fields(self, totals: bool) -> int:
         return 5 if totals else self.nfield
@@ -312,7 +317,7 @@ def run_forward(geom: ElasticGeometry, coef, pml_x, pml_z, src, scalars, *, reco
         if rec is not None:
             for i in range(5):
                 a.rec[i] = rec[i].data_ptr()
-        launches = tile_launches(t0, a.nsteps, int(a.ckpt_every), TILE_STEPS) if totals else a.nsteps
+        launches = tile_launches(t0, a.nsteps, int(a.ckpt_every), geom.tile_steps) if totals else a.nsteps
         TIMELINE.call("forward" if t0 < head else "forward+trace", "el_fwd_tile" if totals else geom.kernel_names[0],
                       launches, dev,
                       lambda: nat.check(lib.adfwi_elastic_forward(ctypes.byref(d), ctypes.byref(a), stream),

@@ -236,9 +236,10 @@ typedef struct adfwi_elastic_fwd_args {
   int32_t t0, nsteps;
   int32_t trace_totals;    /* 1: `trace` receives the five totals after every step (txx, tzz, txz, vx, vz
                               as split sums, [nsteps][5][S][Z][pitch]) and the states go through
-                              work[]; only where adfwi_elastic_forward can run its tile kernels: 4th-order
-                              PML, aniso 0, shots_per_wave and tile_z 0, rcv_map given when records are
-                              taken, state sets under 2 GiB.  0: full states, as described at trace */
+                              work[]; only where adfwi_elastic_forward runs its tile kernels: PML, aniso 0,
+                              shots_per_wave and tile_z 0, rcv_map given when records are taken, state
+                              sets under 2 GiB, with nn > 2 at most 768 tiles of 52 x 52 window points
+                              over the shots.  0: full states, as described at trace */
   float *rec[5];           /* txx, tzz, txz, vx, vz records [S][nt][R], or all NULL */
   float *trace;            /* [nsteps][10][S][Z][pitch] or NULL: the state after every step of the
                               call is written to its slot (work[] unused; ckpt must be NULL) */
