@@ -2303,7 +2303,7 @@ struct ElAdjTile { int rows, spg, groups; };
 ElAdjTile el_adj_tile_shape(const adfwi_elastic_desc *d) {
   const int nn = d->nn == 0 ? 2 : d->nn;
   auto tiles = [&](int rows) {
-    const int oz = rows - 12, ox = 52;   // stored rows and columns
+    const int oz = rows - 12, ox = d->damping ? 48 : 52;   // stored rows and columns
     return (long long)((d->nx - 2 * nn + ox - 1) / ox) * ((d->nz - 2 * nn + oz - 1) / oz);
   };
   constexpr long long CUS = 256;
@@ -2383,7 +2383,7 @@ int el_layout(const adfwi_elastic_desc *d, adfwi_layout *L) {
   L->state_floats = nf * L->field_floats;
   // gradient planes: a set per group of the adjoint that may run (step kernels or tiles)
   int sets = L->ngroups;
-  if (!d->damping && !d->aniso && d->shots_per_wave == 0 && d->tile_z == 0)
+  if (!d->aniso && d->shots_per_wave == 0 && d->tile_z == 0)
     sets = max(sets, el_adj_tile_shape(d).groups);
   L->accum_floats = (int64_t)sets * NCOEF * d->nz * d->pitch;
   return ADFWI_OK;
@@ -2401,12 +2401,12 @@ ElDev el_dev(const adfwi_elastic_desc *d, const adfwi_layout &L) {
   v.field = (long long)d->nshots * v.plane;
   v.coef = d->coef; v.pml_x = d->pml_x; v.pml_z = d->pml_z; v.src = d->src; v.src_m = d->src_m;
   v.src_fz = d->src_fz;
-  v.damp = d->damp;
+  v.damp = d->damping ? d->damp : nullptr;
   v.src_z = d->src_z; v.src_x = d->src_x; v.rcv_z = d->rcv_z; v.rcv_x = d->rcv_x;
   return v;
 }
 
-// ---- tiles (elastic_tile.hpp): the PML scheme without C15 / C35, where the caller left the layout
+// ---- tiles (elastic_tile.hpp): no C15 / C35, where the caller left the layout
 // to the library, records (if any) go through the receiver map, and a state set stays under the
 // 2 GiB that dropped buffer accesses need.  Two steps per launch at 4th order.  With three-term
 // differences it is one, the halo's price is not halved, and what the tiles gain is that no lane
@@ -2415,10 +2415,14 @@ ElDev el_dev(const adfwi_elastic_desc *d, const adfwi_layout &L) {
 // 17; 214 x 393, 8 shots (256 tiles) 25 -> 18 / 29 -> 20 / 46 -> 37; 24 shots (768) 49 -> 50 / 63 -> 55 /
 // 111 -> 78; 32 shots 59 -> 66 / 78 -> 81 / 150 -> 113; 243 x 680, 32 shots 151 -> 158 / 152 -> 191 /
 // 268 -> 224.
-constexpr long long EL3_TILES = 768;
+// The damping scheme's five fields: 122 x 240, 1 shot 11 -> 4 / 11 -> 4 / 25 -> 11; 182 x 361, 6 shots
+// 17 -> 5.5 / 17 -> 6 / 30 -> 13; 242 x 680, 32 shots 62 -> 46 / 78 -> 67 / 163 -> 125; 362 x 1040, 48 shots
+// 297 -> 165 / 297 -> 216 / 442 -> 365; with three terms, 214 x 393, 8 shots 22 -> 17 / 23 -> 18 / 40 ->
+// 30, 24 shots 37 -> 39 / 39 -> 41 / 79 -> 80: up to one and a half rounds.
+constexpr long long EL3_TILES = 768, EL3_TILES_DAMPED = 384;
 bool el_tile_ok(const adfwi_elastic_desc *d, const ElDev &v, const adfwi_layout &L, bool recs) {
   const long long tiles64 = (long long)((v.X - 2 * v.nn + 51) / 52) * ((v.Z - 2 * v.nn + 51) / 52) * v.S;
-  return !d->damping && !d->aniso && d->shots_per_wave == 0 && d->tile_z == 0 && (v.nn == 2 || tiles64 <= EL3_TILES) &&
+  return !d->aniso && d->shots_per_wave == 0 && d->tile_z == 0 && (v.nn == 2 || tiles64 <= (d->damping ? EL3_TILES_DAMPED : EL3_TILES)) &&
          (!recs || d->rcv_map) && L.state_floats * 4 < ((int64_t)1 << 31) &&
          (int64_t)NCOEF * d->nz * d->pitch * 4 < ((int64_t)1 << 31);
 }
@@ -2426,7 +2430,24 @@ bool el_tile_ok(const adfwi_elastic_desc *d, const ElDev &v, const adfwi_layout 
 template <int NW>
 tile::Grid el_tile_grid(const ElDev &v) {
   constexpr int oz = tile::out_rows(4 * NW);
-  return {(v.X - 2 * v.nn + tile::OX - 1) / tile::OX, (v.Z - 2 * v.nn + oz - 1) / oz};
+  const int ox = v.damp ? tile::OX5 : tile::OX;
+  return {(v.X - 2 * v.nn + ox - 1) / ox, (v.Z - 2 * v.nn + oz - 1) / oz};
+}
+
+template <int NW>
+void launch_abl_fwd_tile_c(const ElDev &v, hipStream_t st, const tile::AblFwdIO &io) {
+  const tile::Grid g = el_tile_grid<NW>(v);
+  const dim3 grid((unsigned)(g.ntx * g.ntz * v.S)), block(NW * WAVE);
+  if (v.nn == 2) hipLaunchKernelGGL((tile::abl_fwd_tile<2, 4, NW>), grid, block, 0, st, v, g, io);
+  else hipLaunchKernelGGL((tile::abl_fwd_tile<3, 4, NW>), grid, block, 0, st, v, g, io);
+}
+
+template <int NW>
+void launch_abl_adj_tile_c(const ElDev &v, hipStream_t st, const tile::AdjIO &io, int groups) {
+  const tile::Grid g = el_tile_grid<NW>(v);
+  const dim3 grid((unsigned)(g.ntx * g.ntz * groups)), block(NW * WAVE);
+  if (v.nn == 2) hipLaunchKernelGGL((tile::abl_adj_tile<2, 4, NW>), grid, block, 0, st, v, g, io);
+  else hipLaunchKernelGGL((tile::abl_adj_tile<3, 4, NW>), grid, block, 0, st, v, g, io);
 }
 
 template <int NW>
@@ -2446,13 +2467,25 @@ void launch_el_fwd_tile_c(const ElDev &v, hipStream_t st, const tile::FwdIO &io)
 // 9.7; 242 x 680, 32 shots 80 / 119 / 106; 362 x 1040, 48 shots 271 / 390 / 336.  With three-term
 // differences a launch is one step and the smaller halo counts for more: 64 rows then (214 x 393,
 // 16 shots 37 / 40 / 34; 24 shots 52 / 62 / 50).
+int el_fwd_tile_waves(const ElDev &v) {
+  auto fits = [&](const tile::Grid &g) { return (long long)g.ntx * g.ntz * v.S <= 256; };
+  if (fits(el_tile_grid<8>(v))) return 8;
+  if (fits(el_tile_grid<12>(v))) return 12;
+  return fits(el_tile_grid<16>(v)) || (v.nn > 2 && !v.damp) ? 16 : 8;
+}
+
 void launch_el_fwd_tile(const ElDev &v, hipStream_t st, const tile::FwdIO &io) {
-  auto count = [&](const tile::Grid &g) { return (long long)g.ntx * g.ntz * v.S; };
-  constexpr long long CUS = 256;
-  if (count(el_tile_grid<8>(v)) <= CUS) launch_el_fwd_tile_c<8>(v, st, io);
-  else if (count(el_tile_grid<12>(v)) <= CUS) launch_el_fwd_tile_c<12>(v, st, io);
-  else if (v.nn > 2 || count(el_tile_grid<16>(v)) <= CUS) launch_el_fwd_tile_c<16>(v, st, io);
-  else launch_el_fwd_tile_c<8>(v, st, io);
+  const int nw = el_fwd_tile_waves(v);
+  if (nw == 8) launch_el_fwd_tile_c<8>(v, st, io);
+  else if (nw == 12) launch_el_fwd_tile_c<12>(v, st, io);
+  else launch_el_fwd_tile_c<16>(v, st, io);
+}
+
+void launch_abl_fwd_tile(const ElDev &v, hipStream_t st, const tile::AblFwdIO &io) {
+  const int nw = el_fwd_tile_waves(v);
+  if (nw == 8) launch_abl_fwd_tile_c<8>(v, st, io);
+  else if (nw == 12) launch_abl_fwd_tile_c<12>(v, st, io);
+  else launch_abl_fwd_tile_c<16>(v, st, io);
 }
 
 template <int NW>
@@ -2464,8 +2497,10 @@ void launch_el_adj_tile_c(const ElDev &v, hipStream_t st, const tile::AdjIO &io,
 }
 
 void launch_el_adj_tile(const ElDev &v, hipStream_t st, const tile::AdjIO &io, const ElAdjTile &sh) {
-  static_assert(tile::OX == 52 && tile::out_rows(32) == 32 - 12, "el_adj_tile_shape counts these");
-  if (sh.rows == 32) launch_el_adj_tile_c<8>(v, st, io, sh.groups);
+  static_assert(tile::OX == 52 && tile::OX5 == 48 && tile::out_rows(32) == 32 - 12, "el_adj_tile_shape counts these");
+  if (v.damp && sh.rows == 32) launch_abl_adj_tile_c<8>(v, st, io, sh.groups);
+  else if (v.damp) launch_abl_adj_tile_c<12>(v, st, io, sh.groups);
+  else if (sh.rows == 32) launch_el_adj_tile_c<8>(v, st, io, sh.groups);
   else launch_el_adj_tile_c<12>(v, st, io, sh.groups);
 }
 
@@ -2511,9 +2546,31 @@ int adfwi_elastic_forward(const adfwi_elastic_desc *d, adfwi_elastic_fwd_args *a
     rk.map = d->rcv_map;
     for (int q = 0; q < 5; ++q) rk.r[q] = a->rec[q];
   }
-  ADFWI_CHECK_ARG(!a->trace_totals || (a->trace && tiles),
+  ADFWI_CHECK_ARG(!a->trace_totals || (a->trace && tiles && !d->damping),
                   "a trace of totals needs a trace buffer and the tile kernels (PML without C15 / C35, "
                   "library tiling, a receiver map for records, state sets under 2 GiB)");
+  if (tiles && d->damping) {
+    for (int k = 0; k < a->nsteps;) {
+      const int t = a->t0 + k;
+      int n = min(tile::steps_of(v.nn), a->nsteps - k);
+      if (a->ckpt) n = min(n, a->ckpt_every - t % a->ckpt_every);   // up to the next checkpoint
+      tile::AblFwdIO io{};
+      io.in = cur; io.t = t; io.n = n; io.rec = rk;
+      if (a->trace) {
+        for (int j = 0; j < n; ++j) io.out[j] = a->trace + (long long)(k + j) * L.state_floats;
+      } else if (a->ckpt && (t + n) % a->ckpt_every == 0 && t + n < d->nt) {
+        io.out[n - 1] = a->ckpt + (long long)((t + n) / a->ckpt_every - 1) * L.state_floats;
+      } else {
+        io.out[n - 1] = (cur == a->work[0]) ? a->work[1] : a->work[0];
+      }
+      launch_abl_fwd_tile(v, st, io);
+      if ((rc = adfwi::check_launch("abl_fwd_tile"))) return rc;
+      cur = io.out[n - 1];
+      k += n;
+    }
+    a->state_out = cur;
+    return ADFWI_OK;
+  }
   if (tiles && (!a->trace || a->trace_totals)) {
     for (int k = 0; k < a->nsteps;) {
       const int t = a->t0 + k;
@@ -2604,7 +2661,8 @@ static int elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *
   const bool recs = a->grad_rec[0] || a->grad_rec[1] || a->grad_rec[2] || a->grad_rec[3] || a->grad_rec[4];
   if (recs && d->nrec > 0) ADFWI_CHECK_ARG(d->rcv_z && d->rcv_x, "null receiver table pointer");
   ElDev v = el_dev(d, L);
-  ADFWI_CHECK_ARG(!totals || el_tile_ok(d, v, L, recs && d->nrec > 0),
+  const bool tiles = (totals || d->damping) && el_tile_ok(d, v, L, recs && d->nrec > 0);
+  ADFWI_CHECK_ARG(!totals || (tiles && !d->damping),
                   "a trace of totals needs the tile kernels (PML without C15 / C35, library tiling, a "
                   "receiver map for record adjoints, state sets under 2 GiB)");
   // the free-surface transposes need rows 0..3 inside the first strip (every strip height here
@@ -2642,14 +2700,14 @@ static int elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *
   // the 4th-order PML adjoint step adds the record adjoints itself when the receiver map is given
   const bool fused = recs && ng > 0 && d->rcv_map && !d->damping && v.nn == 2;
   ElInj ij{};
-  if (fused || (totals && recs && ng > 0)) {
+  if (fused || (tiles && recs && ng > 0)) {
     ij.map = d->rcv_map;
     for (int q = 0; q < 5; ++q) ij.g[q] = a->grad_rec[q];
   }
   float *cur = a->lam_in;
-  if (totals) {
+  if (tiles) {
     const ElAdjTile sh = el_adj_tile_shape(d);
-    const long long slot = NFIELD5 * L.field_floats;
+    const long long slot = NFIELD5 * L.field_floats;   // totals, or the damping scheme's state
     for (int i = a->nsteps - 1; i >= 0;) {   // two steps per launch, the last launch the odd one
       tile::AdjIO io;
       io.t = t_lo + i;
@@ -2666,7 +2724,7 @@ static int elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *
       io.gsrc = a->grad_src;
       io.inj = ij;
       launch_el_adj_tile(v, st, io, sh);
-      if ((rc = adfwi::check_launch("el_adj_tile"))) return rc;
+      if ((rc = adfwi::check_launch(d->damping ? "abl_adj_tile" : "el_adj_tile"))) return rc;
       cur = io.lout;
       i -= io.n;
     }

@@ -654,4 +654,416 @@ __global__ __launch_bounds__(NW *WAVE, NW / 4) void el_adj_tile(ElDev d, Grid g,
   }
 }
 
+// ---- the damping scheme (el_abl_fwd and el3_abl_fwd state a step): five fields, 40 B per point and
+// step in the state alone at one step per launch, 20 B at two; records and record adjoints, which
+// were launches of their own, go with the step.  182 x 361, 6 shots, us per step: forward 12.5 + 4.2
+// for the records -> 5.5, adjoint 25 + 4.6 -> 12.7.  The free-surface rows nn-2 and nn-1 are state and
+// stored by the first tiles.  Those rows reach one column further
+// per step (forward to the right, adjoint to the left), so 8 columns on a side are halo.
+constexpr int HX5 = 8;
+constexpr int OX5 = WAVE - 2 * HX5;
+
+struct AblFwdIO {
+  const float *in;
+  float *out[TK];        // state after each step, or NULL
+  int t, n;
+  ElRec rec;             // rec.map NULL: no records
+};
+
+template <int ORD, int NR, int NW>
+__global__ __launch_bounds__(NW *WAVE, 4) void abl_fwd_tile(ElDev d, Grid g, AblFwdIO io) {
+  static_assert(NR == 4 && H == 6, "rows nn-2 .. nn+1, which the free surface ties together, are wavefront 1 of the first tiles");
+  using Up = Rows<ORD, ORD - 1, NR>;
+  using Dn = Rows<ORD - 1, ORD, NR>;
+  constexpr int Q = 2 * ORD - 1;
+  const int nn = ORD == 2 ? 2 : d.nn;
+  constexpr int OZ = out_rows(NR * NW);
+  constexpr int QN = 2 * (2 * ORD - 1);
+  __shared__ float sv[NW + 2][QN][WAVE], ss[NW + 2][QN][WAVE];
+  int tx, tzi, s;
+  place(g, tx, tzi, s);
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+  if (wv == 0) {
+#pragma unroll
+    for (int q = 0; q < QN; ++q) sv[0][q][lane] = sv[NW + 1][q][lane] = ss[0][q][lane] = ss[NW + 1][q][lane] = 0.f;
+  }
+  const int x0 = nn + tx * OX5, z0 = nn + tzi * OZ;
+  const int c = x0 - HX5 + lane, zt = z0 - H + wv * NR;
+  const int zw1 = d.Z - nn - 1, xw1 = d.X - nn - 1;
+  const unsigned rowb = 4u * (unsigned)d.pitch, planeb = 4u * (unsigned)d.plane, fieldb = 4u * (unsigned)d.field;
+  const bool own = c >= x0 && c < min(x0 + OX5, xw1 + 1);
+  auto bits = [&](int lo, int hi) -> unsigned {   // rows lo .. hi-1 of this wavefront
+    const int a = min(max(lo - zt, 0), NR), b = min(max(hi - zt, 0), NR);
+    return b > a ? ((1u << b) - 1u) & ~((1u << a) - 1u) : 0u;
+  };
+  const unsigned ownbits = bits(z0, min(z0 + OZ, zw1 + 1));
+  const bool fsw = d.fsurf && tzi == 0 && wv == 1;   // this wavefront's rows are nn-2 .. nn+1
+  unsigned vi[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r)
+    vi[r] = c >= 0 && c < d.X && zt + r >= 0 && zt + r < d.Z ? (unsigned)(zt + r) * rowb + 4u * (unsigned)c : DROP;
+  auto vo = [&](int r) -> unsigned { return own && (((ownbits | (fsw ? 3u : 0u)) >> r) & 1u) ? vi[r] : DROP; };
+  auto in_win = [&](int x) -> int { int m = x >= nn && x <= xw1 ? -1 : 0; asm volatile("" : "+v"(m)); return m; };
+  int mfs = __builtin_amdgcn_readfirstlane(fsw ? -1 : 0);
+  asm volatile("" : "+s"(mfs));
+  const int mcw = in_win(c), mj1 = in_win(c + 1), mfc = mfs & mcw;
+  const Fd<ORD> D{d.c0, d.c1, ORD == 2 ? 0.f : d.c2};
+  const double rdx = 1.0 / (double)d.dx, rdz = 1.0 / (double)d.dz;
+
+  float f[NFIELD5][NR], C[4][NR], bx[NR], bz[NR], dm[NR];
+  {
+    const rsrc_t rIn = rsrc(io.in + (long long)s * d.plane, (NFIELD5 - 1) * fieldb + planeb);
+    const rsrc_t rC = rsrc(d.coef, (unsigned)NCOEF * planeb), rD = rsrc(d.damp, planeb);
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+#pragma unroll
+      for (int q = 0; q < NFIELD5; ++q) f[q][r] = bld(rIn, vi[r], (unsigned)q * fieldb);
+    }
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const unsigned v = mcw && zt + r >= nn && zt + r <= zw1 ? vi[r] : DROP;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) C[q][r] = bld(rC, v, (unsigned)q * planeb);
+      bx[r] = bld(rC, v, BX * planeb);
+      bz[r] = bld(rC, v, BZ * planeb);
+      dm[r] = bld(rD, vi[r], 0u);
+    }
+  }
+  const int zs = scalar_ld(d.src_z + s), xs = scalar_ld(d.src_x + s);
+  const bool src_here = zs >= zt && zs < zt + NR;
+  unsigned rbits = 0;
+  if (io.rec.map) {
+    const bool mine = lane < NR && ((ownbits >> (lane & 31)) & 1u);
+    rbits = (unsigned)__ballot(mine && io.rec.map[mine ? zt + lane : 0] > 0);
+  }
+
+#pragma unroll 1
+  for (int i = 0; i < io.n; ++i) {
+    const float wsrc = src_here ? scalar_ld(d.src + (long long)s * d.nt + io.t + i) : 0.f;
+    auto &vx = f[VX], &vz = f[VZ], &xx = f[TXX], &zz = f[TZZ], &xz = f[TXZ];
+    Dn::put(sv, wv, 0, lane, vx);
+    Up::put(sv, wv, Q, lane, vz);
+    lds_barrier();
+    {
+      const Dn VXr(sv, wv, 0, lane, vx);
+      const Up VZr(sv, wv, Q, lane, vz);
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        __builtin_amdgcn_sched_barrier(0);
+        const float dxb_vx = D.dxb(vx[r]), dzb_vz = D.dzb(VZr, r);
+        const float dxf_vz = D.dxf(vz[r]), dzf_vx = D.dzf(VXr, r);
+        xx[r] = xx[r] + d.dt * (quot(C[0][r] * dxb_vx, rdx) + quot(C[1][r] * dzb_vz, rdz));
+        zz[r] = zz[r] + d.dt * (quot(C[1][r] * dxb_vx, rdx) + quot(C[2][r] * dzb_vz, rdz));
+        xz[r] = xz[r] + d.dt * (quot(C[3][r] * dxf_vz, rdx) + quot(C[3][r] * dzf_vx, rdz));
+        pin(xx[r], zz[r]);
+        asm volatile("" : "+v"(xz[r]));
+      }
+    }
+    if (src_here) {
+      const float mxx = d.src_m[3 * s], mzz = d.src_m[3 * s + 1], mxz = d.src_m[3 * s + 2];
+#pragma unroll
+      for (int r = 0; r < NR; ++r)
+        if (zs == zt + r && c == xs) {
+          xx[r] = xx[r] + mxx * wsrc;
+          zz[r] = zz[r] + mzz * wsrc;
+          xz[r] = xz[r] + mxz * wsrc;
+        }
+    }
+    zz[2] = keep(~mfs, zz[2]);   // stress free surface
+    zz[1] = pick(mfc, -zz[3], zz[1]);
+    xz[1] = pick(mfc, -xz[2], xz[1]);
+    xz[0] = pick(mfc, -xz[3], xz[0]);
+    Dn::put(ss, wv, 0, lane, zz);
+    Up::put(ss, wv, Q, lane, xz);
+    lds_barrier();
+    {
+      const Dn ZZr(ss, wv, 0, lane, zz);
+      const Up XZr(ss, wv, Q, lane, xz);
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        __builtin_amdgcn_sched_barrier(0);
+        const float dxf_txx = D.dxf(xx[r]), dzb_txz = D.dzb(XZr, r);
+        const float dxb_txz = D.dxb(xz[r]), dzf_tzz = D.dzf(ZZr, r);
+        vx[r] = vx[r] + (d.dt * bx[r]) * (quot(dxf_txx, rdx) + quot(dzb_txz, rdz));
+        vz[r] = vz[r] + (d.dt * bz[r]) * (quot(dxb_txz, rdx) + quot(dzf_tzz, rdz));
+        pin(vx[r], vz[r]);
+      }
+    }
+    if (src_here && d.src_fz) {   // vertical force
+      const float a = scalar_ld(d.src_fz + s) * wsrc;
+#pragma unroll
+      for (int r = 0; r < NR; ++r)
+        if (zs == zt + r && c == xs) vz[r] = vz[r] + a;
+    }
+    {   // velocity free surface from the new rows, then the taper
+      const float vzn = from_right(vz[2]);
+      const float vz1m_n = keep(mj1, vzn), vz1m = keep(mcw, vz[2]);
+      const float nx1 = (((vz1m_n - vz1m) + vzn) - vz[2]) + vx[3];
+      vx[1] = pick(mfc, nx1, vx[1]);
+      vz[1] = pick(mfc, vz1m, vz[1]);
+      vz[0] = pick(mfc, vz1m, vz[0]);
+    }
+#pragma unroll
+    for (int r = 0; r < NR; ++r) { vx[r] = vx[r] * dm[r]; vz[r] = vz[r] * dm[r]; }
+    if (rbits) {
+      const long long ro = ((long long)s * d.nt + io.t + i) * d.nrec;
+      const unsigned rbytes = 4u * (unsigned)d.nrec;
+#pragma unroll
+      for (int r = 0; r < NR; ++r)
+        if ((rbits >> r) & 1u) {
+          const int m = __builtin_bit_cast(int, bld(rsrc(io.rec.map + d.Z, planeb), vi[r], 0u));
+          const unsigned v = own && m >= 0 ? 4u * (unsigned)m : DROP;
+#pragma unroll
+          for (int q = 0; q < NFIELD5; ++q) bst(f[q][r], rsrc(io.rec.r[q] + ro, rbytes), v, 0u);
+        }
+    }
+    float *o = io.out[i];
+    const rsrc_t rOut = rsrc(o ? o + (long long)s * d.plane : nullptr, o ? (NFIELD5 - 1) * fieldb + planeb : 0u);
+    if (o) {
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        const unsigned v = vo(r);
+#pragma unroll
+        for (int q = 0; q < NFIELD5; ++q) bst(f[q][r], rOut, v, (unsigned)q * fieldb);
+      }
+    }
+  }
+}
+
+// Its adjoint (el_abl_adj and el3_abl_adj list the transposes), grouped as el_adj_tile.  Stress
+// adjoints outside the window take values that nothing reads or stores; the velocity adjoints of
+// the free-surface rows are state.
+template <int ORD, int NR, int NW>
+__global__ __launch_bounds__(NW *WAVE, NW / 4) void abl_adj_tile(ElDev d, Grid g, AdjIO io) {
+  static_assert(NR == 4 && H == 6, "rows nn-2 .. nn+1, which the free surface ties together, are wavefront 1 of the first tiles");
+  using Up = Rows<ORD, ORD - 1, NR>;
+  using Dn = Rows<ORD - 1, ORD, NR>;
+  constexpr int Q = 2 * ORD - 1;
+  const int nn = ORD == 2 ? 2 : d.nn;
+  constexpr int OZ = out_rows(NR * NW);
+  __shared__ float sv[NW + 2][6 * (2 * ORD - 1)][WAVE], ss[NW + 2][2 * (2 * ORD - 1)][WAVE];
+  int tx, tzi, grp;
+  place(g, tx, tzi, grp);
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+  if (wv == 0) {
+#pragma unroll
+    for (int q = 0; q < 6 * Q; ++q) sv[0][q][lane] = sv[NW + 1][q][lane] = 0.f;
+#pragma unroll
+    for (int q = 0; q < 2 * Q; ++q) ss[0][q][lane] = ss[NW + 1][q][lane] = 0.f;
+  }
+  const int x0 = nn + tx * OX5, z0 = nn + tzi * OZ;
+  const int c = x0 - HX5 + lane, zt = z0 - H + wv * NR;
+  const int zw1 = d.Z - nn - 1, xw1 = d.X - nn - 1;
+  const unsigned rowb = 4u * (unsigned)d.pitch, planeb = 4u * (unsigned)d.plane, fieldb = 4u * (unsigned)d.field;
+  const bool own = c >= x0 && c < min(x0 + OX5, xw1 + 1);
+  auto bits = [&](int lo, int hi) -> unsigned {   // rows lo .. hi-1 of this wavefront
+    const int a = min(max(lo - zt, 0), NR), b = min(max(hi - zt, 0), NR);
+    return b > a ? ((1u << b) - 1u) & ~((1u << a) - 1u) : 0u;
+  };
+  const unsigned ownbits = bits(z0, min(z0 + OZ, zw1 + 1));
+  const bool fsw = d.fsurf && tzi == 0 && wv == 1;   // this wavefront's rows are nn-2 .. nn+1
+  unsigned vi[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r)
+    vi[r] = c >= 0 && c < d.X && zt + r >= 0 && zt + r < d.Z ? (unsigned)(zt + r) * rowb + 4u * (unsigned)c : DROP;
+  auto vo = [&](int r) -> unsigned { return own && ((ownbits >> r) & 1u) ? vi[r] : DROP; };
+  auto in_win = [&](int x) -> int { int m = x >= nn && x <= xw1 ? -1 : 0; asm volatile("" : "+v"(m)); return m; };
+  int mfs = __builtin_amdgcn_readfirstlane(fsw ? -1 : 0);
+  asm volatile("" : "+s"(mfs));
+  const int mcw = in_win(c), mm1 = in_win(c - 1), mfc = mfs & mcw;
+  const Fd<ORD> D{d.c0, d.c1, ORD == 2 ? 0.f : d.c2};
+  const double rdx = 1.0 / (double)d.dx, rdz = 1.0 / (double)d.dz;
+  const float dtdx = d.dt_dx, dtdz = d.dt_dz;
+
+  float C[4][NR], bx[NR], bz[NR], dm[NR];
+  {
+    const rsrc_t rC = rsrc(d.coef, (unsigned)NCOEF * planeb), rD = rsrc(d.damp, planeb);
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const unsigned v = mcw && zt + r >= nn && zt + r <= zw1 ? vi[r] : DROP;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) C[q][r] = bld(rC, v, (unsigned)q * planeb);
+      bx[r] = bld(rC, v, BX * planeb);
+      bz[r] = bld(rC, v, BZ * planeb);
+      dm[r] = bld(rD, vi[r], 0u);
+    }
+  }
+  unsigned rbits = 0;   // rows with receivers: of the halo, too
+  if (io.inj.map) {
+    const bool mine = lane < NR && zt + lane >= nn && zt + lane <= zw1;
+    rbits = (unsigned)__ballot(mine && io.inj.map[mine ? zt + lane : 0] > 0);
+  }
+  float G[6][NR];
+#pragma unroll
+  for (int q = 0; q < 6; ++q)
+#pragma unroll
+    for (int r = 0; r < NR; ++r) G[q][r] = 0.f;
+
+  const int s_end = min((grp + 1) * io.spg, d.S);
+#pragma unroll 1
+  for (int s = grp * io.spg; s < s_end; ++s) {
+    const int zs = scalar_ld(d.src_z + s), xs = scalar_ld(d.src_x + s);
+    const bool src_here = io.gsrc && zs >= zt && zs < zt + NR && ((ownbits >> (zs - zt)) & 1u) && xs >= x0 && xs < x0 + OX5;
+    float f[NFIELD5][NR];
+    {
+      const rsrc_t rIn = rsrc(io.lin + (long long)s * d.plane, (NFIELD5 - 1) * fieldb + planeb);
+#pragma unroll
+      for (int r = 0; r < NR; ++r)
+#pragma unroll
+        for (int q = 0; q < NFIELD5; ++q) f[q][r] = bld(rIn, vi[r], (unsigned)q * fieldb);
+    }
+    auto &lx = f[VX], &lz = f[VZ];
+#pragma unroll 1
+    for (int i = 0; i < io.n; ++i) {
+      const int t = io.t - i;
+      float vx[NR], vz[NR], xx[NR], zz[NR], xz[NR];
+      {
+        const rsrc_t rV = rsrc(io.fv[i] + (long long)s * d.plane, (NFIELD5 - 1) * fieldb + planeb);
+        const rsrc_t rS = rsrc(io.fs[i] + (long long)s * d.plane, (NFIELD5 - 1) * fieldb + planeb);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          vx[r] = bld(rV, vi[r], VX * fieldb);
+          vz[r] = bld(rV, vi[r], VZ * fieldb);
+        }
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          xx[r] = bld(rS, vi[r], TXX * fieldb);
+          zz[r] = bld(rS, vi[r], TZZ * fieldb);
+          xz[r] = bld(rS, vi[r], TXZ * fieldb);
+        }
+      }
+      if (rbits) {   // record adjoints of step t
+        const long long ro = ((long long)s * d.nt + t) * d.nrec;
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          if ((rbits >> r) & 1u) {
+            const int m = __builtin_bit_cast(int, bld(rsrc(io.inj.map + d.Z, planeb), vi[r], 0u));
+            const unsigned v = mcw && m >= 0 ? 4u * (unsigned)m : DROP;
+#pragma unroll
+            for (int q = 0; q < NFIELD5; ++q) {
+              const float *p = io.inj.g[q];
+              f[q][r] += bld(rsrc(p ? p + ro : nullptr, p ? 4u * (unsigned)d.nrec : 0u),
+                             q == TZZ && d.fsurf && zt + r == nn ? DROP : v, 0u);
+            }
+          }
+      }
+      // taper, then the velocity free surface transposed
+#pragma unroll
+      for (int r = 0; r < NR; ++r) { lx[r] = lx[r] * dm[r]; lz[r] = lz[r] * dm[r]; }
+      {
+        const float wz0 = lz[0], wz1 = lz[1], wx1 = lx[1];
+        const float add = ((wz1 + wz0) - 2.0f * wx1) + keep(mm1, 2.0f * from_left(wx1));
+        lz[0] = keep(~mfc, lz[0]);
+        lz[1] = keep(~mfc, lz[1]);
+        lx[1] = keep(~mfc, lx[1]);
+        lz[2] = lz[2] + keep(mfc, add);
+        lx[3] = lx[3] + keep(mfc, wx1);
+      }
+      float eb[NR], ed[NR];
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        asm volatile("" : "+v"(bx[r]), "+v"(bz[r]));   // (the products below, kept over the loops, would cost registers)
+        eb[r] = lx[r] * quot(d.dt * bx[r], rdz);
+        ed[r] = lz[r] * quot(d.dt * bz[r], rdz);
+      }
+      Dn::put(sv, wv, 0, lane, eb);
+      Up::put(sv, wv, Q, lane, ed);
+      Dn::put(sv, wv, 2 * Q, lane, vx);
+      Up::put(sv, wv, 3 * Q, lane, vz);
+      Dn::put(sv, wv, 4 * Q, lane, zz);
+      Up::put(sv, wv, 5 * Q, lane, xz);
+      lds_barrier();
+      {   // buoyancy gradients
+        const Dn ZZr(sv, wv, 4 * Q, lane, zz);
+        const Up XZr(sv, wv, 5 * Q, lane, xz);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          __builtin_amdgcn_sched_barrier(0);
+          const float dxf_txx = D.dxf(xx[r]), dzb_txz = D.dzb(XZr, r);
+          const float dxb_txz = D.dxb(xz[r]), dzf_tzz = D.dzf(ZZr, r);
+          G[4][r] += lx[r] * (d.dt * (quot(dxf_txx, rdx) + quot(dzb_txz, rdz)));
+          G[5][r] += lz[r] * (d.dt * (quot(dxb_txz, rdx) + quot(dzf_tzz, rdz)));
+          pin(G[4][r], G[5][r]);
+        }
+      }
+      float P1[NR], Q2[NR], Q3[NR], P4[NR];
+      {
+        const Dn EB(sv, wv, 0, lane, eb), VXr(sv, wv, 2 * Q, lane, vx);
+        const Up ED(sv, wv, Q, lane, ed), VZr(sv, wv, 3 * Q, lane, vz);
+        float ltxz0 = 0.f, ltxz1 = 0.f, ltzz1 = 0.f;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          __builtin_amdgcn_sched_barrier(0);
+          const float ea = lx[r] * quot(d.dt * bx[r], rdx), ec = lz[r] * quot(d.dt * bz[r], rdx);
+          const float lt_xx = D.dxfT(ea);
+          float lt_xz = D.dzbT(EB, r) + D.dxbT(ec), lt_zz = D.dzfT(ED, r);
+          // stress free surface transposed; the stored tzz of row nn is a constant
+          if (r == 0) ltxz0 = keep(mfs, lt_xz);
+          if (r == 1) { ltzz1 = keep(mfs, lt_zz); ltxz1 = keep(mfs, lt_xz); }
+          if (r == 2) lt_xz = lt_xz - ltxz1;
+          if (r == 3) { lt_zz = lt_zz - ltzz1; lt_xz = lt_xz - ltxz0; }
+          f[TXX][r] += lt_xx;
+          f[TZZ][r] += lt_zz;
+          f[TXZ][r] += lt_xz;
+          if (r == 2) f[TZZ][r] = keep(~mfs, f[TZZ][r]);
+          const float axx_x = dtdx * f[TXX][r], axx_z = dtdz * f[TXX][r];
+          const float azz_x = dtdx * f[TZZ][r], azz_z = dtdz * f[TZZ][r];
+          const float axz_x = dtdx * f[TXZ][r], axz_z = dtdz * f[TXZ][r];
+          P1[r] = C[0][r] * axx_x + C[1][r] * azz_x;
+          Q2[r] = C[1][r] * axx_z + C[2][r] * azz_z;
+          Q3[r] = C[3][r] * axz_x;
+          P4[r] = C[3][r] * axz_z;
+          const float dxb_vx = D.dxb(vx[r]), dzb_vz = D.dzb(VZr, r);
+          const float dxf_vz = D.dxf(vz[r]), dzf_vx = D.dzf(VXr, r);
+          G[0][r] += axx_x * dxb_vx;
+          G[1][r] += axx_z * dzb_vz + azz_x * dxb_vx;
+          G[2][r] += azz_z * dzb_vz;
+          G[3][r] += axz_x * dxf_vz + axz_z * dzf_vx;
+          pin(G[0][r], G[1][r]); pin(G[2][r], G[3][r]);
+          pin(P1[r], Q2[r]); pin(Q3[r], P4[r]);
+        }
+      }
+      Dn::put(ss, wv, 0, lane, Q2);
+      Up::put(ss, wv, Q, lane, P4);
+      if (src_here) {
+        const float mxx = d.src_m[3 * s], mzz = d.src_m[3 * s + 1], mxz = d.src_m[3 * s + 2];
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          if (zs == zt + r && c == xs) {
+            float gm = (mxx * f[TXX][r] + mzz * f[TZZ][r]) + mxz * f[TXZ][r];
+            if (d.src_fz) gm = gm + d.src_fz[s] * lz[r];
+            io.gsrc[(long long)s * d.nt + t] = gm;
+          }
+      }
+      lds_barrier();
+      {
+        const Dn Q2r(ss, wv, 0, lane, Q2);
+        const Up P4r(ss, wv, Q, lane, P4);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          __builtin_amdgcn_sched_barrier(0);
+          lx[r] += D.dxbT(P1[r]) + D.dzfT(P4r, r);
+          lz[r] += D.dzbT(Q2r, r) + D.dxfT(Q3[r]);
+        }
+      }
+    }
+    const rsrc_t rOut = rsrc(io.lout + (long long)s * d.plane, (NFIELD5 - 1) * fieldb + planeb);
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const unsigned v = vo(r), w = own && fsw && r < 2 ? vi[r] : v;
+#pragma unroll
+      for (int q = 0; q < NFIELD5; ++q) bst(f[q][r], rOut, q >= VX ? w : v, (unsigned)q * fieldb);
+    }
+  }
+  const rsrc_t rG = rsrc(io.gacc + (long long)grp * NCOEF * d.Z * d.pitch, (unsigned)NCOEF * planeb);
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const unsigned v = vo(r);
+#pragma unroll
+    for (int q = 0; q < 6; ++q) bst(bld(rG, v, (unsigned)q * planeb) + G[q][r], rG, v, (unsigned)q * planeb);
+  }
+}
+
 }  // namespace tile

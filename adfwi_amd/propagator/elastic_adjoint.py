@@ -25,7 +25,7 @@ def run_backward(geom, coef: torch.Tensor, src: torch.Tensor, pml_x: Optional[to
     record adjoints (txx, tzz, txz, vx, vz; None = zero).  traces: {segment: per-step states}
     kept by run_forward(resident=...); those segments are not recomputed, and each is released
     once the segment before it no longer needs its last state.  totals: whether traces hold the
-    five totals of a state instead of its fields (run_forward's; default geom.tiled).  Returns (list of 8 (Z, pitch)
+    five totals of a state instead of its fields (run_forward's; default geom.totals).  Returns (list of 8 (Z, pitch)
     gradients of the padded coefficient planes C11, C13, C33, C55, bx, bz, C15, C35 -- None
     where not needed -- and the (S, nt) wavelet gradient or None).
     """
@@ -38,7 +38,8 @@ def run_backward(geom, coef: torch.Tensor, src: torch.Tensor, pml_x: Optional[to
     first_resident = min(traces) if traces else nseg
     if first_resident > 1 and (ckpt is None or ckpt.shape[0] < first_resident - 1):
         raise RuntimeError("the forward pass kept no checkpoints for the adjoint")
-    totals = geom.tiled if totals is None else bool(totals)
+    totals = geom.totals if totals is None else bool(totals)
+    tiled = totals or (geom.damping and geom.tiled)
     lam = geom.state(2)
     trace = geom.trace(min(k, nt), totals) if len(traces) < nseg else None
     # with totals: ping-pong states of the recomputation, and the totals before a segment
@@ -73,8 +74,8 @@ def run_backward(geom, coef: torch.Tensor, src: torch.Tensor, pml_x: Optional[to
             if totals:
                 fa.trace_totals = 1
                 fa.work[0], fa.work[1] = rw[0].data_ptr(), rw[1].data_ptr()
-            TIMELINE.call("recompute", "el_fwd_tile" if totals else geom.kernel_names[0],
-                          tile_launches(t0, n, 0, geom.tile_steps) if totals else n, dev, lambda: nat.check(
+            TIMELINE.call("recompute", geom.step_kernels[0] if tiled else geom.kernel_names[0],
+                          tile_launches(t0, n, 0, geom.tile_steps) if tiled else n, dev, lambda: nat.check(
                 lib.adfwi_elastic_forward(ctypes.byref(d), ctypes.byref(fa), stream),
                 "adfwi_elastic_forward (recompute)"), steps=n)
         if totals and seg - 1 not in traces:   # (a resident segment's last totals are there already)
@@ -93,8 +94,8 @@ def run_backward(geom, coef: torch.Tensor, src: torch.Tensor, pml_x: Optional[to
             aa.grad_rec[i] = None if g[i] is None else g[i].data_ptr()
         aa.grad_coef = gacc.data_ptr()
         aa.grad_src = gsrc.data_ptr()
-        TIMELINE.call("adjoint", "el_adj_tile" if totals else geom.kernel_names[1],
-                      tile_launches(0, n, 0, geom.tile_steps) if totals else n, dev, lambda: nat.check(
+        TIMELINE.call("adjoint", geom.step_kernels[1] if tiled else geom.kernel_names[1],
+                      tile_launches(0, n, 0, geom.tile_steps) if tiled else n, dev, lambda: nat.check(
             adjoint(ctypes.byref(d), ctypes.byref(aa), stream), "adfwi_elastic_adjoint"), steps=n)
         cur = lam[0] if aa.lam_out == lam[0].data_ptr() else lam[1]
         traces.pop(seg, None)              # done; segment seg + 1, which read its last state, too

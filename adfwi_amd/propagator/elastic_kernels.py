@@ -113,15 +113,27 @@ class ElasticGeometry:
 
     @property
     def tiled(self) -> bool:
-        """Whether the tile kernels run (tile_steps per launch; a trace then holds the five totals of
-        a step instead of its ten splits): the PML scheme without C15 / C35, library tiling, a
+        """Whether the tile kernels run, tile_steps per launch: no C15 / C35, library tiling, a
         receiver map if there are receivers, state sets and coefficients under 2 GiB, at 6th to
-        10th order no more than three rounds of tiles (el_tile_ok's rule)."""
+        10th order only so many tiles (el_tile_ok's rule)."""
         plane = 4 * self.Z * self.pitch
         tiles64 = -(-(self.X - 2 * self.nn) // 52) * -(-(self.Z - 2 * self.nn) // 52) * self.S
-        return (not self.damping and (self.nn == 2 or tiles64 <= 768) and not self.aniso and not self.shots_per_wave and not self.tile_z
+        return (not self.aniso and not self.shots_per_wave and not self.tile_z
+                and (self.nn == 2 or tiles64 <= (384 if self.damping else 768))
                 and (self.R == 0 or self.rcv_map is not None) and self.nfield * self.S * plane < 1 << 31
                 and 8 * plane < 1 << 31)
+
+    @property
+    def totals(self) -> bool:
+        """Whether a trace holds the five totals of a step instead of the PML scheme's ten splits."""
+        return self.tiled and not self.damping
+
+    @property
+    def step_kernels(self):
+        """(forward, adjoint) kernels that run, as the timeline names them."""
+        if not self.tiled:
+            return self.kernel_names
+        return ("abl_fwd_tile", "abl_adj_tile") if self.damping else ("el_fwd_tile", "el_adj_tile")
 
     @property
     def tile_steps(self) -> int:
@@ -227,7 +239,7 @@ def resident_trace_segments(geom: ElasticGeometry, k: int) -> int:
         return 0
     state_bytes = int(geom.layout.state_floats) * 4
     seg_bytes = k * state_bytes
-    if getattr(geom, "tiled", False):     # five totals instead of ten splits
+    if getattr(geom, "totals", False):    # five totals instead of ten splits
         seg_bytes //= 2
     if cap is None:
         cap = resident_budget_bytes(geom.device, (nseg + 5) * state_bytes + seg_bytes) // seg_bytes
@@ -253,7 +265,7 @@ def run_forward(geom: ElasticGeometry, coef, pml_x, pml_z, src, scalars, *, reco
     """All nt steps from a zero state.  Returns dict(rec=[5 x (S, nt, R)] or None,
     energy=[5 x (Z, X)] summed over the states after the steps in energy_ends, ckpt,
     traces={segment: per-step states}, totals: whether the traces hold five totals instead of the
-    state's fields, geom.tiled).
+    state's fields, geom.totals).
 
     resident > 0 (with ckpt_every): the last `resident` checkpoint segments write the state after
     each of their steps to a trace buffer of their own, which run_backward uses instead of
@@ -261,7 +273,7 @@ def run_forward(geom: ElasticGeometry, coef, pml_x, pml_z, src, scalars, *, reco
     lib = nat.load()
     dev = geom.device
     S, nt, R = geom.S, geom.nt, geom.R
-    totals = geom.tiled
+    totals, tiled = geom.totals, geom.tiled
     work = geom.state(2)
     k = int(ckpt_every)
     nseg = -(-nt // k) if k else 1
@@ -317,8 +329,8 @@ def run_forward(geom: ElasticGeometry, coef, pml_x, pml_z, src, scalars, *, reco
         if rec is not None:
             for i in range(5):
                 a.rec[i] = rec[i].data_ptr()
-        launches = tile_launches(t0, a.nsteps, int(a.ckpt_every), geom.tile_steps) if totals else a.nsteps
-        TIMELINE.call("forward" if t0 < head else "forward+trace", "el_fwd_tile" if totals else geom.kernel_names[0],
+        launches = tile_launches(t0, a.nsteps, int(a.ckpt_every), geom.tile_steps) if tiled else a.nsteps
+        TIMELINE.call("forward" if t0 < head else "forward+trace", geom.step_kernels[0],
                       launches, dev,
                       lambda: nat.check(lib.adfwi_elastic_forward(ctypes.byref(d), ctypes.byref(a), stream),
                                         "adfwi_elastic_forward"), steps=a.nsteps)

@@ -419,9 +419,9 @@ def main():
             byts = d["steps"] * BYTES_ADJ * N * S
         elif name in ("el_fwd_step", "el_fwd_tile", "el3_fwd_step"):
             byts = d["steps"] * EL_BYTES_FWD * N * S
-        elif name in ("el_abl_fwd", "el3_abl_fwd"):
+        elif name in ("el_abl_fwd", "el3_abl_fwd", "abl_fwd_tile"):
             byts = d["steps"] * EL_BYTES_FWD / 2 * N * S
-        elif name in ("el_abl_adj", "el3_abl_adj"):
+        elif name in ("el_abl_adj", "el3_abl_adj", "abl_adj_tile"):
             byts = d["steps"] * EL_BYTES_ADJ / 2 * N * S
         else:
             byts = d["steps"] * EL_BYTES_ADJ * N * S

@@ -59,6 +59,16 @@ def test_three_term_tiles_equal_one_step_kernels(Z, X, S, fs, force, nn):
     _compare(Z, X, S, fs, force, nn)
 
 
+@pytest.mark.parametrize("Z,X,S,fs,force,nn", [c + (2,) for c in CASES if c[2] != 80] + CASES3[:5] + [
+    (24, 52, 3, True, True, 2),    # one tile of 20 x 48, filled
+    (25, 53, 3, True, True, 2),    # one past it
+    (64, 60, 140, True, False, 2),  # more tiles than compute units at every height: 32 rows
+    (66, 62, 80, True, True, 3),
+])
+def test_damping_tiles_equal_one_step_kernels(Z, X, S, fs, force, nn):
+    _compare(Z, X, S, fs, force, nn, damping=True)
+
+
 def test_three_term_tiles_end_at_three_rounds():
     from adfwi_amd.propagator import elastic_kernels as ek
     for S, tiled in ((192, True), (193, False)):   # 2 x 2 tiles of 52 x 52 each
@@ -67,7 +77,7 @@ def test_three_term_tiles_end_at_three_rounds():
         assert g.tiled == tiled
 
 
-def _compare(Z, X, S, fs, force, nn):
+def _compare(Z, X, S, fs, force, nn, damping=False):
     from adfwi_amd.propagator import elastic_adjoint as ea
     from adfwi_amd.propagator import elastic_kernels as ek
     rng = np.random.default_rng(Z * 1000 + X)
@@ -84,25 +94,32 @@ def _compare(Z, X, S, fs, force, nn):
     src_m, src_fz = rand(-1, 1, S, 3), rand(-1, 1, S) if force else None
     coef_fields = [rand(a, b, Z, X).to(DEV) for a, b in ((5, 9), (1, 3), (5, 9), (1, 3), (.3, .6), (.3, .6))]
     bcx, bcz = rand(0, 20, 1, X).expand(Z, X), rand(0, 20, Z, 1).expand(Z, X)
+    taper = rand(0.9, 1.0, Z, X).to(DEV)
     src = torch.randn((S, nt), generator=gen).to(DEV)
     scalars = (1e-2, 2e-2, 2.5e-2, 0.5, 0.4) + ((1.125, -1.0 / 24) if nn == 2 else (75.0 / 64, -25.0 / 384))
     out = []
     for tile_z in (0, 8):   # three-term: c2 = 3 / 640
         g = ek.ElasticGeometry(Z, X, nt, fs, src_z, src_x, src_m, pts[:, 0], pts[:, 1], DEV, tile_z=tile_z,
-                               shots_per_wave=int(tile_z > 0), src_fz=src_fz, nn=nn, c2=0.0 if nn == 2 else 3.0 / 640)
+                               shots_per_wave=int(tile_z > 0), src_fz=src_fz, nn=nn, c2=0.0 if nn == 2 else 3.0 / 640,
+                               damping=damping)
         assert g.tiled == (tile_z == 0)
         px, pz = (t.to(DEV) for t in ek.pml_factors(bcx, bcz, scalars[0], g.pitch))
         coef = g.pack_coef(coef_fields + [None, None])
-        out.append((g, coef, px, pz, ek.run_forward(g, coef, px, pz, src, scalars, ckpt_every=k)))
-    (g, coef, px, pz, a), b = out[0], out[1][4]
+        damp = g.pack_plane(taper) if damping else None
+        out.append((g, coef, px, pz, damp, ek.run_forward(g, coef, px, pz, src, scalars, ckpt_every=k, damp=damp)))
+    (g, coef, px, pz, damp, a), b = out[0], out[1][5]
     torch.cuda.synchronize()
     for i in range(5):
         assert torch.isfinite(b["rec"][i]).all() and b["rec"][i].abs().max() > 0
         assert torch.equal(a["rec"][i], b["rec"][i]), ("record", i, rel_l2(a["rec"][i].cpu(), b["rec"][i].cpu()))
     assert torch.equal(a["ckpt"], b["ckpt"]) and torch.equal(a["final"], b["final"])
     g_rec = [torch.randn((S, nt, len(pts)), generator=gen).to(DEV) for _ in range(5)]
-    grads = [ea.run_backward(g, coef, src, px, pz, scalars, a["ckpt"], k, g_rec, [True] * 6 + [False] * 2 + [True],
-                             totals=totals) for totals in (True, False)]
+    needs = [True] * 6 + [False] * 2 + [True]
+    if damping:   # the trace is the state's five fields with either kernel
+        grads = [ea.run_backward(x[0], coef, src, px, pz, scalars, x[5]["ckpt"], k, g_rec, needs, damp=x[4]) for x in out]
+    else:
+        grads = [ea.run_backward(g, coef, src, px, pz, scalars, a["ckpt"], k, g_rec, needs, totals=totals)
+                 for totals in (True, False)]
     torch.cuda.synchronize()
     for i in range(6):
         assert grads[1][0][i].abs().max() > 0
