@@ -69,6 +69,10 @@ __device__ __forceinline__ T scalar_ld(const T *p) {
   return *(const __attribute__((address_space(4))) T *)(unsigned long long)p;
 }
 
+// forms the value where this stands: left to itself the compiler moves a sum whose only use lies past
+// a later branch there, and holds its terms till then
+__device__ __forceinline__ void pin(float &v) { asm volatile("" : "+v"(v)); }
+
 struct Grid {
   int ntx, ntz, ngroups, spg;      // tiles along x and z, shot groups, shots per group
 };
@@ -451,7 +455,12 @@ __global__ __launch_bounds__(NW *WAVE) void ac_adj_tile(AcDev d, Grid g, AdjIO i
     return b > a ? ((1u << b) - 1u) & ~((1u << a) - 1u) : 0u;
   };
   const unsigned ownbits = bits(z0, zend), wbits = bits(z0, min(zend, d.Z - 1));
-  auto span = [&](unsigned b, int r) -> unsigned { return (b >> r) & 1u ? planeb : 0u; };
+  // an access to row r only where mask b has it: with two columns per lane through the size of the
+  // plane (as above), with one through the lane's offset, for which there are registers (one
+  // descriptor per plane instead of one per row: 3-6 % faster, but with two columns it spills)
+  auto span = [&](unsigned b, int r) -> unsigned { return CPL == 1 || ((b >> r) & 1u) ? planeb : 0u; };
+  auto vrow = [&](unsigned b, int r) -> unsigned { return CPL > 1 || ((b >> r) & 1u) ? vout : DROP; };
+  constexpr bool PIN = CPL == 1 || !FULL;   // (two columns with all records: 5 % slower pinned)
   auto off = [&](int row) -> unsigned { return (unsigned)min(max(row, 0), d.Z - 1) * rowb; };
   const int s0 = grp * g.spg, ns = min(g.spg, d.S - s0);
 
@@ -560,12 +569,6 @@ __global__ __launch_bounds__(NW *WAVE) void ac_adj_tile(AcDev d, Grid g, AdjIO i
 #pragma unroll 1
     for (int i = 0; i < io.n; ++i) {
       const long long fi = (long long)s * d.plane - (long long)i * d.field;
-      C im[NR];
-      if (io.grad_a1) {
-        const float *const img = io.img_d + fi;
-#pragma unroll
-        for (int r = 0; r < NR; ++r) im[r] = ldc<CPL>(rsrc(img, span(ownbits, r)), vout, off(zt + r));
-      }
       // pressures of rows -1 .. NR+1 after the step: one lane column leaves the registers to fetch
       // them this early
       C q0[A2 ? NR + 3 : 1];
@@ -623,14 +626,15 @@ __global__ __launch_bounds__(NW *WAVE) void ac_adj_tile(AcDev d, Grid g, AdjIO i
         sw[wv + 1][2][lane] = z;
       }
       lds_barrier();
+      C im[NR];
+      if (io.grad_a1) {
+        const float *const img = io.img_d + fi;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) im[r] = ldc<CPL>(rsrc(img, span(ownbits, r)), vrow(ownbits, r), off(zt + r));
+      }
       const C wa2 = sw[wv][1][lane], wa1 = sw[wv][2][lane], wb = sw[wv + 2][0][lane];
       {
-        float f[NR + 3][CPL];   // a2 lambda_w of rows -2 .. NR
-#pragma unroll
-        for (int r = 0; r < NR + 3; ++r)
-#pragma unroll
-          for (int q = 0; q < CPL; ++q)
-            f[r][q] = r == 0 ? wa2.v[q] : r == 1 ? wa1.v[q] : r == NR + 2 ? wb.v[q] : fw(r - 2, q);
+        auto f = [&](int r, int q) -> float { return r == 0 ? wa2.v[q] : r == 1 ? wa1.v[q] : r == NR + 2 ? wb.v[q] : fw(r - 2, q); };
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
           __builtin_amdgcn_sched_barrier(0);
@@ -651,8 +655,9 @@ __global__ __launch_bounds__(NW *WAVE) void ac_adj_tile(AcDev d, Grid g, AdjIO i
 #pragma unroll
           for (int q = 0; q < CPL; ++q) {
             const float dxt = C1 * dx1[q] + C2 * dx2[q];
-            const float dzt = C1 * (f[r + 1][q] - f[r + 2][q]) + C2 * (f[r][q] - f[r + 3][q]);
+            const float dzt = C1 * (f(r + 1, q) - f(r + 2, q)) + C2 * (f(r, q) - f(r + 3, q));
             p[r][q] = p[r][q] - (dxt + dzt);
+            if constexpr (PIN) pin(p[r][q]);
           }
         }
       }
@@ -676,7 +681,10 @@ __global__ __launch_bounds__(NW *WAVE) void ac_adj_tile(AcDev d, Grid g, AdjIO i
 #pragma unroll
         for (int r = 0; r < NR; ++r)
 #pragma unroll
-          for (int q = 0; q < CPL; ++q) ga1[r][q] -= p[r][q] * im[r].v[q];
+          for (int q = 0; q < CPL; ++q) {
+            ga1[r][q] -= p[r][q] * im[r].v[q];
+            if constexpr (PIN) pin(ga1[r][q]);
+          }
       }
       {
         C x, y, z;
@@ -756,9 +764,9 @@ __global__ __launch_bounds__(NW *WAVE) void ac_adj_tile(AcDev d, Grid g, AdjIO i
 #pragma unroll
       for (int r = 0; r < NR; ++r) {
         const unsigned o = off(zt + r), b = span(ownbits, r);
-        stc<CPL>(p[r], rsrc(io.out + so, b), vout, o);
-        stc<CPL>(u[r], rsrc(io.out + d.field + so, b), vout, o);
-        stc<CPL>(w[r], rsrc(io.out + 2 * d.field + so, span(wbits, r)), vout, o);
+        stc<CPL>(p[r], rsrc(io.out + so, b), vrow(ownbits, r), o);
+        stc<CPL>(u[r], rsrc(io.out + d.field + so, b), vrow(ownbits, r), o);
+        stc<CPL>(w[r], rsrc(io.out + 2 * d.field + so, span(wbits, r)), vrow(wbits, r), o);
       }
     }
     if (j + 1 < ns) load(s + 1);
@@ -770,13 +778,13 @@ __global__ __launch_bounds__(NW *WAVE) void ac_adj_tile(AcDev d, Grid g, AdjIO i
     const unsigned b = ownbits & bits(r0, r1);
     C old[NR];
 #pragma unroll
-    for (int r = 0; r < NR; ++r) old[r] = ldc<CPL>(rsrc(plane, span(b, r)), vout, off(zt + r));
+    for (int r = 0; r < NR; ++r) old[r] = ldc<CPL>(rsrc(plane, span(b, r)), vrow(b, r), off(zt + r));
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
       float v[CPL];
 #pragma unroll
       for (int q = 0; q < CPL; ++q) v[q] = old[r].v[q] + (ca + q >= c0 && ca + q < c1 ? sum[r][q] : 0.f);
-      stc<CPL>(v, rsrc(plane, span(b, r)), vout, off(zt + r));
+      stc<CPL>(v, rsrc(plane, span(b, r)), vrow(b, r), off(zt + r));
     }
   };
   if (io.grad_a1) add(io.grad_a1 + (long long)grp * d.plane, ga1, fs + 1, d.Z - 2, 2, d.X - 2);
