@@ -1259,9 +1259,9 @@ bool tile_ok(const adfwi_acoustic_desc *d) {
 // tile the more of it is halo, but the sooner its workgroup is done: a launch whose workgroups
 // all run at once (one per CU) lasts as long as one of them.  So: the smallest shape that still
 // gives at most one workgroup per CU, else the largest.  Measured, forward with records / adjoint,
-// us per step: 140 x 240, 1 shot (54 / 24 / 12 workgroups): 2.4 / 2.9 / 4.3 and 2.6 / 3.0 / 4.7;
-// 10 shots (540 / 240 / 120): 5.1 / 3.3 / 4.6 and 5.5 / 3.5 / 5.2; 149 x 263, 40 shots
-// (2520 / 1120 / 480): 16.2 / 13.3 / 9.6 and 18.3 / 14.4 / 10.1.
+// us per step: 140 x 240, 1 shot (54 / 24 / 12 workgroups): 1.9 / 2.3 / 3.4 and 2.5 / 2.8 / 4.6;
+// 10 shots (540 / 240 / 120): 4.0 / 2.6 / 3.7 and 6.2 / 3.1 / 4.8; 149 x 263, 40 shots
+// (2520 / 1120 / 480): 12.5 / 9.6 / 7.3 and 19.2 / 12.5 / 9.5.
 enum class TileShape { SMALL, MEDIUM, LARGE };
 constexpr long long TILE_CUS = 256;
 
@@ -1333,10 +1333,10 @@ void launch_adj_tile_f(const AcDev &v, hipStream_t st, const tile::AdjIO &io) {
 }
 
 // With the rho gradient the adjoint reads the pressure image with its halo too, and the tile's
-// registers hold one column per lane only: 18.2 us per step against the two-step strips' 24.2 on
-// 241 x 441 with 12 shots (1008 tiles of 64 x 64), 21.9 against 31.2 on 149 x 263 with 40 (1120),
-// but 56.5 against 50.2 on 296 x 808 with 16 (2688) and 424 against 298 on 464 x 1232 with 64.
-constexpr long long A2_TILES = 1536;
+// registers hold one column per lane only: 15.5 us per step against the two-step strips' 24.0 on
+// 241 x 441 with 12 shots (1008 tiles of 64 x 64), 17.2 against 31.1 on 149 x 263 with 40 (1120),
+// 40.5 against 50.1 on 296 x 808 with 16 (2688), but 303 against 298 on 464 x 1232 with 64.
+constexpr long long A2_TILES = 4096;
 bool adj_tile_ok(const AcDev &v, bool a2) {
   return !a2 || tile_count<4, 16, 1>(v) * ((v.S + v.spb - 1) / v.spb) <= A2_TILES;
 }

@@ -201,10 +201,10 @@ class AcousticGeometry:
                                               or self.tile_z)
 
     def adjoint_tiled(self, need_a2: bool) -> bool:
-        """Whether the adjoint does too: with the rho gradient on up to 1536 tiles of 40 x 40
+        """Whether the adjoint does too: with the rho gradient on up to 4096 tiles of 40 x 40
         points and shot groups, as the library chooses."""
         tiles = -(-self.X // 40) * -(-(self.Z - int(self.layout.zbase)) // 40) * -(-self.S // self.gradient_group)
-        return self.tiled and (not need_a2 or tiles <= 1536)
+        return self.tiled and (not need_a2 or tiles <= 4096)
 
     @property
     def gradient_group(self) -> int:
