@@ -14,7 +14,7 @@
 //      vx[1]=vz[1,j+1]-vz[1,j]+vz[2,j+1]-vz[2,j]+vx[3,j], vz[0]=vz[1];
 //   6. records of the five totals.
 // Every expression keeps the reference's fp32 association (compiled with
-// -ffp-contract=off, IEEE division), so a step is bit-identical to the reference's CPU
+// -ffp-contract=off, IEEE division; the tile kernels form the same quotients otherwise), so a step is bit-identical to the reference's CPU
 // op sequence given identical coefficients.  C15/C35 terms are skipped for isotropic and
 // VTI media (exact: they multiply zeros).
 //
@@ -22,6 +22,9 @@
 // txz_x, txz_z, vx_x, vx_z, vz_x, vz_z.  The splits are identically zero outside the window
 // (never updated there); totals and free-surface rows are derived when needed, so the
 // reference's five total arrays need no storage.
+//
+// The kernels here march strips, a step per launch; elastic_tile.hpp holds the ones that keep tiles in
+// registers, which run wherever el_tile_ok (below) says so.
 //
 // Work decomposition: one wavefront owns 64 columns x0-4 .. x0+59 of a TZ-row strip and
 // writes the 55 columns x0 .. x0+54: stress is valid on lanes 2..60 (it reads velocities

@@ -3,7 +3,7 @@
 Drop-in for ADFWI/propagator/elastic_kernels.py: ``pad_torchSingle`` (:175-216),
 ``DiffCoef`` (:20-58) and ``forward_kernel`` (:917-1037, 4th-order PML branch) keep
 their signatures and results.  The per-step op sequence of step_forward_PML_4order
-(:222-423) runs as one fused HIP kernel per step; its autograd replay is replaced by
+(:222-423) runs as fused HIP kernels of one or two steps; its autograd replay is replaced by
 ``ElasticWave``, whose backward is the hand-written discrete adjoint with sqrt(nt)
 wavefield checkpoints and segment recomputation.
 """
