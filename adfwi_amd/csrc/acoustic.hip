@@ -1261,7 +1261,8 @@ bool tile_ok(const adfwi_acoustic_desc *d) {
 // gives at most one workgroup per CU, else the largest.  Measured, forward with records / adjoint,
 // us per step: 140 x 240, 1 shot (54 / 24 / 12 workgroups): 1.9 / 2.3 / 3.4 and 2.5 / 2.8 / 4.6;
 // 10 shots (540 / 240 / 120): 4.0 / 2.6 / 3.7 and 6.2 / 3.1 / 4.8; 149 x 263, 40 shots
-// (2520 / 1120 / 480): 12.5 / 9.6 / 7.3 and 19.2 / 12.5 / 9.5.
+// (2520 / 1120 / 480): 12.5 / 9.6 / 7.3 and 19.2 / 12.5 / 9.5
+// (6.7 and 7.9 with pairs of shots, below).
 enum class TileShape { SMALL, MEDIUM, LARGE };
 constexpr long long TILE_CUS = 256;
 
@@ -1278,20 +1279,42 @@ TileShape tile_shape(const AcDev &v) {
   return TileShape::LARGE;
 }
 
+// Shots per group: a group's shots follow each other in a workgroup, which reads the five
+// coefficient planes (20 bytes per point against a shot's 12) and adds to the energy or gradient planes
+// once for all of them, but a launch takes whole rounds of one workgroup per CU.  A round of groups of
+// g shots measured 12 + 9.5 g us forward (64 x 128 points, 4 steps), so: the least rounds * (1.2 + g),
+// a larger g only if it is 3 % better.  us per step for g = 1 / 2 / 4 / 8, forward and adjoint: 296 x 808, 16
+// shots 19.0 / 15.0 / 12.9 / 22.1 and 20.9 / 17.0 / 16.6 / 28.8; 149 x 263, 40 shots 9.1 / 7.6 / 12.1 / 22.0
+// and 9.4 / 7.9 / 13.3 / 24.8; 464 x 1232, 64 shots 128 at each and 169 (2) / 149 / 151.  With the rho
+// gradient (64 x 64 points) the time goes with the shots alone: pairs, 241 x 441, 12 shots 15.3 / 13.3 /
+// 13.8; 296 x 808, 16 shots 40.2 / 34.6 / 37.3.  Shots that bring their own coefficient sets keep the
+// layout's groups.
 template <int NR, int NW, int CPL>
-tile::Grid tile_grid(const AcDev &v, int spg) {
+tile::Grid tile_grid(const AcDev &v, bool a2 = false) {
   constexpr int oz = tile::out_rows(NR * NW), ox = tile::out_cols(CPL);
   tile::Grid g;
   g.ntx = (v.X + ox - 1) / ox;
   g.ntz = (v.Z - v.zbase + oz - 1) / oz;
-  g.spg = spg;
-  g.ngroups = (v.S + spg - 1) / spg;
+  g.spp = g.spg = v.spb;
+  if (!v.coef_set && tile_count<NR, NW, CPL>(v) * ((v.S + v.spb - 1) / v.spb) > TILE_CUS) {
+    if (a2) {
+      g.spg = max(v.spb, 2);
+    } else {
+      double least = 0;
+      for (int n = v.spb; n <= 8; ++n) {
+        const long long rounds = (tile_count<NR, NW, CPL>(v) * ((v.S + n - 1) / n) + TILE_CUS - 1) / TILE_CUS;
+        const double cost = (double)rounds * (1.2 + n);
+        if (n == v.spb || cost < 0.97 * least) { least = cost; g.spg = n; }
+      }
+    }
+  }
+  g.ngroups = (v.S + g.spg - 1) / g.spg;
   return g;
 }
 
 template <int NR, int NW, int CPL, int F>
 void launch_fwd_tile_c(const AcDev &v, hipStream_t st, const tile::FwdIO &io) {
-  const tile::Grid g = tile_grid<NR, NW, CPL>(v, v.spb);
+  const tile::Grid g = tile_grid<NR, NW, CPL>(v);
   hipLaunchKernelGGL((tile::ac_fwd_tile<NR, NW, CPL, F>), dim3((unsigned)(g.ntx * g.ntz * g.ngroups)),
                      dim3(NW * WAVE), 0, st, v, g, io);
 }
@@ -1316,7 +1339,7 @@ void launch_fwd_tile(const AcDev &v, hipStream_t st, const tile::FwdIO &io) {
 
 template <int NR, int NW, int CPL, bool A2, bool FULL>
 void launch_adj_tile_c(const AcDev &v, hipStream_t st, const tile::AdjIO &io) {
-  const tile::Grid g = tile_grid<NR, NW, CPL>(v, v.spb);
+  const tile::Grid g = tile_grid<NR, NW, CPL>(v, A2);
   hipLaunchKernelGGL((tile::ac_adj_tile<NR, NW, CPL, A2, FULL>), dim3((unsigned)(g.ntx * g.ntz * g.ngroups)),
                      dim3(NW * WAVE), 0, st, v, g, io);
 }
@@ -1333,9 +1356,9 @@ void launch_adj_tile_f(const AcDev &v, hipStream_t st, const tile::AdjIO &io) {
 }
 
 // With the rho gradient the adjoint reads the pressure image with its halo too, and the tile's
-// registers hold one column per lane only: 15.5 us per step against the two-step strips' 24.0 on
-// 241 x 441 with 12 shots (1008 tiles of 64 x 64), 17.2 against 31.1 on 149 x 263 with 40 (1120),
-// 40.5 against 50.1 on 296 x 808 with 16 (2688), but 303 against 298 on 464 x 1232 with 64.
+// registers hold one column per lane only: 13.3 us per step against the two-step strips' 24.0 on
+// 241 x 441 with 12 shots (1008 tiles of 64 x 64), 16.7 against 31.1 on 149 x 263 with 40 (1120),
+// 34.6 against 50.1 on 296 x 808 with 16 (2688), but 303 against 298 on 464 x 1232 with 64.
 constexpr long long A2_TILES = 4096;
 bool adj_tile_ok(const AcDev &v, bool a2) {
   return !a2 || tile_count<4, 16, 1>(v) * ((v.S + v.spb - 1) / v.spb) <= A2_TILES;

@@ -75,6 +75,7 @@ __device__ __forceinline__ void pin(float &v) { asm volatile("" : "+v"(v)); }
 
 struct Grid {
   int ntx, ntz, ngroups, spg;      // tiles along x and z, shot groups, shots per group
+  int spp;                         // shots per plane of the energy maps and gradients (<= spg)
 };
 
 struct FwdIO {
@@ -388,7 +389,7 @@ __global__ __launch_bounds__(NW *WAVE) void ac_fwd_tile(AcDev d, Grid g, FwdIO i
   else march(std::integral_constant<int, 0>{});
   if constexpr (FR) {
     if (io.energy) {
-      float *const e = io.energy + (long long)grp * 2 * d.plane;
+      float *const e = io.energy + (long long)(s0 / g.spp) * 2 * d.plane;
       auto add = [&](float *plane, const float (&sum)[FR ? NR : 1][CPL]) {
         C old[NR];
 #pragma unroll
@@ -787,8 +788,8 @@ __global__ __launch_bounds__(NW *WAVE) void ac_adj_tile(AcDev d, Grid g, AdjIO i
       stc<CPL>(v, rsrc(plane, span(b, r)), vrow(b, r), off(zt + r));
     }
   };
-  if (io.grad_a1) add(io.grad_a1 + (long long)grp * d.plane, ga1, fs + 1, d.Z - 2, 2, d.X - 2);
-  if constexpr (A2) add(io.grad_a2 + (long long)grp * d.plane, ga2, fs, d.Z - 1, 1, d.X - 1);
+  if (io.grad_a1) add(io.grad_a1 + (long long)(s0 / g.spp) * d.plane, ga1, fs + 1, d.Z - 2, 2, d.X - 2);
+  if constexpr (A2) add(io.grad_a2 + (long long)(s0 / g.spp) * d.plane, ga2, fs, d.Z - 1, 1, d.X - 1);
 }
 
 }  // namespace tile

@@ -8,9 +8,9 @@ and 40 x 104) and put the grid's edges at, one short of and one past a tile's; o
 lane with one column; one grid is the smallest the library takes.  nt and the checkpoint interval
 leave launches of one, two, three and four steps.
 
-Tolerance of the reordered sums: N = shots * steps terms per point, at most 64 * 37 = 2368, each
-addition rounding to 2^-24: sqrt(N) * 2^-24 = 2.9e-6 for terms of one sign (the energy maps); 5e-6
-leaves room for the gradients' cancellation.
+Tolerance of the reordered sums: N = shots * steps terms per point, each addition rounding to 2^-24:
+sqrt(N) * 2^-24 for terms of one sign (the energy maps), 2.9e-6 for 64 shots; 5e-6, and for more shots
+twice that bound, leaves room for the gradients' cancellation.
 """
 import numpy as np
 import pytest
@@ -31,6 +31,8 @@ CASES = [
     (41, 105, 64, 0),        # 64 x 128 tiles, one past a tile each way
     (40, 208, 63, 6),        # 64 x 128 tiles ending at the grid's edges
     (79, 103, 64, 0),        # odd width, last tile one column short
+    (41, 105, 81, 0),        # over 256 workgroups: pairs of shots, the last group one shot
+    (41, 105, 161, 5),       # groups of three, the last of two
 ]
 
 
@@ -39,6 +41,7 @@ CASES = [
 def test_tiles_equal_one_step_kernels(monkeypatch, Z, X, S, fs, needs):
     from adfwi_amd.propagator import acoustic_kernels as ak
     rng = np.random.default_rng(Z * 1000 + X)
+    tol = max(5e-6, 2 * (S * 37) ** 0.5 * 2 ** -24 if S > 64 else 0)
     nt, k = 37, 11                       # segments of 11: launches of 4, 4 and 3 steps; the last of 4
     nabc = fs if fs else 1
     lo = max(fs, 1)
@@ -71,8 +74,8 @@ def test_tiles_equal_one_step_kernels(monkeypatch, Z, X, S, fs, needs):
     for i in range(3):
         assert np.array_equal(r0[i], r1[i]), ("record", i, rel_l2(r1[i], r0[i]))
     for i in range(3, 6):
-        assert rel_l2(r1[i], r0[i]) <= 5e-6, ("energy", i, rel_l2(r1[i], r0[i]))
-    assert rel_l2(g1, g0) <= 5e-6, rel_l2(g1, g0)
+        assert rel_l2(r1[i], r0[i]) <= tol, ("energy", i, rel_l2(r1[i], r0[i]))
+    assert rel_l2(g1, g0) <= tol, rel_l2(g1, g0)
     if needs == "all":
-        assert rel_l2(h1, h0) <= 5e-6, rel_l2(h1, h0)
+        assert rel_l2(h1, h0) <= tol, rel_l2(h1, h0)
         assert np.array_equal(w0, w1), rel_l2(w1, w0)
