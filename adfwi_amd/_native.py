@@ -90,6 +90,10 @@ _SIGNATURES = {
                                               ctypes.POINTER(AcousticFwdArgs), _vp]),
     "adfwi_acoustic_adjoint": (ctypes.c_int, [ctypes.POINTER(AcousticDesc),
                                               ctypes.POINTER(AcousticAdjArgs), _vp]),
+    "adfwi_acoustic_forward_sum": (ctypes.c_int, [ctypes.POINTER(AcousticDesc),
+                                                  ctypes.POINTER(AcousticFwdArgs), _vp]),
+    "adfwi_acoustic_adjoint_sum": (ctypes.c_int, [ctypes.POINTER(AcousticDesc),
+                                                  ctypes.POINTER(AcousticAdjArgs), _vp]),
     "adfwi_acoustic_adjoint_noalloc": (ctypes.c_int, [ctypes.POINTER(AcousticDesc),
                                                       ctypes.POINTER(AcousticAdjArgs), _vp, _vp, _vp]),
     "adfwi_elastic_get_layout": (ctypes.c_int, [ctypes.POINTER(ElasticDesc), ctypes.POINTER(Layout)]),

@@ -1287,16 +1287,17 @@ TileShape tile_shape(const AcDev &v) {
 // shots 19.0 / 15.0 / 12.9 / 22.1 and 20.9 / 17.0 / 16.6 / 28.8; 149 x 263, 40 shots 9.1 / 7.6 / 12.1 / 22.0
 // and 9.4 / 7.9 / 13.3 / 24.8; 464 x 1232, 64 shots 128 at each and 169 (2) / 149 / 151.  With the rho
 // gradient (64 x 64 points) the time goes with the shots alone: pairs, 241 x 441, 12 shots 15.3 / 13.3 /
-// 13.8; 296 x 808, 16 shots 40.2 / 34.6 / 37.3.  Shots that bring their own coefficient sets keep the
-// layout's groups.
+// 13.8; 296 x 808, 16 shots 40.2 / 34.6 / 37.3.  A group adds all its shots to the plane of its first
+// one, so shots keep the layout's groups where those planes are to stay apart (`apart`), and where they
+// bring their own coefficient sets.
 template <int NR, int NW, int CPL>
-tile::Grid tile_grid(const AcDev &v, bool a2 = false) {
+tile::Grid tile_grid(const AcDev &v, bool apart, bool a2) {
   constexpr int oz = tile::out_rows(NR * NW), ox = tile::out_cols(CPL);
   tile::Grid g;
   g.ntx = (v.X + ox - 1) / ox;
   g.ntz = (v.Z - v.zbase + oz - 1) / oz;
   g.spp = g.spg = v.spb;
-  if (!v.coef_set && tile_count<NR, NW, CPL>(v) * ((v.S + v.spb - 1) / v.spb) > TILE_CUS) {
+  if (!v.coef_set && !apart && tile_count<NR, NW, CPL>(v) * ((v.S + v.spb - 1) / v.spb) > TILE_CUS) {
     if (a2) {
       g.spg = max(v.spb, 2);
     } else {
@@ -1313,45 +1314,45 @@ tile::Grid tile_grid(const AcDev &v, bool a2 = false) {
 }
 
 template <int NR, int NW, int CPL, int F>
-void launch_fwd_tile_c(const AcDev &v, hipStream_t st, const tile::FwdIO &io) {
-  const tile::Grid g = tile_grid<NR, NW, CPL>(v);
+void launch_fwd_tile_c(const AcDev &v, hipStream_t st, const tile::FwdIO &io, bool apart) {
+  const tile::Grid g = tile_grid<NR, NW, CPL>(v, apart && io.energy, false);
   hipLaunchKernelGGL((tile::ac_fwd_tile<NR, NW, CPL, F>), dim3((unsigned)(g.ntx * g.ntz * g.ngroups)),
                      dim3(NW * WAVE), 0, st, v, g, io);
 }
 
 template <int F>
-void launch_fwd_tile_f(const AcDev &v, hipStream_t st, const tile::FwdIO &io) {
+void launch_fwd_tile_f(const AcDev &v, hipStream_t st, const tile::FwdIO &io, bool apart) {
   switch (tile_shape(v)) {
-    case TileShape::SMALL: launch_fwd_tile_c<4, 10, 1, F>(v, st, io); break;
-    case TileShape::MEDIUM: launch_fwd_tile_c<4, 16, 1, F>(v, st, io); break;
-    default: launch_fwd_tile_c<4, 16, 2, F>(v, st, io);
+    case TileShape::SMALL: launch_fwd_tile_c<4, 10, 1, F>(v, st, io, apart); break;
+    case TileShape::MEDIUM: launch_fwd_tile_c<4, 16, 1, F>(v, st, io, apart); break;
+    default: launch_fwd_tile_c<4, 16, 2, F>(v, st, io, apart);
   }
 }
 
-void launch_fwd_tile(const AcDev &v, hipStream_t st, const tile::FwdIO &io) {
+void launch_fwd_tile(const AcDev &v, hipStream_t st, const tile::FwdIO &io, bool apart) {
   const bool rec = io.energy || io.rec_p;
-  if (!io.img_d && !io.img_p) launch_fwd_tile_f<PF_REC>(v, st, io);
-  else if (!rec && !io.img_p) launch_fwd_tile_f<PF_IMGD>(v, st, io);
-  else if (!rec) launch_fwd_tile_f<PF_IMGD | PF_IMGP>(v, st, io);
-  else if (!io.img_p) launch_fwd_tile_f<PF_REC | PF_IMGD>(v, st, io);
-  else launch_fwd_tile_f<PF_REC | PF_IMGD | PF_IMGP>(v, st, io);
+  if (!io.img_d && !io.img_p) launch_fwd_tile_f<PF_REC>(v, st, io, apart);
+  else if (!rec && !io.img_p) launch_fwd_tile_f<PF_IMGD>(v, st, io, apart);
+  else if (!rec) launch_fwd_tile_f<PF_IMGD | PF_IMGP>(v, st, io, apart);
+  else if (!io.img_p) launch_fwd_tile_f<PF_REC | PF_IMGD>(v, st, io, apart);
+  else launch_fwd_tile_f<PF_REC | PF_IMGD | PF_IMGP>(v, st, io, apart);
 }
 
 template <int NR, int NW, int CPL, bool A2, bool FULL>
-void launch_adj_tile_c(const AcDev &v, hipStream_t st, const tile::AdjIO &io) {
-  const tile::Grid g = tile_grid<NR, NW, CPL>(v, A2);
+void launch_adj_tile_c(const AcDev &v, hipStream_t st, const tile::AdjIO &io, bool apart) {
+  const tile::Grid g = tile_grid<NR, NW, CPL>(v, apart && (io.grad_a1 || io.grad_a2), A2);
   hipLaunchKernelGGL((tile::ac_adj_tile<NR, NW, CPL, A2, FULL>), dim3((unsigned)(g.ntx * g.ntz * g.ngroups)),
                      dim3(NW * WAVE), 0, st, v, g, io);
 }
 
 template <bool A2, bool FULL>
-void launch_adj_tile_f(const AcDev &v, hipStream_t st, const tile::AdjIO &io) {
+void launch_adj_tile_f(const AcDev &v, hipStream_t st, const tile::AdjIO &io, bool apart) {
   switch (tile_shape(v)) {
-    case TileShape::SMALL: launch_adj_tile_c<4, 10, 1, A2, FULL>(v, st, io); break;
-    case TileShape::MEDIUM: launch_adj_tile_c<4, 16, 1, A2, FULL>(v, st, io); break;
+    case TileShape::SMALL: launch_adj_tile_c<4, 10, 1, A2, FULL>(v, st, io, apart); break;
+    case TileShape::MEDIUM: launch_adj_tile_c<4, 16, 1, A2, FULL>(v, st, io, apart); break;
     default:
-      if constexpr (A2) launch_adj_tile_c<4, 16, 1, A2, FULL>(v, st, io);   // (two columns per lane spill)
-      else launch_adj_tile_c<4, 16, 2, A2, FULL>(v, st, io);
+      if constexpr (A2) launch_adj_tile_c<4, 16, 1, A2, FULL>(v, st, io, apart);   // (two columns per lane spill)
+      else launch_adj_tile_c<4, 16, 2, A2, FULL>(v, st, io, apart);
   }
 }
 
@@ -1364,10 +1365,10 @@ bool adj_tile_ok(const AcDev &v, bool a2) {
   return !a2 || tile_count<4, 16, 1>(v) * ((v.S + v.spb - 1) / v.spb) <= A2_TILES;
 }
 
-void launch_adj_tile(const AcDev &v, hipStream_t st, const tile::AdjIO &io) {
+void launch_adj_tile(const AcDev &v, hipStream_t st, const tile::AdjIO &io, bool apart) {
   const bool full = io.grad_src || io.g_u || io.g_w, a2 = io.grad_a2 && io.img_p;
-  if (a2) full ? launch_adj_tile_f<true, true>(v, st, io) : launch_adj_tile_f<true, false>(v, st, io);
-  else full ? launch_adj_tile_f<false, true>(v, st, io) : launch_adj_tile_f<false, false>(v, st, io);
+  if (a2) full ? launch_adj_tile_f<true, true>(v, st, io, apart) : launch_adj_tile_f<true, false>(v, st, io, apart);
+  else full ? launch_adj_tile_f<false, true>(v, st, io, apart) : launch_adj_tile_f<false, false>(v, st, io, apart);
 }
 
 dim3 step_grid(const adfwi_layout &L) { return dim3((L.ntiles + WPB - 1) / WPB, L.ngroups); }
@@ -1482,7 +1483,8 @@ int adfwi_acoustic_get_layout(const adfwi_acoustic_desc *d, adfwi_layout *out) {
   return layout_of(d, out);
 }
 
-int adfwi_acoustic_forward(const adfwi_acoustic_desc *d, adfwi_acoustic_fwd_args *a, adfwi_stream_t stream) {
+// apart: the energy planes hold their own group's shots each (else only their sum counts)
+static int acoustic_forward(const adfwi_acoustic_desc *d, adfwi_acoustic_fwd_args *a, adfwi_stream_t stream, bool apart) {
   if (int rc = adfwi::fault_injected("adfwi_acoustic_forward")) return rc;
   adfwi_layout L;
   int rc = layout_of(d, &L);
@@ -1534,7 +1536,7 @@ int adfwi_acoustic_forward(const adfwi_acoustic_desc *d, adfwi_acoustic_fwd_args
       io.img_p = a->image_p ? a->image_p + (long long)k * L.field_floats : nullptr;
       io.rmap = recs && d->nrec > 0 ? a->rcv_map : nullptr;
       io.rec_p = recs ? a->rec_p : nullptr; io.rec_u = a->rec_u; io.rec_w = a->rec_w;
-      launch_fwd_tile(v, st, io);
+      launch_fwd_tile(v, st, io, apart);
       if ((rc = adfwi::check_launch("ac_fwd_tile"))) return rc;
       cur = nxt;
       k += n;
@@ -1576,7 +1578,16 @@ int adfwi_acoustic_forward(const adfwi_acoustic_desc *d, adfwi_acoustic_fwd_args
   return ADFWI_OK;
 }
 
-int adfwi_acoustic_adjoint(const adfwi_acoustic_desc *d, adfwi_acoustic_adj_args *a, adfwi_stream_t stream) {
+int adfwi_acoustic_forward(const adfwi_acoustic_desc *d, adfwi_acoustic_fwd_args *a, adfwi_stream_t stream) {
+  return acoustic_forward(d, a, stream, true);
+}
+
+int adfwi_acoustic_forward_sum(const adfwi_acoustic_desc *d, adfwi_acoustic_fwd_args *a, adfwi_stream_t stream) {
+  return acoustic_forward(d, a, stream, false);
+}
+
+// apart: as above, for the planes of the coefficient gradients
+static int acoustic_adjoint(const adfwi_acoustic_desc *d, adfwi_acoustic_adj_args *a, adfwi_stream_t stream, bool apart) {
   if (int rc = adfwi::fault_injected("adfwi_acoustic_adjoint")) return rc;
   adfwi_layout L;
   int rc = layout_of(d, &L);
@@ -1625,7 +1636,7 @@ int adfwi_acoustic_adjoint(const adfwi_acoustic_desc *d, adfwi_acoustic_adj_args
       io.grad_a1 = a->grad_a1; io.grad_a2 = a->grad_a2; io.grad_src = a->grad_src;
       io.rmap = recs && d->nrec > 0 ? a->rcv_map : nullptr;
       io.g_p = a->grad_rec_p; io.g_u = a->grad_rec_u; io.g_w = a->grad_rec_w;
-      launch_adj_tile(v1, st, io);
+      launch_adj_tile(v1, st, io, apart);
       if ((rc = adfwi::check_launch("ac_adj_tile"))) return rc;
       cur = nxt;
       k += n;
@@ -1668,6 +1679,14 @@ int adfwi_acoustic_adjoint(const adfwi_acoustic_desc *d, adfwi_acoustic_adj_args
   }
   a->lam_out = cur;
   return ADFWI_OK;
+}
+
+int adfwi_acoustic_adjoint(const adfwi_acoustic_desc *d, adfwi_acoustic_adj_args *a, adfwi_stream_t stream) {
+  return acoustic_adjoint(d, a, stream, true);
+}
+
+int adfwi_acoustic_adjoint_sum(const adfwi_acoustic_desc *d, adfwi_acoustic_adj_args *a, adfwi_stream_t stream) {
+  return acoustic_adjoint(d, a, stream, false);
 }
 
 }  // extern "C"
@@ -1765,7 +1784,7 @@ int adfwi_acoustic_adjoint_noalloc(const adfwi_acoustic_desc *d, adfwi_acoustic_
     hipLaunchKernelGGL(fill_zero, flat_grid(need), dim3(256), 0, st, base, need);
     if ((rc = adfwi::check_launch("fill_zero"))) return rc;
   }
-  if ((rc = adfwi_acoustic_adjoint(d, &b, stream))) return rc;
+  if ((rc = adfwi_acoustic_adjoint_sum(d, &b, stream))) return rc;
   a->lam_out = b.lam_out;
   if (grad_a1_sum) {
     hipLaunchKernelGGL(add_plane_sum, flat_grid(plane), dim3(256), 0, st, b.grad_a1, (int)nplanes, plane, grad_a1_sum);

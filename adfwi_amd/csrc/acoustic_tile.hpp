@@ -75,7 +75,7 @@ __device__ __forceinline__ void pin(float &v) { asm volatile("" : "+v"(v)); }
 
 struct Grid {
   int ntx, ntz, ngroups, spg;      // tiles along x and z, shot groups, shots per group
-  int spp;                         // shots per plane of the energy maps and gradients (<= spg)
+  int spp;                         // shots per plane of the energy maps and gradients (<= spg; a group's go to its first one)
 };
 
 struct FwdIO {

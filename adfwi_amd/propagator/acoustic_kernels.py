@@ -386,7 +386,7 @@ def run_forward(geom: AcousticGeometry, coef: torch.Tensor, src: torch.Tensor, *
             name, launches = ("ac_fwd_pair" if fused else "ac_fwd_step",
                               sum(forward_launches(t0, nsteps, nt, int(a.ckpt_every), fused)))
         TIMELINE.call(kind, name, launches, dev, lambda: nat.check(
-            lib.adfwi_acoustic_forward(ctypes.byref(d), ctypes.byref(a), nat.stream_handle(dev)),
+            lib.adfwi_acoustic_forward_sum(ctypes.byref(d), ctypes.byref(a), nat.stream_handle(dev)),
             "adfwi_acoustic_forward"), steps=nsteps)
         return a.state_out
 
@@ -518,8 +518,8 @@ def run_backward(geom: AcousticGeometry, coef: torch.Tensor, src: torch.Tensor, 
                 ctypes.byref(d), ctypes.byref(aa), nat.ptr(ga1), nat.ptr(ga2), stream),
                 "adfwi_acoustic_adjoint_noalloc")
         else:
-            call = lambda: nat.check(lib.adfwi_acoustic_adjoint(ctypes.byref(d), ctypes.byref(aa), stream),
-                                     "adfwi_acoustic_adjoint")
+            adjoint = lib.adfwi_acoustic_adjoint if group_planes else lib.adfwi_acoustic_adjoint_sum
+            call = lambda: nat.check(adjoint(ctypes.byref(d), ctypes.byref(aa), stream), "adfwi_acoustic_adjoint")
         if fused and geom.adjoint_tiled(need_a2):
             name, launches = "ac_adj_tile", -(-n // TILE_STEPS)
         else:

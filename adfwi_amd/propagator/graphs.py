@@ -70,8 +70,9 @@ class GraphedForward:
                 g = torch.cuda.CUDAGraph()
                 g.capture_begin(capture_error_mode="thread_local")
                 try:
-                    nat.check(lib.adfwi_acoustic_forward(ctypes.byref(self._desc), ctypes.byref(a),
-                                                         nat.stream_handle(dev)), "adfwi_acoustic_forward (graph)")
+                    nat.check(lib.adfwi_acoustic_forward_sum(ctypes.byref(self._desc), ctypes.byref(a),
+                                                             nat.stream_handle(dev)),
+                              "adfwi_acoustic_forward (graph)")
                     if advance:
                         self.tb.add_(self.K)
                 finally:

@@ -128,9 +128,15 @@ typedef struct adfwi_acoustic_fwd_args {
                               are skipped).  Requires ckpt == NULL. */
 } adfwi_acoustic_fwd_args;
 
-/* Forward time stepping (replaces step_forward, acoustic_kernels.py:40-176). */
+/* Forward time stepping (replaces step_forward, acoustic_kernels.py:40-176).  Plane g of `energy`
+ * holds the shots of group g, [g * shots_per_block, (g + 1) * shots_per_block). */
 int adfwi_acoustic_forward(const adfwi_acoustic_desc *d, adfwi_acoustic_fwd_args *a,
                            adfwi_stream_t stream);
+
+/* The same for callers that only use the sum of the energy planes: a shot's terms may go to any of
+ * them, so that a launch may take more shots together (which reads the coefficients less often). */
+int adfwi_acoustic_forward_sum(const adfwi_acoustic_desc *d, adfwi_acoustic_fwd_args *a,
+                               adfwi_stream_t stream);
 
 typedef struct adfwi_acoustic_adj_args {
   const float *lam_in;     /* adjoint state after step t_hi, receiver sources of t_hi not yet
@@ -142,7 +148,8 @@ typedef struct adfwi_acoustic_adj_args {
   const float *image;      /* stencil images written by adfwi_acoustic_forward */
   const float *image_p;    /* pressure images, or NULL when grad_a2 is NULL */
   const float *grad_rec_p, *grad_rec_u, *grad_rec_w; /* [S][nt][R] or NULL */
-  float *grad_a1, *grad_a2; /* [ngroups][Z][pitch] (+=) or NULL */
+  float *grad_a1, *grad_a2; /* [groups][Z][pitch] (+=) or NULL: accum_floats / (Z * pitch) planes of
+                               min(shots_per_block, layout.reserved) consecutive shots each */
   float *grad_src;          /* [S][nt] or NULL: d loss / d src */
   const float *lam_out;     /* OUT: adjoint state after step t_hi-nsteps (its sources not added) */
   const int32_t *rcv_map;   /* as in adfwi_acoustic_fwd_args: lets several steps share one
@@ -155,6 +162,11 @@ typedef struct adfwi_acoustic_adj_args {
  * acoustic_kernels.py:115-169), with zero-lag imaging of dL/dA1 and dL/dA2. */
 int adfwi_acoustic_adjoint(const adfwi_acoustic_desc *d, adfwi_acoustic_adj_args *a,
                            adfwi_stream_t stream);
+
+/* The same for callers that only use the sum of the gradient planes: a shot's terms may go to any
+ * of them, so that a launch may take more shots together. */
+int adfwi_acoustic_adjoint_sum(const adfwi_acoustic_desc *d, adfwi_acoustic_adj_args *a,
+                               adfwi_stream_t stream);
 
 /* Size of the library's per-GPU scratch array used by adfwi_acoustic_adjoint_noalloc, in
  * floats (128 MiB). */
