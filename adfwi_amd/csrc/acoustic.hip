@@ -1519,7 +1519,9 @@ static int acoustic_forward(const adfwi_acoustic_desc *d, adfwi_acoustic_fwd_arg
     return nullptr;
   };
   const float *cur = a->state_in;
-  if (fuse && tile_ok(d)) {
+  // (the tile kernels that write the pressure image write the stencil image too: a pressure image
+  // alone, for a gradient of A2 and not of A1, is left to the strip kernels)
+  if (fuse && tile_ok(d) && (a->image || !a->image_p)) {
     for (int k = 0; k < a->nsteps;) {
       const int t = a->t0 + k;
       int n = min(tile::TK, a->nsteps - k);

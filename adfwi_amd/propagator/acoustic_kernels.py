@@ -196,7 +196,7 @@ class AcousticGeometry:
     @property
     def tiled(self) -> bool:
         """Whether fused steps run on the tile kernels (the strip options of the descriptor ask
-        for the strip kernels)."""
+        for the strip kernels; so does a forward that writes the pressure image alone)."""
         return bool(self.fuse_steps) and not (self.shots_per_block or self.adj_shots_per_block or self.row_unroll
                                               or self.tile_z)
 
@@ -380,7 +380,7 @@ def run_forward(geom: AcousticGeometry, coef: torch.Tensor, src: torch.Tensor, *
         a.image_p = None if img_p is None else img_p.data_ptr()
         a.rcv_map = None if geom.rcv_map is None else geom.rcv_map.data_ptr()
         a.fuse_steps = geom.fuse_steps
-        if fused and geom.tiled:
+        if fused and geom.tiled and (img is not None or img_p is None):
             name, launches = "ac_fwd_tile", tile_launches(t0, nsteps, int(a.ckpt_every))
         else:
             name, launches = ("ac_fwd_pair" if fused else "ac_fwd_step",
@@ -489,7 +489,7 @@ def run_backward(geom: AcousticGeometry, coef: torch.Tensor, src: torch.Tensor, 
             fa.image = None if image is None else image.data_ptr()
             fa.image_p = None if image_p is None else image_p.data_ptr()
             fa.fuse_steps = geom.fuse_steps
-            if geom.tiled:
+            if geom.tiled and need_a1:
                 name, launches = "ac_fwd_tile", tile_launches(t_lo, n, 0)
             else:
                 name, launches = ("ac_fwd_pair" if geom.fuse_steps else "ac_fwd_step",

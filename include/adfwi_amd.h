@@ -109,7 +109,9 @@ typedef struct adfwi_acoustic_fwd_args {
   float *rec_p, *rec_u, *rec_w; /* [S][nt][R] or NULL */
   float *energy;           /* [ngroups][2][Z][pitch] (+=) or NULL: sum over shots of p^2 every
                               step and of u^2 from step energy_u_from on */
-  float *image;            /* [nsteps][S][Z][pitch] or NULL: p-update stencil of each step */
+  float *image;            /* [nsteps][S][Z][pitch] or NULL: p-update stencil of each step (at the points
+                              that the update leaves alone, the two outer rows and columns and the rows
+                              down to fs, it is unspecified, and the adjoint does not use it) */
   float *image_p;          /* [nsteps][S][Z][pitch] or NULL: p after each step */
   const float *state_out;  /* OUT: buffer holding the state after the last step */
   const int32_t *rcv_map;  /* [nz + nz*pitch] or NULL: receivers per row, then the receiver index
@@ -119,7 +121,8 @@ typedef struct adfwi_acoustic_fwd_args {
   int32_t fuse_steps;      /* 1: advance several steps per launch where possible (four on register
                               tiles; two when the descriptor sets shots_per_block,
                               adj_shots_per_block, row_unroll or tile_z, which are options of the
-                              strip kernels, or the pitch is odd); 0: one */
+                              strip kernels, the pitch is odd, or image_p is set without image);
+                              0: one */
   int32_t reserved2;
   const int32_t *t_base;   /* device int or NULL: added at run time to every step index of the
                               call (t0 .. t0+nsteps-1 are then relative), so that one captured
