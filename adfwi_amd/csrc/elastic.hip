@@ -2384,10 +2384,10 @@ int el_layout(const adfwi_elastic_desc *d, adfwi_layout *L) {
                   "grid of %d x %d (pitch %d) exceeds the 2 GiB of one set of gradient planes",
                   d->nz, d->nx, d->pitch);
   L->state_floats = nf * L->field_floats;
-  // gradient planes: a set per group of the adjoint that may run (step kernels or tiles)
+  // gradient planes: a set per group of the adjoint that may run (step kernels or tiles).  Whatever
+  // `aniso` says now: a problem's buffers serve models with and without C15 / C35
   int sets = L->ngroups;
-  if (!d->aniso && d->shots_per_wave == 0 && d->tile_z == 0)
-    sets = max(sets, el_adj_tile_shape(d).groups);
+  if (d->shots_per_wave == 0 && d->tile_z == 0) sets = max(sets, el_adj_tile_shape(d).groups);
   L->accum_floats = (int64_t)sets * NCOEF * d->nz * d->pitch;
   return ADFWI_OK;
 }

@@ -7,6 +7,7 @@ their signatures and results.  The per-step op sequence of step_forward_PML_4ord
 ``ElasticWave``, whose backward is the hand-written discrete adjoint with sqrt(nt)
 wavefield checkpoints and segment recomputation.
 """
+import copy
 import ctypes
 import math
 import os
@@ -443,6 +444,8 @@ def forward_kernel(nx: int, nz: int, dx: float, dz: float, nt: int, dt: float,
                                    (rcv_x + nabc).cpu().numpy(), device, aniso=aniso, damping=not use_pml,
                                    src_fz=src_fz, nn=fso, c2=float(fdc[2]) if fso > 2 else 0.0)
     elif geometry.aniso != aniso:
+        # a copy: the caller's geometry may still have a backward pass to run for another model
+        geometry = copy.copy(geometry)
         geometry.aniso = aniso
     if use_pml:
         bcx_p = pad_torchSingle(bcx.to(device=device, dtype=torch.float32), 0, fso, free_surface, device)
