@@ -2322,6 +2322,11 @@ ElAdjTile el_adj_tile_shape(const adfwi_elastic_desc *d) {
   return best;
 }
 
+// workgroups of the step kernels along the shots
+int step_groups(const adfwi_elastic_desc *d, const adfwi_layout &L) {
+  return (d->nshots + L.shots_per_block - 1) / L.shots_per_block;
+}
+
 int el_layout(const adfwi_elastic_desc *d, adfwi_layout *L) {
   if (!d) { adfwi::set_error("null descriptor"); return ADFWI_E_ARG; }
   if (d->abi_version != ADFWI_ABI_VERSION || d->struct_size != (int32_t)sizeof(adfwi_elastic_desc)) {
@@ -2369,7 +2374,6 @@ int el_layout(const adfwi_elastic_desc *d, adfwi_layout *L) {
       spw *= 2;
   }
   L->shots_per_block = spw * EWPB;
-  L->ngroups = (d->nshots + L->shots_per_block - 1) / L->shots_per_block;
   ADFWI_CHECK_ARG(d->damping == 0 || d->damping == 1, "damping must be 0 (PML) or 1 (got %d)", d->damping);
   const int nf = d->damping ? NFIELD5 : NFIELD;
   L->nfields = nf;
@@ -2386,9 +2390,9 @@ int el_layout(const adfwi_elastic_desc *d, adfwi_layout *L) {
   L->state_floats = nf * L->field_floats;
   // gradient planes: a set per group of the adjoint that may run (step kernels or tiles).  Whatever
   // `aniso` says now: a problem's buffers serve models with and without C15 / C35
-  int sets = L->ngroups;
-  if (d->shots_per_wave == 0 && d->tile_z == 0) sets = max(sets, el_adj_tile_shape(d).groups);
-  L->accum_floats = (int64_t)sets * NCOEF * d->nz * d->pitch;
+  L->ngroups = step_groups(d, *L);
+  if (d->shots_per_wave == 0 && d->tile_z == 0) L->ngroups = max(L->ngroups, el_adj_tile_shape(d).groups);
+  L->accum_floats = (int64_t)L->ngroups * NCOEF * d->nz * d->pitch;
   return ADFWI_OK;
 }
 
@@ -2537,7 +2541,7 @@ int adfwi_elastic_forward(const adfwi_elastic_desc *d, adfwi_elastic_fwd_args *a
   ADFWI_CHECK_ARG(!a->ckpt || a->ckpt_every >= 1, "ckpt_every must be >= 1 with a checkpoint buffer");
   ElDev v = el_dev(d, L);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const dim3 grid(L.ntiles, L.ngroups), block(ENT);
+  const dim3 grid(L.ntiles, step_groups(d, L)), block(ENT);
   const long long ng = (long long)d->nshots * d->nrec;
   const dim3 ggrid((unsigned)((ng + 255) / 256)), gblock(256);
   // the 4th-order PML step takes its records itself when the receiver map is given
@@ -2689,14 +2693,14 @@ static int elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *
       tz = 8;
       for (int n = 1; (rows + n - 1) / n >= 8; ++n) {
         const int cand = ((rows + n - 1) / n + 3) / 4 * 4;
-        if (cand <= ETZ_MAX && (long long)n * v.nsx * L.ngroups * EWPB >= 2048) { tz = cand; break; }
+        if (cand <= ETZ_MAX && (long long)n * v.nsx * step_groups(d, L) * EWPB >= 2048) { tz = cand; break; }
       }
     }
     v.tz = tz;
   }
   v.nstrips = ((rows + v.tz - 1) / v.tz) * v.nsx;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const dim3 grid(v.nstrips, L.ngroups), block(ENT);
+  const dim3 grid(v.nstrips, step_groups(d, L)), block(ENT);
   const long long ng = (long long)d->nshots * d->nrec;
   const dim3 ggrid((unsigned)((ng + 255) / 256)), gblock(256);
   const int t_lo = a->t_hi - a->nsteps;

@@ -237,10 +237,10 @@ typedef struct adfwi_elastic_desc {
 } adfwi_elastic_desc;
 
 /* Tiling and buffer sizes; layout.nfields = 10 (PML split fields) or 5 (damping), layout.reserved = shots per
- * wavefront, layout.shots_per_block = shots per workgroup, layout.ngroups = workgroups along
- * the shots, layout.accum_floats = size of the gradient accumulator of the adjoint,
- * [sets][8][nz][pitch] (one set of planes per workgroup's shots; layout.accum_floats gives the
- * sets, at least ngroups), their sum over the sets. */
+ * wavefront, layout.shots_per_block = shots per workgroup (of the step kernels), layout.ngroups = sets
+ * of gradient planes (the adjoint may group the shots otherwise), layout.accum_floats = size of the
+ * gradient accumulator of the adjoint, [ngroups][8][nz][pitch]; the gradient is the sum over the sets.
+ * The layout does not depend on aniso. */
 int adfwi_elastic_get_layout(const adfwi_elastic_desc *d, adfwi_layout *out);
 
 typedef struct adfwi_elastic_fwd_args {
