@@ -72,7 +72,7 @@ class ElasticDesc(ctypes.Structure):
 
 class ElasticFwdArgs(ctypes.Structure):
     _fields_ = [("state_in", _vp), ("work", _vp * 2), ("ckpt", _vp), ("ckpt_every", _i32), ("t0", _i32),
-                ("nsteps", _i32), ("trace_totals", _i32), ("rec", _vp * 5), ("trace", _vp), ("state_out", _vp)]
+                ("nsteps", _i32), ("reserved", _i32), ("rec", _vp * 5), ("trace", _vp), ("state_out", _vp)]
 
 
 class ElasticAdjArgs(ctypes.Structure):
@@ -98,6 +98,8 @@ _SIGNATURES = {
                                                       ctypes.POINTER(AcousticAdjArgs), _vp, _vp, _vp]),
     "adfwi_elastic_get_layout": (ctypes.c_int, [ctypes.POINTER(ElasticDesc), ctypes.POINTER(Layout)]),
     "adfwi_elastic_forward": (ctypes.c_int, [ctypes.POINTER(ElasticDesc), ctypes.POINTER(ElasticFwdArgs), _vp]),
+    "adfwi_elastic_forward_totals": (ctypes.c_int, [ctypes.POINTER(ElasticDesc), ctypes.POINTER(ElasticFwdArgs),
+                                                    _vp]),
     "adfwi_elastic_adjoint": (ctypes.c_int, [ctypes.POINTER(ElasticDesc), ctypes.POINTER(ElasticAdjArgs), _vp]),
     "adfwi_elastic_adjoint_totals": (ctypes.c_int, [ctypes.POINTER(ElasticDesc), ctypes.POINTER(ElasticAdjArgs),
                                                     _vp]),

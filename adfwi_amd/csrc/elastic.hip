@@ -2520,7 +2520,8 @@ int adfwi_elastic_get_layout(const adfwi_elastic_desc *d, adfwi_layout *out) {
   return el_layout(d, out);
 }
 
-int adfwi_elastic_forward(const adfwi_elastic_desc *d, adfwi_elastic_fwd_args *a, adfwi_stream_t stream) {
+// totals: a->trace receives the totals after every step, not the states
+static int elastic_forward(const adfwi_elastic_desc *d, adfwi_elastic_fwd_args *a, adfwi_stream_t stream, bool totals) {
   if (int rc = adfwi::fault_injected("adfwi_elastic_forward")) return rc;
   adfwi_layout L;
   int rc = el_layout(d, &L);
@@ -2533,7 +2534,7 @@ int adfwi_elastic_forward(const adfwi_elastic_desc *d, adfwi_elastic_fwd_args *a
   ADFWI_CHECK_ARG(!recs || (a->rec[0] && a->rec[1] && a->rec[2] && a->rec[3] && a->rec[4]),
                   "records must be all set or all NULL");
   if (recs && d->nrec > 0) ADFWI_CHECK_ARG(d->rcv_z && d->rcv_x, "null receiver table pointer");
-  ADFWI_CHECK_ARG(a->state_in && ((a->trace && !a->trace_totals) || (a->work[0] && a->work[1] && a->work[0] != a->work[1])),
+  ADFWI_CHECK_ARG(a->state_in && ((a->trace && !totals) || (a->work[0] && a->work[1] && a->work[0] != a->work[1])),
                   "state_in and two distinct work buffers (or a trace buffer) are required");
   ADFWI_CHECK_ARG(!(a->trace && a->ckpt), "trace and ckpt are exclusive");
   ADFWI_CHECK_ARG(a->t0 >= 0 && a->nsteps >= 0 && a->t0 + a->nsteps <= d->nt,
@@ -2553,7 +2554,7 @@ int adfwi_elastic_forward(const adfwi_elastic_desc *d, adfwi_elastic_fwd_args *a
     rk.map = d->rcv_map;
     for (int q = 0; q < 5; ++q) rk.r[q] = a->rec[q];
   }
-  ADFWI_CHECK_ARG(!a->trace_totals || (a->trace && tiles && !d->damping),
+  ADFWI_CHECK_ARG(!totals || (a->trace && tiles && !d->damping),
                   "a trace of totals needs a trace buffer and the tile kernels (PML without C15 / C35, "
                   "library tiling, a receiver map for records, state sets under 2 GiB)");
   if (tiles && d->damping) {
@@ -2578,7 +2579,7 @@ int adfwi_elastic_forward(const adfwi_elastic_desc *d, adfwi_elastic_fwd_args *a
     a->state_out = cur;
     return ADFWI_OK;
   }
-  if (tiles && (!a->trace || a->trace_totals)) {
+  if (tiles && (!a->trace || totals)) {
     for (int k = 0; k < a->nsteps;) {
       const int t = a->t0 + k;
       int n = min(tile::steps_of(v.nn), a->nsteps - k);
@@ -2650,6 +2651,14 @@ int adfwi_elastic_forward(const adfwi_elastic_desc *d, adfwi_elastic_fwd_args *a
   }
   a->state_out = cur;
   return ADFWI_OK;
+}
+
+int adfwi_elastic_forward(const adfwi_elastic_desc *d, adfwi_elastic_fwd_args *a, adfwi_stream_t stream) {
+  return elastic_forward(d, a, stream, false);
+}
+
+int adfwi_elastic_forward_totals(const adfwi_elastic_desc *d, adfwi_elastic_fwd_args *a, adfwi_stream_t stream) {
+  return elastic_forward(d, a, stream, true);
 }
 
 static int elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a, adfwi_stream_t stream, bool totals) {

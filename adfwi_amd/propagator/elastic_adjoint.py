@@ -45,7 +45,8 @@ def run_backward(geom, coef: torch.Tensor, src: torch.Tensor, pml_x: Optional[to
     # with totals: ping-pong states of the recomputation, and the totals before a segment
     rw = geom.state(2) if totals and trace is not None else None
     before = geom.trace(1, True)[0] if totals else None
-    adjoint = lib.adfwi_elastic_adjoint_totals if totals else lib.adfwi_elastic_adjoint
+    forward, adjoint = ((lib.adfwi_elastic_forward_totals, lib.adfwi_elastic_adjoint_totals) if totals else
+                        (lib.adfwi_elastic_forward, lib.adfwi_elastic_adjoint))
     zero = None
     gacc = torch.zeros(int(L.accum_floats), device=dev, dtype=torch.float32)
     gsrc = torch.zeros((S, nt), device=dev, dtype=torch.float32)
@@ -72,11 +73,10 @@ def run_backward(geom, coef: torch.Tensor, src: torch.Tensor, pml_x: Optional[to
             fa.trace = trace.data_ptr()
             fa.t0, fa.nsteps = t0, n
             if totals:
-                fa.trace_totals = 1
                 fa.work[0], fa.work[1] = rw[0].data_ptr(), rw[1].data_ptr()
             TIMELINE.call("recompute", geom.step_kernels[0] if tiled else geom.kernel_names[0],
                           tile_launches(t0, n, 0, geom.tile_steps) if tiled else n, dev, lambda: nat.check(
-                lib.adfwi_elastic_forward(ctypes.byref(d), ctypes.byref(fa), stream),
+                forward(ctypes.byref(d), ctypes.byref(fa), stream),
                 "adfwi_elastic_forward (recompute)"), steps=n)
         if totals and seg - 1 not in traces:   # (a resident segment's last totals are there already)
             if seg == 0:

@@ -322,7 +322,6 @@ def run_forward(geom: ElasticGeometry, coef, pml_x, pml_z, src, scalars, *, reco
         if t0 >= head:            # inside a resident segment: every state goes to its trace
             seg = t0 // k
             a.trace = traces[seg][t0 - seg * k].data_ptr()
-            a.trace_totals = int(totals)
         else:
             a.ckpt = None if ckpt is None else ckpt.data_ptr()
             a.ckpt_every = k if ckpt is not None else 0
@@ -330,10 +329,11 @@ def run_forward(geom: ElasticGeometry, coef, pml_x, pml_z, src, scalars, *, reco
         if rec is not None:
             for i in range(5):
                 a.rec[i] = rec[i].data_ptr()
+        forward = lib.adfwi_elastic_forward_totals if totals and t0 >= head else lib.adfwi_elastic_forward
         launches = tile_launches(t0, a.nsteps, int(a.ckpt_every), geom.tile_steps) if tiled else a.nsteps
         TIMELINE.call("forward" if t0 < head else "forward+trace", geom.step_kernels[0],
                       launches, dev,
-                      lambda: nat.check(lib.adfwi_elastic_forward(ctypes.byref(d), ctypes.byref(a), stream),
+                      lambda: nat.check(forward(ctypes.byref(d), ctypes.byref(a), stream),
                                         "adfwi_elastic_forward"), steps=a.nsteps)
         cur = _state_at(a.state_out, work, bufs)
         if energy_ends is not None and te in ends:

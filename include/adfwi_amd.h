@@ -249,12 +249,7 @@ typedef struct adfwi_elastic_fwd_args {
   float *ckpt;             /* [n][10][S][Z][pitch] or NULL */
   int32_t ckpt_every;
   int32_t t0, nsteps;
-  int32_t trace_totals;    /* 1: `trace` receives the five totals after every step (txx, tzz, txz, vx, vz
-                              as split sums, [nsteps][5][S][Z][pitch]) and the states go through
-                              work[]; only where adfwi_elastic_forward runs its tile kernels: PML, aniso 0,
-                              shots_per_wave and tile_z 0, rcv_map given when records are taken, state
-                              sets under 2 GiB, with nn > 2 at most 768 tiles of 52 x 52 window points
-                              over the shots.  0: full states, as described at trace */
+  int32_t reserved;
   float *rec[5];           /* txx, tzz, txz, vx, vz records [S][nt][R], or all NULL */
   float *trace;            /* [nsteps][10][S][Z][pitch] or NULL: the state after every step of the
                               call is written to its slot (work[] unused; ckpt must be NULL) */
@@ -264,6 +259,13 @@ typedef struct adfwi_elastic_fwd_args {
 /* Forward time stepping (replaces step_forward_PML_4order, elastic_kernels.py:222-423,
  * step_forward_PML_6order :426-584 and step_forward_ABL_4order :585-777). */
 int adfwi_elastic_forward(const adfwi_elastic_desc *d, adfwi_elastic_fwd_args *a, adfwi_stream_t stream);
+
+/* The same with a trace of totals: a->trace (not NULL) receives the five totals after every step (txx,
+ * tzz, txz, vx, vz as split sums, [nsteps][5][S][Z][pitch]) and the states go through work[].  Only
+ * where adfwi_elastic_forward runs its tile kernels, else ADFWI_E_ARG: PML, aniso 0, shots_per_wave and
+ * tile_z 0, rcv_map given when records are taken, state sets under 2 GiB, with nn > 2 at most 768 tiles
+ * of 52 x 52 window points over the shots. */
+int adfwi_elastic_forward_totals(const adfwi_elastic_desc *d, adfwi_elastic_fwd_args *a, adfwi_stream_t stream);
 
 typedef struct adfwi_elastic_adj_args {
   float *lam_in;           /* adjoint of the state after step t_hi-1: work[0] or work[1]; without
@@ -286,11 +288,11 @@ typedef struct adfwi_elastic_adj_args {
  * autograd replay of step_forward_PML_4order (elastic_kernels.py:975-1008 checkpoints). */
 int adfwi_elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a, adfwi_stream_t stream);
 
-/* The same from a trace of totals (adfwi_elastic_fwd_args.trace_totals): a->trace holds
+/* The same from a trace of totals (adfwi_elastic_forward_totals): a->trace holds
  * [nsteps][5][S][Z][pitch] and a->fwd0 the totals before step t_hi-nsteps, [5][S][Z][pitch] (vx and
  * vz are read).  Half the bytes of the forward wavefield, and two steps per launch; the gradients
  * are the same to rounding (their terms are added in another order), the adjoint states and the
- * wavelet gradient bit for bit.  For what adfwi_elastic_fwd_args.trace_totals takes. */
+ * wavelet gradient bit for bit.  For what adfwi_elastic_forward_totals takes. */
 int adfwi_elastic_adjoint_totals(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a, adfwi_stream_t stream);
 
 /* ------------------------------------------------------------------------ */

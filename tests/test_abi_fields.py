@@ -21,3 +21,17 @@ def test_elastic_accumulator_is_ngroups_sets(S, Z, X, damping, nn):
     d, L = _desc(S, Z, X, damping, nn), nat.Layout()
     assert nat.load().adfwi_elastic_get_layout(ctypes.byref(d), ctypes.byref(L)) == 0
     assert L.accum_floats == L.ngroups * 8 * Z * d.pitch
+
+
+def test_elastic_forward_ignores_its_reserved_field():
+    from adfwi_amd import _native as nat
+    at = next(f[0] for f in nat.ElasticFwdArgs._fields_
+              if getattr(nat.ElasticFwdArgs, f[0]).offset == nat.ElasticFwdArgs.nsteps.offset + 4)
+    fake = 0x1000
+    d, a = _desc(3, 60, 90), nat.ElasticFwdArgs()
+    for f in ("coef", "src", "src_m", "src_z", "src_x", "pml_x", "pml_z"):
+        setattr(d, f, fake)
+    a.state_in, a.trace, a.nsteps = fake, fake, 0
+    for value in (0, 1, -1):     # a trace of states needs no work buffers
+        setattr(a, at, value)
+        assert nat.load().adfwi_elastic_forward(ctypes.byref(d), ctypes.byref(a), None) == 0, nat.load().adfwi_last_error()
