@@ -2662,6 +2662,7 @@ int adfwi_elastic_forward_totals(const adfwi_elastic_desc *d, adfwi_elastic_fwd_
 }
 
 static int elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a, adfwi_stream_t stream, bool totals) {
+  if (int rc = adfwi::fault_injected("adfwi_elastic_adjoint")) return rc;
   adfwi_layout L;
   int rc = el_layout(d, &L);
   if (rc) return rc;
@@ -2798,7 +2799,6 @@ static int elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *
 }
 
 int adfwi_elastic_adjoint(const adfwi_elastic_desc *d, adfwi_elastic_adj_args *a, adfwi_stream_t stream) {
-  if (int rc = adfwi::fault_injected("adfwi_elastic_adjoint")) return rc;
   return elastic_adjoint(d, a, stream, false);
 }
 

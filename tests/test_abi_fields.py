@@ -1,8 +1,13 @@
 """The C ABI as callers built against earlier headers of the same version use it (host only, no GPU:
 calls of zero steps launch nothing)."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def _desc(S, Z, X, damping=0, nn=2):
@@ -35,3 +40,13 @@ def test_elastic_forward_ignores_its_reserved_field():
     for value in (0, 1, -1):     # a trace of states needs no work buffers
         setattr(a, at, value)
         assert nat.load().adfwi_elastic_forward(ctypes.byref(d), ctypes.byref(a), None) == 0, nat.load().adfwi_last_error()
+
+
+@pytest.mark.parametrize("name,variant", [("adfwi_acoustic_forward", "sum"), ("adfwi_acoustic_adjoint", "sum"),
+                                          ("adfwi_elastic_forward", "totals"), ("adfwi_elastic_adjoint", "totals")])
+def test_a_fault_injected_into_an_entry_point_reaches_its_variants(name, variant):
+    code = ("from adfwi_amd import _native as nat; lib = nat.load(); "
+            f"print(lib.{name}(None, None, None), lib.{name}_{variant}(None, None, None))")
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True,
+                         env=dict(os.environ, ADFWI_FAULT_INJECT=name), cwd=ROOT)
+    assert out.stdout.split() == ["-4", "-4"], out.stderr
