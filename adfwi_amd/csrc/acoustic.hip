@@ -1331,7 +1331,8 @@ void launch_fwd_tile_f(const AcDev &v, hipStream_t st, const tile::FwdIO &io, bo
 
 void launch_fwd_tile(const AcDev &v, hipStream_t st, const tile::FwdIO &io, bool apart) {
   const bool rec = io.energy || io.rec_p;
-  if (!io.img_d && !io.img_p) launch_fwd_tile_f<PF_REC>(v, st, io, apart);
+  if (v.tbase) launch_fwd_tile_f<PF_REC | tile::PF_TBASE>(v, st, io, apart);
+  else if (!io.img_d && !io.img_p) launch_fwd_tile_f<PF_REC>(v, st, io, apart);
   else if (!rec && !io.img_p) launch_fwd_tile_f<PF_IMGD>(v, st, io, apart);
   else if (!rec) launch_fwd_tile_f<PF_IMGD | PF_IMGP>(v, st, io, apart);
   else if (!io.img_p) launch_fwd_tile_f<PF_REC | PF_IMGD>(v, st, io, apart);
@@ -1519,9 +1520,10 @@ static int acoustic_forward(const adfwi_acoustic_desc *d, adfwi_acoustic_fwd_arg
     return nullptr;
   };
   const float *cur = a->state_in;
-  // (the tile kernels that write the pressure image write the stencil image too: a pressure image
-  // alone, for a gradient of A2 and not of A1, is left to the strip kernels)
-  if (fuse && tile_ok(d) && (a->image || !a->image_p)) {
+  // (the tile kernels that write the pressure image write the stencil image too, and those with a
+  // device time base neither: a pressure image alone, for a gradient of A2 and not of A1, and images
+  // with a time base are left to the strip kernels)
+  if (fuse && tile_ok(d) && (a->t_base ? !a->image && !a->image_p : a->image || !a->image_p)) {
     for (int k = 0; k < a->nsteps;) {
       const int t = a->t0 + k;
       int n = min(tile::TK, a->nsteps - k);

@@ -121,8 +121,8 @@ typedef struct adfwi_acoustic_fwd_args {
   int32_t fuse_steps;      /* 1: advance several steps per launch where possible (four on register
                               tiles; two when the descriptor sets shots_per_block,
                               adj_shots_per_block, row_unroll or tile_z, which are options of the
-                              strip kernels, the pitch is odd, or image_p is set without image);
-                              0: one */
+                              strip kernels, the pitch is odd, image_p is set without image, or an
+                              image with t_base); 0: one */
   int32_t reserved2;
   const int32_t *t_base;   /* device int or NULL: added at run time to every step index of the
                               call (t0 .. t0+nsteps-1 are then relative), so that one captured
