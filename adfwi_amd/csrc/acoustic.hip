@@ -1279,6 +1279,19 @@ TileShape tile_shape(const AcDev &v) {
   return TileShape::LARGE;
 }
 
+// A launch cut to a step or two, by checkpoints that close together or at the end of a call, pays the
+// tiles' halo for them: on more than one round of workgroups a single step, on more than eight two
+// forward steps without images go to the strip kernels (those with a time base stay on tiles).  Forward,
+// us per step with a checkpoint every step / second step, strips -> tiles: 241 x 441, 64 shots 62 -> 80 /
+// 51 -> 48; 464 x 1232, 4 shots 28 -> 33 / 21 -> 20, 16 shots 86 -> 106 / 56 -> 62, 32 shots 170 -> 201 /
+// 98 -> 114; 140 x 240, 10 shots 12 -> 9 / 10.5 -> 5.1.  The rest of the gradient (a step or two with
+// images, and the adjoint of them): 241 x 441, 64 shots 125 -> 156 / 117 -> 96; 464 x 1232, 16 shots
+// 172 -> 203 / 128 -> 126, 32 shots 331 -> 366 / 231 -> 223.
+bool tile_short(const AcDev &v, int n, bool modelling) {
+  const long long wgs = tile_count<4, 16, 2>(v) * v.S;
+  return !v.tbase && ((n == 1 && wgs > TILE_CUS) || (modelling && n == 2 && wgs > 8 * TILE_CUS));
+}
+
 // Shots per group: a group's shots follow each other in a workgroup, which reads the five
 // coefficient planes (20 bytes per point against a shot's 12) and adds to the energy or gradient planes
 // once for all of them, but a launch takes whole rounds of one workgroup per CU.  A round of groups of
@@ -1523,14 +1536,15 @@ static int acoustic_forward(const adfwi_acoustic_desc *d, adfwi_acoustic_fwd_arg
   // (the tile kernels that write the pressure image write the stencil image too, and those with a
   // device time base neither: a pressure image alone, for a gradient of A2 and not of A1, and images
   // with a time base are left to the strip kernels)
-  if (fuse && tile_ok(d) && (a->t_base ? !a->image && !a->image_p : a->image || !a->image_p)) {
-    for (int k = 0; k < a->nsteps;) {
-      const int t = a->t0 + k;
-      int n = min(tile::TK, a->nsteps - k);
-      // with a device time base the state returns to work[0] after whole windows of 4 steps: an
-      // even number of launches
-      if (a->t_base && k == 0 && ((a->nsteps + tile::TK - 1) / tile::TK) % 2) n = max(1, n / 2);
-      if (a->ckpt) n = min(n, a->ckpt_every - t % a->ckpt_every);   // up to the next checkpoint
+  const bool tiles = fuse && tile_ok(d) && (a->t_base ? !a->image && !a->image_p : a->image || !a->image_p);
+  for (int k = 0; k < a->nsteps;) {
+    const int t = a->t0 + k;
+    int n = min(tile::TK, a->nsteps - k);   // steps of a tile launch
+    // with a device time base the state returns to work[0] after whole windows of 4 steps: an
+    // even number of launches
+    if (a->t_base && k == 0 && ((a->nsteps + tile::TK - 1) / tile::TK) % 2) n = max(1, n / 2);
+    if (a->ckpt) n = min(n, a->ckpt_every - t % a->ckpt_every);   // up to the next checkpoint
+    if (tiles && !tile_short(v, n, !a->image)) {
       float *nxt = ckpt_slot(t + n - 1);
       if (!nxt) nxt = (cur == a->work[0]) ? a->work[1] : a->work[0];
       tile::FwdIO io;
@@ -1544,12 +1558,8 @@ static int acoustic_forward(const adfwi_acoustic_desc *d, adfwi_acoustic_fwd_arg
       if ((rc = adfwi::check_launch("ac_fwd_tile"))) return rc;
       cur = nxt;
       k += n;
+      continue;
     }
-    a->state_out = cur;
-    return ADFWI_OK;
-  }
-  for (int k = 0; k < a->nsteps;) {
-    const int t = a->t0 + k;
     const bool pair = fuse && k + 1 < a->nsteps && ckpt_slot(t) == nullptr;
     const int tl = pair ? t + 1 : t;         // last step of this launch
     float *nxt = ckpt_slot(tl);
@@ -1629,9 +1639,10 @@ static int acoustic_adjoint(const adfwi_acoustic_desc *d, adfwi_acoustic_adj_arg
   const dim3 grid1(grid.x, (d->nshots + v1.spb - 1) / v1.spb);
   auto slot = [&](int t) -> long long { return (long long)(t - a->image_t0) * L.field_floats; };
   float *cur = const_cast<float *>(a->lam_in);
-  if (fuse && tile_ok(d) && adj_tile_ok(v1, a->grad_a2 && a->image_p)) {
-    for (int k = 0; k < a->nsteps;) {
-      const int t = a->t_hi - k, n = min(tile::TK, a->nsteps - k);
+  const bool tiles = fuse && tile_ok(d) && adj_tile_ok(v1, a->grad_a2 && a->image_p);
+  for (int k = 0; k < a->nsteps;) {
+    const int t = a->t_hi - k, n = min(tile::TK, a->nsteps - k);
+    if (tiles && !tile_short(v1, n, false)) {
       float *nxt = (cur == a->work[0]) ? a->work[1] : a->work[0];
       tile::AdjIO io;
       io.in = cur; io.out = nxt; io.t = t; io.n = n;
@@ -1644,12 +1655,8 @@ static int acoustic_adjoint(const adfwi_acoustic_desc *d, adfwi_acoustic_adj_arg
       if ((rc = adfwi::check_launch("ac_adj_tile"))) return rc;
       cur = nxt;
       k += n;
+      continue;
     }
-    a->lam_out = cur;
-    return ADFWI_OK;
-  }
-  for (int k = 0; k < a->nsteps;) {
-    const int t = a->t_hi - k;
     const bool pair = fuse && k + 1 < a->nsteps;
     float *nxt = (cur == a->work[0]) ? a->work[1] : a->work[0];
     AdjPairIO io{};
