@@ -25,7 +25,7 @@ def run_backward(geom, coef: torch.Tensor, src: torch.Tensor, pml_x: Optional[to
     record adjoints (txx, tzz, txz, vx, vz; None = zero).  traces: {segment: per-step states}
     kept by run_forward(resident=...); those segments are not recomputed, and each is released
     once the segment before it no longer needs its last state.  totals: whether traces hold the
-    five totals of a state instead of its fields (run_forward's; default geom.totals).  Returns (list of 8 (Z, pitch)
+    five totals of a state instead of its fields (run_forward's; default geom.trace_totals(k)).  Returns (list of 8 (Z, pitch)
     gradients of the padded coefficient planes C11, C13, C33, C55, bx, bz, C15, C35 -- None
     where not needed -- and the (S, nt) wavelet gradient or None).
     """
@@ -38,7 +38,7 @@ def run_backward(geom, coef: torch.Tensor, src: torch.Tensor, pml_x: Optional[to
     first_resident = min(traces) if traces else nseg
     if first_resident > 1 and (ckpt is None or ckpt.shape[0] < first_resident - 1):
         raise RuntimeError("the forward pass kept no checkpoints for the adjoint")
-    totals = geom.totals if totals is None else bool(totals)
+    totals = geom.trace_totals(k) if totals is None else bool(totals)
     tiled = totals or (geom.damping and geom.tiled)
     lam = geom.state(2)
     trace = geom.trace(min(k, nt), totals) if len(traces) < nseg else None

@@ -118,16 +118,27 @@ class ElasticGeometry:
         receiver map if there are receivers, state sets and coefficients under 2 GiB, at 6th to
         10th order only so many tiles (el_tile_ok's rule)."""
         plane = 4 * self.Z * self.pitch
-        tiles64 = -(-(self.X - 2 * self.nn) // 52) * -(-(self.Z - 2 * self.nn) // 52) * self.S
         return (not self.aniso and not self.shots_per_wave and not self.tile_z
-                and (self.nn == 2 or tiles64 <= (384 if self.damping else 768))
+                and (self.nn == 2 or self._tiles64 <= (384 if self.damping else 768))
                 and (self.R == 0 or self.rcv_map is not None) and self.nfield * self.S * plane < 1 << 31
                 and 8 * plane < 1 << 31)
 
     @property
+    def _tiles64(self) -> int:
+        return -(-(self.X - 2 * self.nn) // 52) * -(-(self.Z - 2 * self.nn) // 52) * self.S
+
+    @property
     def totals(self) -> bool:
-        """Whether a trace holds the five totals of a step instead of the PML scheme's ten splits."""
+        """Whether a trace may hold the five totals of a step instead of the PML scheme's ten splits."""
         return self.tiled and not self.damping
+
+    def trace_totals(self, k: int) -> bool:
+        """Whether the traces of checkpoint segments of k steps hold totals: not at 4th order where every
+        step is a segment and the tiles take more than one round of one workgroup per CU.  A launch of
+        the tile adjoint then reverses one step and pays the halo of two (ms per gradient of 60 steps,
+        step kernels -> tiles: 171 x 373, 24 shots 9.9 -> 11.3; 242 x 680, 4 shots 5.3 -> 5.6, 16 shots
+        16.9 -> 19.5, 32 shots 35.7 -> 35.2; in one round 122 x 240, 1 shot 2.7 -> 2.4)."""
+        return self.totals and not (k == 1 and self.nn == 2 and self._tiles64 > 256)
 
     @property
     def step_kernels(self):
@@ -240,7 +251,7 @@ def resident_trace_segments(geom: ElasticGeometry, k: int) -> int:
         return 0
     state_bytes = int(geom.layout.state_floats) * 4
     seg_bytes = k * state_bytes
-    if getattr(geom, "totals", False):    # five totals instead of ten splits
+    if hasattr(geom, "trace_totals") and geom.trace_totals(k):    # five totals instead of ten splits
         seg_bytes //= 2
     if cap is None:
         cap = resident_budget_bytes(geom.device, (nseg + 5) * state_bytes + seg_bytes) // seg_bytes
@@ -266,7 +277,7 @@ def run_forward(geom: ElasticGeometry, coef, pml_x, pml_z, src, scalars, *, reco
     """All nt steps from a zero state.  Returns dict(rec=[5 x (S, nt, R)] or None,
     energy=[5 x (Z, X)] summed over the states after the steps in energy_ends, ckpt,
     traces={segment: per-step states}, totals: whether the traces hold five totals instead of the
-    state's fields, geom.totals).
+    state's fields, geom.trace_totals(ckpt_every)).
 
     resident > 0 (with ckpt_every): the last `resident` checkpoint segments write the state after
     each of their steps to a trace buffer of their own, which run_backward uses instead of
@@ -274,9 +285,9 @@ def run_forward(geom: ElasticGeometry, coef, pml_x, pml_z, src, scalars, *, reco
     lib = nat.load()
     dev = geom.device
     S, nt, R = geom.S, geom.nt, geom.R
-    totals, tiled = geom.totals, geom.tiled
-    work = geom.state(2)
     k = int(ckpt_every)
+    totals, tiled = geom.trace_totals(k), geom.tiled
+    work = geom.state(2)
     nseg = -(-nt // k) if k else 1
     resident = int(resident) if k else 0
     head = (nseg - resident) * k if resident else nt      # steps before the resident segments
@@ -330,9 +341,10 @@ def run_forward(geom: ElasticGeometry, coef, pml_x, pml_z, src, scalars, *, reco
             for i in range(5):
                 a.rec[i] = rec[i].data_ptr()
         forward = lib.adfwi_elastic_forward_totals if totals and t0 >= head else lib.adfwi_elastic_forward
-        launches = tile_launches(t0, a.nsteps, int(a.ckpt_every), geom.tile_steps) if tiled else a.nsteps
-        TIMELINE.call("forward" if t0 < head else "forward+trace", geom.step_kernels[0],
-                      launches, dev,
+        on_tiles = tiled and (t0 < head or totals or geom.damping)
+        launches = tile_launches(t0, a.nsteps, int(a.ckpt_every), geom.tile_steps) if on_tiles else a.nsteps
+        TIMELINE.call("forward" if t0 < head else "forward+trace",
+                      geom.step_kernels[0] if on_tiles else geom.kernel_names[0], launches, dev,
                       lambda: nat.check(forward(ctypes.byref(d), ctypes.byref(a), stream),
                                         "adfwi_elastic_forward"), steps=a.nsteps)
         cur = _state_at(a.state_out, work, bufs)
