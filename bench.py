@@ -39,15 +39,35 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-# algorithmic bytes per padded point, per time step, per shot (fp32 state, imaging traffic)
-BYTES_FWD = 24.0          # forward: read + write p, u, w
-BYTES_RECOMPUTE = 28.0    # recompute: forward + stencil image store
-BYTES_ADJ = 28.0          # adjoint: read + write adjoint p, u, w + stencil image read
-BYTES_GRAD = 80.0         # per shot-gradient: 24 + 28 + 28
+# bytes per padded point and shot: a state is read and written once per launch, an image or a trace
+# once per step (coefficient planes, halos and records are not counted)
+BYTES_STATE = 24.0        # p, u, w, forward or adjoint, per launch
+BYTES_IMAGE = 4.0         # stencil image per step
+# the specified algorithm, one step per launch: forward, recompute with images, adjoint
+BYTES_GRAD = 80.0         # per shot-gradient and step: 24 + 28 + 28
 # elastic: ten split fields
-EL_BYTES_FWD = 80.0       # forward / recompute: read + write the ten splits
-EL_BYTES_ADJ = 120.0      # adjoint: read + write ten adjoint splits, read the forward state before and after
-EL_BYTES_GRAD = 280.0     # per shot-gradient: 80 + 80 + 120
+EL_BYTES_STATE = 80.0     # the ten splits, forward or adjoint, per launch (damping scheme: five fields, half)
+EL_BYTES_FWD_READ = 40.0  # step kernels' adjoint: the forward state before and after, per step
+EL_BYTES_TOTALS = 20.0    # tiles' traces: five totals (damping scheme: five fields) per step
+EL_BYTES_GRAD = 280.0     # per shot-gradient and step: 80 + 80 + 120
+
+
+def launch_bytes(kernel, launches, steps, steps_by_call):
+    """Bytes per point and shot that `launches` of a kernel over `steps` time steps cannot do without."""
+    if kernel.startswith("ac_"):
+        images = (steps if "adj" in kernel else
+                  steps_by_call.get("recompute", 0) + steps_by_call.get("forward+images", 0))
+        return BYTES_STATE * launches + BYTES_IMAGE * images
+    state = EL_BYTES_STATE / (2 if "abl" in kernel else 1)
+    if not kernel.endswith("_tile"):
+        read = EL_BYTES_FWD_READ / (2 if "abl" in kernel else 1)
+        return (state + (read if "adj" in kernel else 0.0)) * steps
+    if "adj" in kernel:
+        return state * launches + EL_BYTES_TOTALS * steps
+    traced = steps_by_call.get("recompute", 0) + steps_by_call.get("forward+trace", 0)
+    if "abl" in kernel:   # its trace is the state itself: the launch's last state counts once
+        traced = max(0.0, traced * (1.0 - launches / max(steps, 1)))
+    return state * launches + EL_BYTES_TOTALS * traced
 
 
 def profiled_traffic(kernel, workload):
@@ -408,23 +428,11 @@ def main():
     N = Z * X
     S = wl.nshots
     value = S * args.steps / elapsed
-    # dominant kernel by total time; its algorithmic bytes per launch
+    # dominant kernel by total time; the bytes its launches cannot do without
     kern = {}
     for name, d in tl.items():
         steps_by = d["steps_by_call"]
-        if name in ("ac_fwd_step", "ac_fwd_pair", "ac_fwd_tile"):
-            byts = (steps_by.get("forward", 0) * BYTES_FWD + (steps_by.get("recompute", 0)
-                    + steps_by.get("forward+images", 0)) * BYTES_RECOMPUTE) * N * S
-        elif name in ("ac_adj_step", "ac_adj_pair", "ac_adj_tile"):
-            byts = d["steps"] * BYTES_ADJ * N * S
-        elif name in ("el_fwd_step", "el_fwd_tile", "el3_fwd_step"):
-            byts = d["steps"] * EL_BYTES_FWD * N * S
-        elif name in ("el_abl_fwd", "el3_abl_fwd", "abl_fwd_tile"):
-            byts = d["steps"] * EL_BYTES_FWD / 2 * N * S
-        elif name in ("el_abl_adj", "el3_abl_adj", "abl_adj_tile"):
-            byts = d["steps"] * EL_BYTES_ADJ / 2 * N * S
-        else:
-            byts = d["steps"] * EL_BYTES_ADJ * N * S
+        byts = launch_bytes(name, d["launches"], d["steps"], steps_by) * N * S
         avg_ms = d["ms"] / max(d["launches"], 1)
         kern[name] = {"total_ms": d["ms"], "launches": d["launches"], "steps": d["steps"],
                       "steps_by_call": d["steps_by_call"], "avg_launch_ms": avg_ms,
@@ -433,8 +441,8 @@ def main():
     dom = max(kern, key=lambda k: kern[k]["total_ms"])
     ach = kern[dom]["achieved_gbs"]
     traffic = profiled_traffic(dom, wl.name)
-    # bytes of the steps actually executed (resident segments skip part of the recompute) against
-    # the specified algorithm's per-pt-step figure
+    # bytes of the launches actually executed (resident segments skip part of the recompute), and the
+    # specified algorithm's per-pt-step figure
     executed = sum(k["bytes_total"] for k in kern.values())
     spec_bytes = ((EL_BYTES_GRAD / (2 if args.abc != "PML" else 1)) if elastic else BYTES_GRAD) * S * N * wl.nt
     out = {
@@ -454,10 +462,11 @@ def main():
                    "nt": wl.nt, "shots_per_launch": S, "receivers": len(wl.rcv_x), "dt": wl.dt, "dx": wl.dx,
                    "checkpoint_interval": ak.checkpoint_interval(wl.nt), "parallelism": "single GPU, shot batch"},
         "gpt_updates_per_s": 2 * S * N * wl.nt * args.steps / elapsed / 1e9,
-        # the executed steps' algorithmic bytes over the whole step time, against 8 TB/s
+        # the executed launches' bytes over the whole step time, against 8 TB/s
         "grad_bytes_roofline_frac": executed / elapsed / 1e9 / HBM_PEAK_GBS,
         "executed_bytes_per_shot_gradient": executed / (S * args.steps),
-        # the specified algorithm's bytes (every segment recomputed) over the same time
+        # the specified algorithm's bytes (one step per launch, every segment recomputed) over the same
+        # time: a rate of work, not of traffic (several steps per launch move fewer bytes)
         "spec_grad_bytes_roofline_frac": spec_bytes * args.steps / elapsed / 1e9 / HBM_PEAK_GBS,
         "roofline": {"bound": "hbm", "kernel": dom, "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": ach / HBM_PEAK_GBS, "traffic": traffic,
