@@ -195,10 +195,12 @@ class AcousticGeometry:
 
     @property
     def tiled(self) -> bool:
-        """Whether fused steps run on the tile kernels (the strip options of the descriptor ask
-        for the strip kernels; so does a forward that writes the pressure image alone)."""
-        return bool(self.fuse_steps) and not (self.shots_per_block or self.adj_shots_per_block or self.row_unroll
-                                              or self.tile_z)
+        """Whether fused steps run on the tile kernels, as the library chooses: not with a strip option
+        set, an odd pitch, or five planes of 2 GiB and more (nor for a forward that writes the pressure
+        image alone, nor for launches cut to a step or two on large grids)."""
+        return (bool(self.fuse_steps) and not (self.shots_per_block or self.adj_shots_per_block or self.row_unroll
+                                               or self.tile_z)
+                and self.pitch % 2 == 0 and 5 * 4 * self.Z * self.pitch < 1 << 31)
 
     def adjoint_tiled(self, need_a2: bool) -> bool:
         """Whether the adjoint does too: with the rho gradient on up to 4096 tiles of 40 x 40
