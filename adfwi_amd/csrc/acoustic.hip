@@ -1258,11 +1258,10 @@ bool tile_ok(const adfwi_acoustic_desc *d) {
 // Tile shapes: 40 x 64 (stores 16 x 40), 64 x 64 (40 x 40), 64 x 128 (40 x 104).  The smaller a
 // tile the more of it is halo, but the sooner its workgroup is done: a launch whose workgroups
 // all run at once (one per CU) lasts as long as one of them.  So: the smallest shape that still
-// gives at most one workgroup per CU, else the largest.  Measured, forward with records / adjoint,
-// us per step: 140 x 240, 1 shot (54 / 24 / 12 workgroups): 1.9 / 2.3 / 3.4 and 2.5 / 2.8 / 4.6;
+// gives at most one workgroup per CU, else the largest.  Measured, forward with records and no energy
+// maps / adjoint, shot by shot, us per step: 140 x 240, 1 shot (54 / 24 / 12 workgroups): 1.9 / 2.3 / 3.4 and 2.5 / 2.8 / 4.6;
 // 10 shots (540 / 240 / 120): 4.0 / 2.6 / 3.7 and 6.2 / 3.1 / 4.8; 149 x 263, 40 shots
-// (2520 / 1120 / 480): 12.5 / 9.6 / 7.3 and 19.2 / 12.5 / 9.5
-// (6.7 and 7.9 with pairs of shots, below).
+// (2520 / 1120 / 480): 12.5 / 9.6 / 7.3 and 19.2 / 12.5 / 9.5.
 enum class TileShape { SMALL, MEDIUM, LARGE };
 constexpr long long TILE_CUS = 256;
 
@@ -1296,8 +1295,8 @@ bool tile_short(const AcDev &v, int n, bool modelling) {
 // coefficient planes (20 bytes per point against a shot's 12) and adds to the energy or gradient planes
 // once for all of them, but a launch takes whole rounds of one workgroup per CU.  A round of groups of
 // g shots measured 12 + 9.5 g us forward (64 x 128 points, 4 steps), so: the least rounds * (1.2 + g),
-// a larger g only if it is 3 % better.  us per step for g = 1 / 2 / 4 / 8, forward and adjoint: 296 x 808, 16
-// shots 19.0 / 15.0 / 12.9 / 22.1 and 20.9 / 17.0 / 16.6 / 28.8; 149 x 263, 40 shots 9.1 / 7.6 / 12.1 / 22.0
+// a larger g only if it is 3 % better.  us per step for g = 1 / 2 / 4 / 8, forward with records and energy
+// maps, and adjoint: 296 x 808, 16 shots 19.0 / 15.0 / 12.9 / 22.1 and 20.9 / 17.0 / 16.6 / 28.8; 149 x 263, 40 shots 9.1 / 7.6 / 12.1 / 22.0
 // and 9.4 / 7.9 / 13.3 / 24.8; 464 x 1232, 64 shots 128 at each and 169 (2) / 149 / 151.  With the rho
 // gradient (64 x 64 points) the time goes with the shots alone: pairs, 241 x 441, 12 shots 15.3 / 13.3 /
 // 13.8; 296 x 808, 16 shots 40.2 / 34.6 / 37.3.  A group adds all its shots to the plane of its first

@@ -429,7 +429,9 @@ struct AdjIO {
   const float *g_p, *g_u, *g_w;    // record adjoints [S][nt][R] or NULL
 };
 
-// FULL: u and w record adjoints or the wavelet gradient; A2: the rho gradient
+// FULL: u and w record adjoints or the wavelet gradient; A2: the rho gradient.  16 wavefronts leave 128
+// VGPRs: with two columns per lane 9 are spilled (27 with FULL, some in the step loop), and scalars go to
+// lanes of others; with one column 83 to 100 are used and none spilled.
 template <int NR, int NW, int CPL, bool A2, bool FULL>
 __global__ __launch_bounds__(NW *WAVE) void ac_adj_tile(AcDev d, Grid g, AdjIO io) {
   static_assert(NR >= 4 && H % NR + 2 < NR, "the free-surface rows fs-1 .. fs+1 lie in one wavefront");

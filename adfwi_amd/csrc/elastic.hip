@@ -14,7 +14,8 @@
 //      vx[1]=vz[1,j+1]-vz[1,j]+vz[2,j+1]-vz[2,j]+vx[3,j], vz[0]=vz[1];
 //   6. records of the five totals.
 // Every expression keeps the reference's fp32 association (compiled with
-// -ffp-contract=off, IEEE division; the tile kernels form the same quotients otherwise), so a step is bit-identical to the reference's CPU
+// -ffp-contract=off, IEEE division; the tile kernels form the same quotients otherwise, but for the last
+// place of some below 2^-126), so a step is bit-identical to the reference's CPU
 // op sequence given identical coefficients.  C15/C35 terms are skipped for isotropic and
 // VTI media (exact: they multiply zeros).
 //
@@ -2417,7 +2418,9 @@ ElDev el_dev(const adfwi_elastic_desc *d, const adfwi_layout &L) {
 // to the library, records (if any) go through the receiver map, and a state set stays under the
 // 2 GiB that dropped buffer accesses need.  Two steps per launch at 4th order.  With three-term
 // differences it is one, the halo's price is not halved, and what the tiles gain is that no lane
-// marches down a strip: up to three rounds of 64-row tiles.  Measured, us per step, step kernels ->
+// marches down a strip: up to three rounds of 64-row tiles.  Above those the forward is slower on tiles
+// (that is where the line is) though the adjoint is not yet; it is one line for both because the tile
+// adjoint reads a trace of totals, which only the tile forward writes.  Measured, us per step, step kernels ->
 // tiles, forward with records / with a trace / adjoint: 163 x 341, 3 shots 20 -> 10 / 19 -> 11 / 36 ->
 // 17; 214 x 393, 8 shots (256 tiles) 25 -> 18 / 29 -> 20 / 46 -> 37; 24 shots (768) 49 -> 50 / 63 -> 55 /
 // 111 -> 78; 32 shots 59 -> 66 / 78 -> 81 / 150 -> 113; 243 x 680, 32 shots 151 -> 158 / 152 -> 191 /

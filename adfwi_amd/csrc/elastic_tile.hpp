@@ -36,11 +36,11 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
-// x / b from rb = 1.0 / (double)b, the same bits as the division: rb and the product are each within
-// 2^-53 of their exact values, relatively, and a quotient of two floats lies at least 2^-49 of its
-// size from any value halfway between two floats, so the last rounding falls as the division's.
-// (Quotients below 2^-126 can lie on such a value; both then round a number of 1e-38 at its last
-// place.)  15 cycles a wavefront against 50 for the division sequence.
+// x / b from rb = 1.0 / (double)b, for quotients of 2^-126 and more the same bits as the division: rb and
+// the product are each within 2^-53 of their exact values, relatively, and a quotient of two floats lies
+// at least 2^-49 of its size from any value halfway between two floats, so the last rounding falls as
+// the division's.  Smaller quotients can lie on such a value, and then may round to its other side:
+// 1.4e-45 apart, as far from the quotient as the division's.  15 cycles a wavefront against 50 for the division sequence.
 __device__ __forceinline__ float quot(float x, double rb) { return (float)((double)x * rb); }
 // a value no kernel writes, at a wave-uniform address: a scalar load
 template <class T>

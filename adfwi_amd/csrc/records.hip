@@ -35,10 +35,10 @@ namespace {
 constexpr int NT = 1024;       // threads per workgroup
 constexpr int NW = NT / 64;
 
-// x / b, bit for bit, from rb = 1.0 / (double)b: rb and the product are within 2^-53 of their exact
-// values, relatively, and a quotient of two floats lies at least 2^-49 of its size from any value
-// halfway between two floats.  (Below 2^-126 a quotient can lie on one, and may round to the other
-// side.)  Three operations against the division's ten.
+// x / b from rb = 1.0 / (double)b, for quotients of 2^-126 and more bit for bit: rb and the product are
+// within 2^-53 of their exact values, relatively, and a quotient of two floats lies at least 2^-49 of its
+// size from any value halfway between two floats.  (Below 2^-126 a quotient can lie on one, and may round
+// to the other side.)  Three operations against the division's ten.
 __device__ __forceinline__ float quot(float x, double rb) { return (float)((double)x * rb); }
 
 template <int RW>
