@@ -11,21 +11,14 @@
 // The points a step leaves alone (outside the update windows, outside the grid) carry the
 // coefficients 1 and 0, so the updates run on every point of the tile without branches or
 // masks: 1*x - 0*d returns x.  u is zero past column X-2, as the stage leaves it.
+#include "tile_common.hpp"
+
 namespace tile {
 
 constexpr int TK = 4;              // steps per launch (at most)
 constexpr int H = 3 * TK;          // halo points per side
 constexpr int out_cols(int cpl) { return cpl * WAVE - 2 * H; }    // stored columns
 constexpr int out_rows(int rows) { return rows - 2 * H; }          // stored rows
-
-// value of the lane one to the left / right (0 past the wavefront's ends, which only halo
-// columns see)
-__device__ __forceinline__ float from_left(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x138, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float from_right(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x130, 0xf, 0xf, true));
-}
 
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 // a lane's CPL adjacent columns
@@ -54,25 +47,6 @@ __device__ __forceinline__ void stc(const float (&x)[CPL], rsrc_t r, unsigned vo
   }
 }
 
-// the exchange between wavefronts goes through LDS only: loads and stores of global memory may
-// stay in flight across it
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// a value no kernel writes, at a wave-uniform address: a scalar load, outside the vector
-// memory queue (a vector load here would make the wave wait for every prefetch issued before it)
-template <class T>
-__device__ __forceinline__ T scalar_ld(const T *p) {
-  return *(const __attribute__((address_space(4))) T *)(unsigned long long)p;
-}
-
-// forms the value where this stands: left to itself the compiler moves a sum whose only use lies past
-// a later branch there, and holds its terms till then
-__device__ __forceinline__ void pin(float &v) { asm volatile("" : "+v"(v)); }
-
 struct Grid {
   int ntx, ntz, ngroups, spg;      // tiles along x and z, shot groups, shots per group
   int spp;                         // shots per plane of the energy maps and gradients (<= spg; a group's go to its first one)
@@ -87,22 +61,6 @@ struct FwdIO {
   const int *rmap;
   float *rec_p, *rec_u, *rec_w;
 };
-
-// workgroup -> (tile, shot group): blocks go round-robin to the 8 XCDs, and every XCD takes a
-// contiguous run of a group's tiles, row by row, so that its L2 serves the halos neighbouring tiles
-// share and joins the ends of their rows, which share cache lines, before they are written back.
-// (With the groups of one tile next to each other instead, for the sake of its coefficients: 136
-// against 128 us per step forward and 190 against 168 adjoint on 464 x 1232 with 64 shots.)
-__device__ __forceinline__ void place(const Grid &g, int &tx, int &tz, int &grp) {
-  const int n = (int)gridDim.x, b = (int)blockIdx.x;
-  const int xcd = b & 7, per = n >> 3, rem = n & 7;
-  const int logical = xcd * per + min(xcd, rem) + (b >> 3);
-  const int nt = g.ntx * g.ntz;
-  grp = logical / nt;
-  const int tl = logical - grp * nt;
-  tz = tl / g.ntx;
-  tx = tl - tz * g.ntx;
-}
 
 // PF_TBASE: with a device time base; the steps that it takes outside the run are skipped.  A variant of
 // its own: in the others the bounds this takes, held over the loops, cost 2 to 4 % in spilled scalars

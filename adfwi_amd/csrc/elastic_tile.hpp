@@ -13,6 +13,8 @@
 // What a step leaves for the adjoint is the five totals, half the bytes of the ten splits: the
 // kernel writes them to a trace after every step, while the splits stay in registers between the
 // launch's steps.
+#include "tile_common.hpp"
+
 namespace tile {
 
 // Differences of ORD terms: 2 (4th order) or 3 (6th to 10th)
@@ -23,30 +25,13 @@ constexpr int OX = WAVE - 2 * H;   // stored columns
 constexpr int out_rows(int rows) { return rows - 2 * H; }
 constexpr unsigned DROP = 0x80000000u;   // a lane offset past every buffer (all under 2 GiB): access dropped
 
-__device__ __forceinline__ float from_left(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x138, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float from_right(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x130, 0xf, 0xf, true));
-}
-// the exchange between wavefronts goes through LDS only: loads and stores of global memory may
-// stay in flight across it
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 // x / b from rb = 1.0 / (double)b, for quotients of 2^-126 and more the same bits as the division: rb and
 // the product are each within 2^-53 of their exact values, relatively, and a quotient of two floats lies
 // at least 2^-49 of its size from any value halfway between two floats, so the last rounding falls as
 // the division's.  Smaller quotients can lie on such a value, and then may round to its other side:
-// 1.4e-45 apart, as far from the quotient as the division's.  15 cycles a wavefront against 50 for the division sequence.
+// 1.4e-45 apart, as far from the quotient as the division's.  15 cycles a wavefront against 50 for the
+// division sequence.
 __device__ __forceinline__ float quot(float x, double rb) { return (float)((double)x * rb); }
-// a value no kernel writes, at a wave-uniform address: a scalar load
-template <class T>
-__device__ __forceinline__ T scalar_ld(const T *p) {
-  return *(const __attribute__((address_space(4))) T *)(unsigned long long)p;
-}
 
 struct Grid { int ntx, ntz; };
 
@@ -124,22 +109,6 @@ struct FwdIO {
   float *trace;          // [n][5][S][Z][pitch] totals after each step, or NULL
   ElRec rec;             // rec.map NULL: no records
 };
-
-// workgroup -> (tile, shot): blocks go round-robin to the 8 XCDs, and every XCD takes a contiguous
-// run of a shot's tiles, row by row, so that its L2 serves the halos neighbouring tiles share and
-// joins the ends of their rows, which share cache lines, before they are written back.  (With the
-// shots of one tile next to each other instead, for the sake of its coefficients: forward with a
-// trace 135 against 108 us per step on 242 x 680 / 32 shots, 464 against 362 on 362 x 1040 / 48.)
-__device__ __forceinline__ void place(const Grid &g, int &tx, int &tz, int &s) {
-  const int n = (int)gridDim.x, b = (int)blockIdx.x;
-  const int xcd = b & 7, per = n >> 3, rem = n & 7;
-  const int logical = xcd * per + min(xcd, rem) + (b >> 3);
-  const int nt = g.ntx * g.ntz;
-  s = logical / nt;
-  const int tl = logical - s * nt;
-  tz = tl / g.ntx;
-  tx = tl - tz * g.ntx;
-}
 
 template <int ORD, int NR, int NW>
 __global__ __launch_bounds__(NW *WAVE, 4) void el_fwd_tile(ElDev d, Grid g, FwdIO io) {
@@ -370,9 +339,6 @@ struct AdjIO {
   ElInj inj;             // inj.map NULL: no record adjoints
 };
 
-// forms the values where this stands: left to itself the compiler moves a sum whose only use lies
-// past a later branch there, and holds its terms till then (50 registers in the kernel below)
-__device__ __forceinline__ void pin(float &a, float &b) { asm volatile("" : "+v"(a), "+v"(b)); }
 __device__ __forceinline__ float keep(int m, float v) {
   return __builtin_bit_cast(float, __builtin_bit_cast(int, v) & m);
 }
